@@ -39,6 +39,24 @@ def _sobol_table():
     raise RuntimeError("scipy's Sobol direction-number table was not found")
 
 
+def _ln_table():
+    """[256][2] float64 (rc, 2 ln rc) for the device's -2 ln q: rc near 1 / c, c the middle of the
+    j-th 256th of [1/2, 1), the one of 2^13 candidates whose 2 ln rc lies closest to a multiple of
+    2^-45, which is what the second column holds (sums with multiples of -2 ln 2 are then exact)."""
+    if np.finfo(np.longdouble).nmant < 63:
+        raise RuntimeError("the logarithm table needs an extended-precision long double")
+    mid = 0.5 * (1.0 + (np.arange(256) + 0.5) / 256.0)
+    cand = (1.0 / mid)[:, None] + (np.arange(8192) - 4096)[None, :] * (1.1875 * 2.0 ** -42)
+    v = 2 * np.log(cand.astype(np.longdouble)) * np.longdouble(2.0 ** 45)
+    grid = np.floor(v + np.longdouble(0.5))
+    off = np.abs(v - grid)
+    best = np.argmin(off, axis=1)
+    at = np.arange(256)
+    if float(off[at, best].max()) > 1e-3:
+        raise RuntimeError("no logarithm table within 1e-3 of the grid")
+    return np.stack([cand[at, best], (grid[at, best] * np.longdouble(2.0 ** -45)).astype(np.float64)], axis=1)
+
+
 def _raw(s, tag="SDEHDR"):
     assert (")" + tag + '"') not in s
     return 'R"' + tag + "(" + s + ")" + tag + '"'
@@ -57,6 +75,7 @@ def generate_embedded(path):
              'extern const int sdesim_jk_dims;',
              'extern const unsigned int sdesim_jk_poly[];',
              'extern const unsigned int sdesim_jk_vinit[];',
+             'extern const double sdesim_ln_table[];',
              'const char* sdesim_embedded_device_header = ' + _raw(dev) + ";",
              'const char* sdesim_embedded_args_header = ' + _raw(args) + ";",
              'const int sdesim_jk_dims = %d;' % len(poly),
@@ -67,6 +86,8 @@ def generate_embedded(path):
     for k in range(0, flat.size, 36):
         lines.append(",".join(str(int(v)) for v in flat[k:k + 36]) + ",")
     lines.append("};")
+    lines.append('extern "C" const double sdesim_ln_table[] = {')
+    lines.append(",".join(float(v).hex() for v in _ln_table().reshape(-1)) + "};")
     lines.append("}")
     text = "\n".join(lines) + "\n"
     old = open(path).read() if os.path.exists(path) else None

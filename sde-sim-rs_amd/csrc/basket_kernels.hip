@@ -225,6 +225,7 @@ struct BasketReverse {
 template <typename R, int D, int SEG, int MODE, bool PADDED>
 __global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
   constexpr bool TAPE = MODE == 2;
+  if constexpr (sizeof(R) == 8) sde_ln_tab_load(a.ln_tab);
   constexpr int NQ = BasketConst<D>::NQ;
   const long long S = a.paths;
   const int N = a.steps;

@@ -54,7 +54,9 @@ __global__ void __launch_bounds__(256) sdesim_batch(const SdeInstance* __restric
                                                      const SdeItem* __restrict__ items, int n_items,
                                                      unsigned int* __restrict__ counter,
                                                      double* __restrict__ partials, R* __restrict__ terminal,
-                                                     const long long* __restrict__ term_offset) {
+                                                     const long long* __restrict__ term_offset,
+                                                     const double* __restrict__ ln_tab) {
+  if constexpr (sizeof(R) == 8) sde_ln_tab_load(ln_tab);
   const int lane = threadIdx.x & 63;
   // A wave can never process more than n_items items, which bounds the loop whatever happens.
   for (int iter = 0; iter < n_items; ++iter) {
@@ -160,12 +162,12 @@ __global__ void sdesim_batch_finalize(const SdeInstance* __restrict__ inst, cons
 // Host launchers (batch runtime in runtime_batch.cpp).
 hipError_t sdesim_launch_batch(int f32, int ppl, int grid, int block, const SdeInstance* inst, const SdeItem* items,
                                int n_items, unsigned int* counter, double* partials, void* terminal,
-                               const long long* term_offset, hipStream_t stream) {
+                               const long long* term_offset, const double* ln_tab, hipStream_t stream) {
   hipLaunchKernelGGL(sdesim_batch_reset, dim3(1), dim3(64), 0, stream, counter);
 #define SDE_BATCH_CASE(R, P)                                                                            \
   if (ppl == P) {                                                                                        \
     hipLaunchKernelGGL((sdesim_batch<R, P>), dim3(grid), dim3(block), 0, stream, inst, items, n_items,     \
-                       counter, partials, (R*)terminal, term_offset);                                   \
+                       counter, partials, (R*)terminal, term_offset, ln_tab);                                \
     return hipGetLastError();                                                                            \
   }
   if (f32) {

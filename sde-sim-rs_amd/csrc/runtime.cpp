@@ -40,6 +40,7 @@ extern "C" const char* sdesim_embedded_args_header;
 extern "C" const int sdesim_jk_dims;
 extern "C" const unsigned int sdesim_jk_poly[];
 extern "C" const unsigned int sdesim_jk_vinit[];  // [dims][18]
+extern "C" const double sdesim_ln_table[];        // [256][2]
 
 // Ahead-of-time kernels (aot_kernels.hip).
 hipError_t sdesim_launch_finalize(const double* partials, int nblocks, int kq, long long S, const double* shifts,
@@ -411,6 +412,31 @@ const float* tail_table() {
   return d;
 }
 
+// The f64 kernels' logarithm table on the current device: one 4 KB copy per device, kept until exit.
+std::mutex g_ln_mu;
+std::map<int, double*> g_ln;
+
+hipError_t sdesim_ln_table_device(const double** out) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_ln_mu);
+  double*& d = g_ln[dev];
+  if (!d) {
+    double* p = nullptr;
+    e = hipMalloc(&p, 512 * sizeof(double));
+    if (e != hipSuccess) return e;
+    e = hipMemcpy(p, sdesim_ln_table, 512 * sizeof(double), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      (void)hipFree(p);
+      return e;
+    }
+    d = p;
+  }
+  *out = d;
+  return hipSuccess;
+}
+
 // Shared with the other runtime files: ChaCha8 words and host Sobol tables.
 void sdesim_chacha8_words(unsigned long long seed, size_t n, std::vector<unsigned int>& out) {
   chacha8_words(seed, n, out);
@@ -640,6 +666,7 @@ int sdesim_plan_create(const sdesim_universe* uh, const double* times, int32_t T
       }
       a.tail_tab = tail_table();
     }
+    if (!co.f32) hip_check(sdesim_ln_table_device(&a.ln_tab), "logarithm table");
     if ((opt.outputs & SDESIM_OUT_FILTRATION) &&
         (long long)P * S * (opt.precision == SDESIM_F32 ? 4 : 8) >= (1LL << 31))
       fail(SDESIM_EVALUE, "one filtration row (processes x scenarios) must be below 2 GiB; split the scenarios");

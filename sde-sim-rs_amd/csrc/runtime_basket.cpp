@@ -15,6 +15,7 @@
 
 hipError_t sdesim_launch_basket(int f32, int assets, int mode, int grid, const BasketArgs& a, int nq,
                                 double* sums, hipStream_t stream);
+hipError_t sdesim_ln_table_device(const double** out);
 int sdesim_set_error(int code, const std::string& msg);
 void sdesim_log(const char* fmt, ...);
 
@@ -135,6 +136,7 @@ int sdesim_basket_eval(sdesim_basket* b, const double* x0, const double* mu, con
     a.states = b->states;
     a.partials = b->partials;
     a.assets = A;
+    if (s.precision != SDESIM_F32) bk(sdesim_ln_table_device(&a.ln_tab), "logarithm table");
     hipStream_t st = (hipStream_t)stream;
     const int mode = !adjoint ? 0 : b->storage == SDESIM_STORAGE_TAPE ? 2 : 1;
     bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, mode, (int)b->grid, a, b->nq, b->sums, st),

@@ -13,6 +13,7 @@
 
 hipError_t sdesim_launch_lmm(int f32, int mode, int grid, const LmmArgs& a, hipStream_t stream);
 hipError_t sdesim_launch_sum_partials(const double* partials, int nblocks, int nq, double* out, hipStream_t stream);
+hipError_t sdesim_ln_table_device(const double** out);
 int sdesim_set_error(int code, const std::string& msg);
 void sdesim_log(const char* fmt, ...);
 void sdesim_host_sobol_tables(int dims, int nslices, std::vector<unsigned int>& out);
@@ -178,6 +179,7 @@ int sdesim_lmm_eval(sdesim_lmm* m, const double* L0, const double* vol, const do
     a.steps = s.steps;
     a.steps_per_period = s.steps_per_period;
     a.expiry_index = s.expiry_index;
+    if (s.precision != SDESIM_F32) lk(sdesim_ln_table_device(&a.ln_tab), "logarithm table");
     const int mode = !adjoint ? 0 : m->storage == SDESIM_STORAGE_TAPE ? 2 : 1;
     lk(sdesim_launch_lmm(s.precision == SDESIM_F32 ? 1 : 0, mode, (int)m->grid, a, st), "lmm launch");
     lk(sdesim_launch_sum_partials(m->partials, (int)m->grid, kNQ, m->sums, st), "lmm reduce");
