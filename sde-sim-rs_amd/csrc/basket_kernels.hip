@@ -102,8 +102,7 @@ __device__ __forceinline__ void basket_noise(const sde_u32 (&key)[8], int n, int
                                              BasketStep<R, D>& st) {
   sde_u32 lo[D], hi[D];
   basket_draws<D, PADDED>(key, n, A, lo, hi);
-#pragma unroll
-  for (int k = 0; k < D; ++k) st.eps[k] = sde_psi_words<R>(lo[k], hi[k]);
+  sde_psi_words<D>(lo, hi, st.eps);
 #pragma unroll
   for (int i = 0; i < D; ++i) {
     R z = R(0);
@@ -225,7 +224,7 @@ struct BasketReverse {
 template <typename R, int D, int SEG, int MODE, bool PADDED>
 __global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
   constexpr bool TAPE = MODE == 2;
-  if constexpr (sizeof(R) == 8) sde_ln_tab_load(a.ln_tab);
+  sde_normal_tab_load<R>(a.normal_tab);
   constexpr int NQ = BasketConst<D>::NQ;
   const long long S = a.paths;
   const int N = a.steps;

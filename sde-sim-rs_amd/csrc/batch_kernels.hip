@@ -55,8 +55,8 @@ __global__ void __launch_bounds__(256) sdesim_batch(const SdeInstance* __restric
                                                      unsigned int* __restrict__ counter,
                                                      double* __restrict__ partials, R* __restrict__ terminal,
                                                      const long long* __restrict__ term_offset,
-                                                     const double* __restrict__ ln_tab) {
-  if constexpr (sizeof(R) == 8) sde_ln_tab_load(ln_tab);
+                                                     const void* __restrict__ normal_tab) {
+  sde_normal_tab_load<R>(normal_tab);
   const int lane = threadIdx.x & 63;
   // A wave can never process more than n_items items, which bounds the loop whatever happens.
   for (int iter = 0; iter < n_items; ++iter) {
@@ -86,22 +86,23 @@ __global__ void __launch_bounds__(256) sdesim_batch(const SdeInstance* __restric
       sde_seed_from_u64(I.seed + (sde_u64)sid[j], key[j]);
     }
     for (int n0 = 0; n0 < N; n0 += 8) {
-      sde_u32 W[PPL][16];
+      R z[PPL][8];
 #pragma unroll
       for (int j = 0; j < PPL; ++j) {
-        sde_u32 blk[16];
+        sde_u32 blk[16], lo[8], hi[8];
         sde_chacha_block<8>(key[j], (sde_u64)(n0 / 8), blk);
 #pragma unroll
-        for (int w = 0; w < 16; ++w) W[j][w] = blk[w];
+        for (int i = 0; i < 8; ++i) {
+          lo[i] = blk[2 * i];
+          hi[i] = blk[2 * i + 1];
+        }
+        sde_psi_words<8>(lo, hi, z[j]);
       }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         if (n0 + i < N) {
 #pragma unroll
-          for (int j = 0; j < PPL; ++j) {
-            const R z = sde_psi_words<R>(W[j][2 * i], W[j][2 * i + 1]);
-            x[j] = sde_euler_builtin<R>(kind, x[j], p0, p1, p2, dt, sdt, z);
-          }
+          for (int j = 0; j < PPL; ++j) x[j] = sde_euler_builtin<R>(kind, x[j], p0, p1, p2, dt, sdt, z[j][i]);
         }
       }
     }
@@ -162,12 +163,12 @@ __global__ void sdesim_batch_finalize(const SdeInstance* __restrict__ inst, cons
 // Host launchers (batch runtime in runtime_batch.cpp).
 hipError_t sdesim_launch_batch(int f32, int ppl, int grid, int block, const SdeInstance* inst, const SdeItem* items,
                                int n_items, unsigned int* counter, double* partials, void* terminal,
-                               const long long* term_offset, const double* ln_tab, hipStream_t stream) {
+                               const long long* term_offset, const void* normal_tab, hipStream_t stream) {
   hipLaunchKernelGGL(sdesim_batch_reset, dim3(1), dim3(64), 0, stream, counter);
 #define SDE_BATCH_CASE(R, P)                                                                            \
   if (ppl == P) {                                                                                        \
     hipLaunchKernelGGL((sdesim_batch<R, P>), dim3(grid), dim3(block), 0, stream, inst, items, n_items,     \
-                       counter, partials, (R*)terminal, term_offset, ln_tab);                                \
+                       counter, partials, (R*)terminal, term_offset, normal_tab);                                \
     return hipGetLastError();                                                                            \
   }
   if (f32) {

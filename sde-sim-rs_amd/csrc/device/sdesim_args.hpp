@@ -22,7 +22,7 @@ struct SimArgs {
                              // wave-aligned XOR mode: slice 0 only, as [N][64][M]
   const sde_u32* sobol_up;   // wave-aligned XOR mode: slices 1.. as [nslices - 1][256][N * M]
   const float* tail_tab;     // [1233] |z| / sqrt(2 ln 2) of XOR uniforms with qi < 1233 (|z| > 5)
-  const double* ln_tab;      // [256][2] logarithm table of the f64 inverse normal (sde_neg2_ln)
+  const void* normal_tab;    // [256][2] logarithm table of the f64 inverse normal (SdeLn)
   const double* injected;    // [N * M][S] injected uniforms (test hook)
   void* filtration;          // [T][P][S] real, or null
   double* partials;          // [gridDim.x][2 * KQ] (sum, sum of squares) of shifted values, or null
@@ -83,7 +83,7 @@ struct BasketArgs {
   void* states;               // adjoint storage: the tape [steps][D][paths] real, or checkpoints
                               // [slots][D][paths] real (one slot per 19 steps)
   double* partials;           // [gridDim.x][NQ]
-  const double* ln_tab;       // [256][2] logarithm table (f64)
+  const void* normal_tab;     // table of the inverse normal in the kernel's precision
   int steps;
   int assets;                 // the basket's asset count A: step n uses draws n * A .. n * A + A - 1
 };
@@ -102,7 +102,7 @@ struct LmmArgs {
   void* checkpoints;                  // [slots][40][paths] real, one slot per 16 steps
   void* tape;                         // [16][40][paths] real, the states of one segment
   double* partials;                   // [gridDim.x][42]
-  const double* ln_tab;               // [256][2] logarithm table (f64)
+  const void* normal_tab;             // table of the f64 inverse normal
   int steps;
   int steps_per_period;
   int expiry_index;

@@ -218,7 +218,7 @@ template <typename R, int MODE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 1 && sizeof(R) == 4 ? 3 : 1)))
 sdesim_lmm(const LmmArgs a) {
   constexpr int NQ = 2 + NF;
-  if constexpr (sizeof(R) == 8) sde_ln_tab_load(a.ln_tab);
+  if constexpr (sizeof(R) == 8) sde_normal_tab_load<R>(a.normal_tab);
   const long long S = a.paths;
   const int N = a.steps;
   const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;

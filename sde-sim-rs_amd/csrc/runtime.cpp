@@ -386,6 +386,12 @@ int sdesim_set_error(int code, const std::string& msg) {
   return code;
 }
 
+// A&S 26.2.23 (src/proc/increment.rs:160-179): |z| of q = min(u, 1 - u) (the formula itself is defined for every q in (0, 1)).
+static double inv_normal_mag(double q) {
+  const double t = std::sqrt(-2.0 * std::log(q));
+  return t - ((0.010328 * t + 0.802853) * t + 2.515517) / (((0.001308 * t + 0.189269) * t + 1.432788) * t + 1.0);
+}
+
 // Tail values of the f32 XOR-mode increment: for qi = 0 .. 1232 (|z| > 5), the A&S inverse
 // normal (src/proc/increment.rs:160-179) of q = (qi + 0.5) 2^-32, divided by sqrt(2 ln 2) and
 // rounded to f32 (the kernel multiplies the signed sqrt(2 ln 2) sqrt(dt) back in). One copy per
@@ -401,32 +407,47 @@ const float* tail_table() {
   if (d) return d;
   std::vector<float> h(1233);
   const double c = std::sqrt(2.0 * std::log(2.0));
-  for (int qi = 0; qi < 1233; ++qi) {
-    const double q = ((double)qi + 0.5) * 0x1.0p-32;
-    const double t = std::sqrt(-2.0 * std::log(q));
-    const double x = t - ((0.010328 * t + 0.802853) * t + 2.515517) / (((0.001308 * t + 0.189269) * t + 1.432788) * t + 1.0);
-    h[qi] = (float)(x / c);
-  }
+  for (int qi = 0; qi < 1233; ++qi) h[qi] = (float)(inv_normal_mag(((double)qi + 0.5) * 0x1.0p-32) / c);
   hip_check(hipMalloc(&d, h.size() * sizeof(float)), "hipMalloc(tail table)");
   hip_check(hipMemcpy(d, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy(tail table)");
   return d;
 }
 
-// The f64 kernels' logarithm table on the current device: one 4 KB copy per device, kept until exit.
-std::mutex g_ln_mu;
-std::map<int, double*> g_ln;
+// The tables behind the device's inverse normal (SdeLn, SdePsi in sdesim_device.hpp) on the current
+// device: 4 KB (f64) and 16 KB (f32), one copy of each per device, kept until exit.
+static std::vector<float> psi_table_f32() {
+  // Segment k: the low 4 bits of v's exponent (112 .. 127 biased) and the top 6 of its mantissa.
+  // The quadratic through the segment's Chebyshev points, its middle among them.
+  std::vector<float> h(1024 * 4);
+  for (int k = 0; k < 1024; ++k) {
+    const double octave = std::ldexp(1.0, (112 + k / 64) - 127), width = octave / 64.0;
+    const double c = octave + (k % 64 + 0.5) * width, s = std::sqrt(0.75) * 0.5 * width;
+    const double f0 = inv_normal_mag(0.5 * c), fp = inv_normal_mag(0.5 * (c + s)), fm = inv_normal_mag(0.5 * (c - s));
+    h[4 * k] = (float)c;
+    h[4 * k + 1] = (float)f0;
+    h[4 * k + 2] = (float)((fp - fm) / (2.0 * s));
+    h[4 * k + 3] = (float)((fp + fm - 2.0 * f0) / (2.0 * s * s));
+  }
+  return h;
+}
 
-hipError_t sdesim_ln_table_device(const double** out) {
+std::mutex g_normal_mu;
+std::map<std::pair<int, int>, void*> g_normal;  // (device, f32)
+
+hipError_t sdesim_normal_table(int f32, const void** out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lock(g_ln_mu);
-  double*& d = g_ln[dev];
+  std::lock_guard<std::mutex> lock(g_normal_mu);
+  void*& d = g_normal[std::make_pair(dev, f32 ? 1 : 0)];
   if (!d) {
-    double* p = nullptr;
-    e = hipMalloc(&p, 512 * sizeof(double));
+    const std::vector<float> h = f32 ? psi_table_f32() : std::vector<float>();
+    const void* src = f32 ? (const void*)h.data() : (const void*)sdesim_ln_table;
+    const size_t bytes = f32 ? h.size() * sizeof(float) : 512 * sizeof(double);
+    void* p = nullptr;
+    e = hipMalloc(&p, bytes);
     if (e != hipSuccess) return e;
-    e = hipMemcpy(p, sdesim_ln_table, 512 * sizeof(double), hipMemcpyHostToDevice);
+    e = hipMemcpy(p, src, bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
       (void)hipFree(p);
       return e;
@@ -666,7 +687,7 @@ int sdesim_plan_create(const sdesim_universe* uh, const double* times, int32_t T
       }
       a.tail_tab = tail_table();
     }
-    if (!co.f32) hip_check(sdesim_ln_table_device(&a.ln_tab), "logarithm table");
+    if (!co.f32) hip_check(sdesim_normal_table(0, &a.normal_tab), "inverse normal table");
     if ((opt.outputs & SDESIM_OUT_FILTRATION) &&
         (long long)P * S * (opt.precision == SDESIM_F32 ? 4 : 8) >= (1LL << 31))
       fail(SDESIM_EVALUE, "one filtration row (processes x scenarios) must be below 2 GiB; split the scenarios");

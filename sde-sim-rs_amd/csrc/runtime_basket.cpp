@@ -15,7 +15,7 @@
 
 hipError_t sdesim_launch_basket(int f32, int assets, int mode, int grid, const BasketArgs& a, int nq,
                                 double* sums, hipStream_t stream);
-hipError_t sdesim_ln_table_device(const double** out);
+hipError_t sdesim_normal_table(int f32, const void** out);
 int sdesim_set_error(int code, const std::string& msg);
 void sdesim_log(const char* fmt, ...);
 
@@ -51,6 +51,7 @@ struct sdesim_basket {
   void* states = nullptr;                   // the tape or the checkpoints
   double* partials = nullptr;
   double* sums = nullptr;
+  const void* normal_tab = nullptr;         // the device's shared table of the inverse normal
   ~sdesim_basket() {
     if (states) (void)hipFree(states);
     if (partials) (void)hipFree(partials);
@@ -98,6 +99,7 @@ int sdesim_basket_create(const sdesim_basket_spec* spec, sdesim_basket** out) {
       if (ck + (64u << 20) > free_b) throw BFail{SDESIM_ERUNTIME, "checkpoints do not fit in free device memory"};
       bk(hipMalloc(&b->states, ck), "hipMalloc(checkpoints)");
     }
+    bk(sdesim_normal_table(s.precision == SDESIM_F32 ? 1 : 0, &b->normal_tab), "inverse normal table");
     bk(hipMalloc(&b->partials, sizeof(double) * b->nq * b->grid), "hipMalloc(partials)");
     bk(hipMalloc(&b->sums, sizeof(double) * b->nq), "hipMalloc(sums)");
     sdesim_log("basket: %d assets, %lld paths, %d steps, adjoint storage %s", s.assets, (long long)s.paths, s.steps,
@@ -136,7 +138,7 @@ int sdesim_basket_eval(sdesim_basket* b, const double* x0, const double* mu, con
     a.states = b->states;
     a.partials = b->partials;
     a.assets = A;
-    if (s.precision != SDESIM_F32) bk(sdesim_ln_table_device(&a.ln_tab), "logarithm table");
+    a.normal_tab = b->normal_tab;
     hipStream_t st = (hipStream_t)stream;
     const int mode = !adjoint ? 0 : b->storage == SDESIM_STORAGE_TAPE ? 2 : 1;
     bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, mode, (int)b->grid, a, b->nq, b->sums, st),

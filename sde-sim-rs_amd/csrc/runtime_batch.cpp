@@ -28,8 +28,8 @@
 
 hipError_t sdesim_launch_batch(int f32, int ppl, int grid, int block, const SdeInstance* inst, const SdeItem* items,
                                int n_items, unsigned int* counter, double* partials, void* terminal,
-                               const long long* term_offset, const double* ln_tab, hipStream_t stream);
-hipError_t sdesim_ln_table_device(const double** out);
+                               const long long* term_offset, const void* normal_tab, hipStream_t stream);
+hipError_t sdesim_normal_table(int f32, const void** out);
 hipError_t sdesim_launch_batch_finalize(const SdeInstance* inst, const int* slot0, int n, const double* partials,
                                         double* out, hipStream_t stream);
 hipError_t sdesim_batch_occupancy(int f32, int ppl, int block, int* blocks_per_cu);
@@ -121,7 +121,7 @@ struct sdesim_batch {
   double* d_partials = nullptr;
   double* d_moments = nullptr;
   long long* d_term_off = nullptr;
-  const double* ln_tab = nullptr;  // f64: the device's shared logarithm table
+  const void* normal_tab = nullptr;  // the device's shared table of the inverse normal
   void* d_terminal = nullptr;
   bool keep_terminal = false;
   hipStream_t capture_stream = nullptr;
@@ -189,7 +189,7 @@ struct sdesim_batch {
 
   void launch(hipStream_t s) {
     bcheck(sdesim_launch_batch(f32, ppl, grid, block, d_inst, d_items, n_items, d_counter, d_partials,
-                               keep_terminal ? d_terminal : nullptr, d_term_off, ln_tab, s),
+                               keep_terminal ? d_terminal : nullptr, d_term_off, normal_tab, s),
            "batch launch");
     bcheck(sdesim_launch_batch_finalize(d_inst, d_slot0, n, d_partials, d_moments, s), "batch finalize");
   }
@@ -238,7 +238,7 @@ int sdesim_batch_create(const sdesim_instance* inst, int32_t n, int32_t precisio
     char kb[64];
     std::snprintf(kb, sizeof kb, "%s-%d-%016llx", b->f32 ? "f32" : "f64", n, sig);
     b->key = kb;
-    if (!b->f32) bcheck(sdesim_ln_table_device(&b->ln_tab), "logarithm table");
+    bcheck(sdesim_normal_table(b->f32, &b->normal_tab), "inverse normal table");
     bcheck(hipMalloc(&b->d_inst, sizeof(SdeInstance) * n), "hipMalloc(instances)");
     bcheck(hipMemcpy(b->d_inst, b->host.data(), sizeof(SdeInstance) * n, hipMemcpyHostToDevice), "hipMemcpy");
     bcheck(hipMalloc(&b->d_term_off, sizeof(long long) * (n + 1)), "hipMalloc(offsets)");

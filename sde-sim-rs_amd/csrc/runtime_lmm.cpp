@@ -13,7 +13,7 @@
 
 hipError_t sdesim_launch_lmm(int f32, int mode, int grid, const LmmArgs& a, hipStream_t stream);
 hipError_t sdesim_launch_sum_partials(const double* partials, int nblocks, int nq, double* out, hipStream_t stream);
-hipError_t sdesim_ln_table_device(const double** out);
+hipError_t sdesim_normal_table(int f32, const void** out);
 int sdesim_set_error(int code, const std::string& msg);
 void sdesim_log(const char* fmt, ...);
 void sdesim_host_sobol_tables(int dims, int nslices, std::vector<unsigned int>& out);
@@ -56,6 +56,7 @@ struct sdesim_lmm {
   float* parf = nullptr;
   double* partials = nullptr;
   double* sums = nullptr;
+  const void* normal_tab = nullptr;  // f64: the device's shared table of the inverse normal
   ~sdesim_lmm() {
     for (void* p : {(void*)tab, (void*)tabup, ckpt, tape, (void*)pard, (void*)parf, (void*)partials, (void*)sums})
       if (p) (void)hipFree(p);
@@ -129,6 +130,7 @@ int sdesim_lmm_create(const sdesim_lmm_spec* spec, sdesim_lmm** out) {
     }
     lk(hipMalloc(&m->pard, sizeof(double) * kNF * (1 + kF)), "hipMalloc(parameters)");
     lk(hipMalloc(&m->parf, sizeof(float) * kNF * (1 + kF)), "hipMalloc(parameters)");
+    if (s.precision != SDESIM_F32) lk(sdesim_normal_table(0, &m->normal_tab), "inverse normal table");
     lk(hipMalloc(&m->partials, sizeof(double) * kNQ * m->grid), "hipMalloc(partials)");
     lk(hipMalloc(&m->sums, sizeof(double) * kNQ), "hipMalloc(sums)");
     sdesim_log("forward-rate model: %lld paths, %d steps, adjoint storage %s", (long long)s.paths, s.steps,
@@ -179,7 +181,7 @@ int sdesim_lmm_eval(sdesim_lmm* m, const double* L0, const double* vol, const do
     a.steps = s.steps;
     a.steps_per_period = s.steps_per_period;
     a.expiry_index = s.expiry_index;
-    if (s.precision != SDESIM_F32) lk(sdesim_ln_table_device(&a.ln_tab), "logarithm table");
+    a.normal_tab = m->normal_tab;
     const int mode = !adjoint ? 0 : m->storage == SDESIM_STORAGE_TAPE ? 2 : 1;
     lk(sdesim_launch_lmm(s.precision == SDESIM_F32 ? 1 : 0, mode, (int)m->grid, a, st), "lmm launch");
     lk(sdesim_launch_sum_partials(m->partials, (int)m->grid, kNQ, m->sums, st), "lmm reduce");

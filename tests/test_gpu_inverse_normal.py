@@ -64,3 +64,22 @@ def test_edge_words_match_the_oracle(oracle, word):
     got = _draws(S, "sobol", "f64", **kw)
     ref = oracle.simulate(NOISE, TIMES, S, {"X": 0.0}, rng="sobol", **kw)[:, 1, 0]
     assert np.all(np.abs(got - ref) <= _bound(ref)), (got, ref)
+
+
+@pytest.mark.parametrize("paths", [1, 65, (1 << 18) + 3])
+def test_batched_f32_draws_match_the_oracle(oracle, paths):
+    """One-step f32 OU instances with dX = 1 dW (kappa = 0, sigma = 1): the terminal value is the draw.
+    2^18 draws reach the rare path (|z| > 4.17) about eight times. Bound: the f32 rational's of
+    fp32_bounds, which the rare draws take, plus one rounding; the table's quadratics round less often and
+    take the same q."""
+    import sde_sim_rs
+    import fp32_bounds as B
+    print("case: batched f32 draws, %d paths" % paths, flush=True)
+    inst = dict(kind=1, steps=1, paths=paths, x0=0.0, horizon=1.0, p0=0.0, p1=0.0, p2=1.0, seed=77)
+    b = sde_sim_rs.Batch([inst], precision="f32", keep_terminal=True)
+    b.run()
+    got = b.terminal().astype(np.float64)
+    u = np.array([oracle.pseudo_f64(77 + s, 1)[0] for s in range(paths)])
+    z = B.inv_normal(u)
+    bound = B.psi_error_words(u) + B.U * np.abs(z)
+    assert np.all(np.abs(got - z) <= bound), np.max(np.abs(got - z) / bound)
