@@ -26,7 +26,7 @@ namespace {
 // state once, as the generated FP32 kernels do: added alone, a drift of a few ulps of x per step
 // (GBM with mu dt ~ 3e-7) is rounded to whole ulps at every step in the same direction, which
 // biased a 1000-step GBM mean by 1.5e-5.
-template <typename R>
+template <typename R, bool LIB>
 __device__ __forceinline__ R sde_euler_builtin(int kind, R x, R p0, R p1, R p2, R dt, R sdt, R z) {
   R v0, v1;
   if (kind == 0) {
@@ -37,7 +37,8 @@ __device__ __forceinline__ R sde_euler_builtin(int kind, R x, R p0, R p1, R p2, 
     v1 = p2;
   } else {
     v0 = p0 * (p1 + (-sde_fmax(x, R(0))));
-    v1 = p2 * sde_sqrt(sde_fmax(x, R(0)));
+    if constexpr (LIB) v1 = p2 * sqrt(sde_fmax(x, R(0)));
+    else v1 = p2 * sde_sqrt(sde_fmax(x, R(0)));
   }
   if constexpr (sizeof(R) == 4) {
     return x + (v0 * dt + v1 * (sdt * z));
@@ -46,6 +47,40 @@ __device__ __forceinline__ R sde_euler_builtin(int kind, R x, R p0, R p1, R p2, 
     a0 = a0 + v0 * dt;
     a0 = a0 + v1 * (sdt * z);
     return a0;
+  }
+}
+
+// All steps of a wave's 64 * PPL paths.
+template <typename R, int PPL, bool LIB>
+__device__ __forceinline__ void batch_steps(const sde_u32 (&key)[PPL][8], int N, int kind, R (&x)[PPL], R p0, R p1, R p2,
+                                            R dt, R sdt) {
+  for (int n0 = 0; n0 < N; n0 += 8) {
+    sde_u32 lo[PPL][8], hi[PPL][8];
+    R z[PPL][8];
+#pragma unroll
+    for (int j = 0; j < PPL; ++j) {
+      sde_u32 blk[16];
+      sde_chacha_block<8>(key[j], (sde_u64)(n0 / 8), blk);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        lo[j][i] = blk[2 * i];
+        hi[j][i] = blk[2 * i + 1];
+      }
+      // f32: one test for rare draws per ChaCha block. f64 draws are taken one by one below (100
+      // registers; all eight at once take 138).
+      if constexpr (sizeof(R) == 4) sde_psi_words<8>(lo[j], hi[j], z[j]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (n0 + i < N) {
+#pragma unroll
+        for (int j = 0; j < PPL; ++j) {
+          if constexpr (LIB) z[j][i] = sde_inv_normal(sde_u01_from_words(lo[j][i], hi[j][i]));
+          else if constexpr (sizeof(R) == 8) z[j][i] = sde_psi_word(lo[j][i], hi[j][i]);
+          x[j] = sde_euler_builtin<R, LIB>(kind, x[j], p0, p1, p2, dt, sdt, z[j][i]);
+        }
+      }
+    }
   }
 }
 
@@ -85,26 +120,14 @@ __global__ void __launch_bounds__(256) sdesim_batch(const SdeInstance* __restric
       x[j] = (R)I.x0;
       sde_seed_from_u64(I.seed + (sde_u64)sid[j], key[j]);
     }
-    for (int n0 = 0; n0 < N; n0 += 8) {
-      R z[PPL][8];
-#pragma unroll
-      for (int j = 0; j < PPL; ++j) {
-        sde_u32 blk[16], lo[8], hi[8];
-        sde_chacha_block<8>(key[j], (sde_u64)(n0 / 8), blk);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          lo[i] = blk[2 * i];
-          hi[i] = blk[2 * i + 1];
-        }
-        sde_psi_words<8>(lo, hi, z[j]);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (n0 + i < N) {
-#pragma unroll
-          for (int j = 0; j < PPL; ++j) x[j] = sde_euler_builtin<R>(kind, x[j], p0, p1, p2, dt, sdt, z[j][i]);
-        }
-      }
+    // A CIR instance whose rounding differences grow (4 kappa theta < sigma^2: reaches_root in
+    // codegen.hpp) keeps the library's logarithm, root and division in f64.
+    bool lib = false;
+    if constexpr (sizeof(R) == 8) lib = kind == 2 && 4.0 * (I.p0 * I.p1) < I.p2 * I.p2;
+    if (lib) {
+      if constexpr (sizeof(R) == 8) batch_steps<R, PPL, true>(key, N, kind, x, p0, p1, p2, dt, sdt);
+    } else {
+      batch_steps<R, PPL, false>(key, N, kind, x, p0, p1, p2, dt, sdt);
     }
     double acc[2] = {0.0, 0.0};
 #pragma unroll

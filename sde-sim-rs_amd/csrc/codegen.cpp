@@ -483,6 +483,7 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
   const int NK = carried.empty() ? 1 : (int)carried.size();
 
   std::ostringstream s;
+  if (o.library_f64) s << "#define SDE_LIBRARY_F64 1\n";
   s << "#include \"sdesim_device.hpp\"\n\n";
   s << "struct SdeModel {\n";
   s << "  typedef " << R << " real;\n";
@@ -523,6 +524,37 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
     << (o.uniform_grid ? "true" : "false") << ", " << (o.wave_aligned ? "true" : "false") << ">(a);\n";
   s << "}\n";
   return s.str();
+}
+
+bool reaches_root(const Universe& u, const std::vector<double>& x0, double t0) {
+  std::map<std::string, double> ns;
+  for (const auto& kv : u.registry) ns[kv.first] = kv.second < (int)x0.size() ? x0[kv.second] : 0.0;
+  ns.emplace("t", t0);
+  // Sum of process p's terms of one kind at the point (squared for noise).
+  auto sum = [&](const ProcessDef& pd, IncKind kind, double x) {
+    ns[pd.name] = x;
+    double v = 0.0;
+    for (const Term& t : pd.terms) {
+      if (t.kind != kind) continue;
+      const double c = eval_host(*t.coef, ns);
+      v += kind == IncKind::Time ? c : c * c;
+    }
+    return v;
+  };
+  for (const ProcessDef& pd : u.processes) {
+    if (!pd.levy) continue;
+    const double own = ns[pd.name];
+    try {
+      const double at0 = sum(pd, IncKind::Wiener, 0.0);
+      const double s2 = sum(pd, IncKind::Wiener, 0x1.0p-40) * 0x1.0p40;
+      const double closer = sum(pd, IncKind::Wiener, 0x1.0p-42) * 0x1.0p42;
+      if (at0 == 0.0 && s2 > 0.0 && closer >= 0.99 * s2 && 4.0 * sum(pd, IncKind::Time, 0.0) < s2) return true;
+    } catch (const std::exception&) {
+      // A coefficient that does not evaluate fails where the kernel is generated.
+    }
+    ns[pd.name] = own;
+  }
+  return false;
 }
 
 std::string kernel_name(const CodegenOptions& o) {

@@ -18,6 +18,7 @@ struct CodegenOptions {
   int nsl = 1;          // Sobol table slices (Gray-code bits covered: 6 + 8 (nsl - 1))
   bool uniform_grid = false;  // every dt and sqrt(dt) is bitwise equal in the kernel's precision
   bool wave_aligned = false;  // Sobol index of path 0 is a multiple of 64 and blocks hold whole waves
+  bool library_f64 = false;   // f64: library logarithm and roots (reaches_root below)
   bool steps = true;    // false when the time grid has a single point (nothing is evaluated)
   std::string payoff;   // expression over process names and t at the last time point
   std::string name = "sdesim_kernel";  // entry point name
@@ -39,5 +40,16 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o);
 
 // Descriptive entry point name: sdesim_<em|rk>_<f32|f64>_<rng>_<filt|term|filt_term>.
 std::string kernel_name(const CodegenOptions& o);
+
+// Whether a process of the universe has noise that vanishes at 0 like a root and a drift there too weak
+// to keep rounding differences from growing: with b(x)^2 / x -> s^2 and drift a as x -> 0 (the
+// other processes at x0, time t0), 4 a < s^2. An Euler path that steps out of 0 lands at about
+// a dt, where its next increment changes by s sqrt(dt) / (2 sqrt(a dt)) = s / (2 sqrt(a)) of any
+// difference: above 1, two copies of a path that differ in one last bit drift apart without bound
+// (CIR with 2 a / s^2 = 0.09: 0.1 apart after 1550 steps), below 1 they come together (Heston's
+// variance at 0.64: 1e-15 after 1024). The f64 kernels of such universes, and the batch kernel's
+// CIR instances, keep the library's logarithm, root and division, so that their paths stay bit for bit
+// those of the general inverse normal.
+bool reaches_root(const Universe& u, const std::vector<double>& x0, double t0);
 
 }  // namespace sdesim

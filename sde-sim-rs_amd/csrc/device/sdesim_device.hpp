@@ -282,15 +282,17 @@ __device__ __forceinline__ void sde_normal_tab_load(const void* src) {
   else sde_psi_tab_load(src);
 }
 
-// Psi of N pseudo-random draws held as their ChaCha words.
-template <int N>
-__device__ __forceinline__ void sde_psi_words(const sde_u32 (&lo)[N], const sde_u32 (&hi)[N], double (&z)[N]) {
+// Psi of pseudo-random draws held as their ChaCha words.
+__device__ __forceinline__ double sde_psi_word(sde_u32 lo, sde_u32 hi) {
   // u - 1/2: the two exact products of sde_u01_from_words with hi's offset taken off its signed
   // conversion.
+  return sde_inv_normal_d<true>(
+      __builtin_fma((double)(int)(hi ^ 0x80000000u), 0x1.0p-32, (double)(lo >> 11) * 0x1.0p-53));
+}
+template <int N>
+__device__ __forceinline__ void sde_psi_words(const sde_u32 (&lo)[N], const sde_u32 (&hi)[N], double (&z)[N]) {
 #pragma unroll
-  for (int k = 0; k < N; ++k)
-    z[k] = sde_inv_normal_d<true>(
-        __builtin_fma((double)(int)(hi[k] ^ 0x80000000u), 0x1.0p-32, (double)(lo[k] >> 11) * 0x1.0p-53));
+  for (int k = 0; k < N; ++k) z[k] = sde_psi_word(lo[k], hi[k]);
 }
 template <int N>
 __device__ __forceinline__ void sde_psi_words(const sde_u32 (&lo)[N], const sde_u32 (&hi)[N], float (&z)[N]) {
@@ -426,12 +428,7 @@ __device__ __forceinline__ double sde_dw(double u, double sdt) { return sdt * sd
 __device__ __forceinline__ float sde_dw(double u, float sdt) { return sdt * sde_inv_normal_f32(u); }
 __device__ __forceinline__ double sde_dw(SdeUnifD u, double sdt) { return sdt * sde_inv_normal_d<true>(u.u - 0.5); }
 __device__ __forceinline__ double sde_dw(SdeUnifX u, double sdt) { return sdt * sde_psi<double>(u); }
-__device__ __forceinline__ double sde_dw(SdeUnifW u, double sdt) {
-  const sde_u32 lo[1] = {u.lo}, hi[1] = {u.hi};
-  double z[1];
-  sde_psi_words<1>(lo, hi, z);
-  return sdt * z[0];
-}
+__device__ __forceinline__ double sde_dw(SdeUnifW u, double sdt) { return sdt * sde_psi_word(u.lo, u.hi); }
 __device__ __forceinline__ float sde_dw(SdeUnifW u, float sdt) { return sdt * sde_inv_normal_f32_words(u.lo, u.hi); }
 __device__ __forceinline__ float sde_dw(SdeUnifX u, float sdt) {
   return sde_sign_select(u.yc, sdt * (float)SDE_PSI_C, u.sm) * sde_inv_normal_f32_x_scaled(u.yc, u.tail);
@@ -486,6 +483,9 @@ template <typename R> __device__ __forceinline__ R sde_add_strict(R a, R b) { re
 // as sqrt does (below 2^-960 the residual underflows and the 0.75 ulp stay). +-0 and infinity
 // return themselves, negative values NaN. 12 instructions instead of 18: no scaling.
 __device__ __forceinline__ double sde_sqrt(double a) {
+#ifdef SDE_LIBRARY_F64
+  return sqrt(a);
+#endif
   const double y = __builtin_amdgcn_rsq(a);
   double t = a * y;
   const double e = __builtin_fma(-t, y, 1.0);
@@ -582,11 +582,18 @@ typedef sde_u32 SdeU32x2 __attribute__((ext_vector_type(2)));
 // The uniform a step consumes: pseudo-random draws (and, in FP32, Sobol points with the random
 // shift) as two 32-bit words of a 53-bit fraction, XOR-scrambled Sobol points as their word,
 // otherwise an f64 value.
+// SDE_LIBRARY_F64 (defined by the generated source of a universe whose paths part from any difference
+// in a last bit, reaches_root in codegen.hpp): f64 kernels keep the uniform's f64 value, and with
+// it the general inverse normal.
 template <int RNG, typename R> struct SdeUnifOf { typedef double type; };
-template <typename R> struct SdeUnifOf<SDE_RNG_SOBOL_XOR, R> { typedef SdeUnifX type; };
-template <typename R> struct SdeUnifOf<SDE_RNG_PSEUDO, R> { typedef SdeUnifW type; };
-template <> struct SdeUnifOf<SDE_RNG_SOBOL_SHIFT, float> { typedef SdeUnifW type; };
+#ifndef SDE_LIBRARY_F64
+template <> struct SdeUnifOf<SDE_RNG_SOBOL_XOR, double> { typedef SdeUnifX type; };
+template <> struct SdeUnifOf<SDE_RNG_PSEUDO, double> { typedef SdeUnifW type; };
 template <> struct SdeUnifOf<SDE_RNG_SOBOL_SHIFT, double> { typedef SdeUnifD type; };
+#endif
+template <> struct SdeUnifOf<SDE_RNG_SOBOL_XOR, float> { typedef SdeUnifX type; };
+template <> struct SdeUnifOf<SDE_RNG_PSEUDO, float> { typedef SdeUnifW type; };
+template <> struct SdeUnifOf<SDE_RNG_SOBOL_SHIFT, float> { typedef SdeUnifW type; };
 
 template <typename R>
 struct SdeGrid {
@@ -660,8 +667,13 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
   constexpr int NB = SdeChunk<M>::BLOCKS;
   constexpr int KQ = P + (Mdl::HAS_PAYOFF ? 1 : 0);
   constexpr bool FILT = (OUT & SDE_OUT_FILTRATION) != 0;
+#ifdef SDE_LIBRARY_F64
+  constexpr bool LIB = sizeof(real) == 8;
+#else
+  constexpr bool LIB = false;
+#endif
 
-  if constexpr (sizeof(real) == 8 && (USE_CHACHA || USE_SOBOL)) sde_normal_tab_load<real>(a.normal_tab);
+  if constexpr (sizeof(real) == 8 && (USE_CHACHA || USE_SOBOL) && !LIB) sde_normal_tab_load<real>(a.normal_tab);
 
   const long long S = a.S;
   const int N = a.N;
@@ -845,7 +857,16 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
             } else if (USE_INJ) {
               v = ni[j][k];
             }
-            if constexpr (RNG == SDE_RNG_SOBOL_XOR) {
+            if constexpr (LIB) {
+              if constexpr (RNG == SDE_RNG_SOBOL_XOR) {
+                u[j][k] = sde_uval(SdeUnifX{nx[j][k], nullptr, 0u, 0u});
+              } else if constexpr (RNG == SDE_RNG_PSEUDO) {
+                const int w = 2 * (i * M + k);
+                u[j][k] = sde_u01_from_words(W[j][USE_CHACHA ? w : 0], W[j][USE_CHACHA ? w + 1 : 0]);
+              } else {
+                u[j][k] = v;
+              }
+            } else if constexpr (RNG == SDE_RNG_SOBOL_XOR) {
               u[j][k].yc = nx[j][k];
               u[j][k].tail = a.tail_tab;
               u[j][k].sm = smask;

@@ -626,13 +626,14 @@ int sdesim_plan_create(const sdesim_universe* uh, const double* times, int32_t T
       else ug = std::memcmp(&dts[n], &dts[0], 8) == 0 && std::memcmp(&sdts[n], &sdts[0], 8) == 0;
     }
     co.uniform_grid = ug;
+    std::vector<double> x0v(x0 ? x0 : nullptr, x0 ? x0 + P : nullptr);
+    if (!x0) x0v.assign(P, 0.0);
+    if (x0v.empty()) x0v.push_back(0.0);
+    co.library_f64 = !co.f32 && sdesim::reaches_root(U, x0v, tv[0]);
     co.name = sdesim::kernel_name(co);
     plan->source = sdesim::generate_kernel_source(U, co);
     plan->kname = co.name;
     plan->kernel = compile_kernel(plan->source, co.name);
-    std::vector<double> x0v(x0 ? x0 : nullptr, x0 ? x0 + P : nullptr);
-    if (!x0) x0v.assign(P, 0.0);
-    if (x0v.empty()) x0v.push_back(0.0);
 
     SimArgs& a = plan->args;
     a.times = plan->own(upload(tv));
