@@ -11,6 +11,7 @@
 #include <mutex>
 
 #include "../../include/sdesim.h"
+#include "reduce.hpp"
 
 // Per-block terminal partials of sdesim_plan_run_scratch, which may not allocate: a fixed array in
 // the library's code object, SDESIM_SCRATCH_BYTES per device (each device that runs the library
@@ -20,37 +21,27 @@ static __device__ __align__(256) double scratch[SDESIM_SCRATCH_BYTES / sizeof(do
 
 namespace {
 
-struct Neumaier {
-  double s = 0.0, c = 0.0;
-  __device__ void add(double x) {
-    const double t = s + x;
-    c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
-    s = t;
-  }
-  __device__ double value() const { return s + c; }
-};
-
-// One block per reduced quantity q; 256 threads.
-__global__ void __launch_bounds__(256) sdesim_finalize(const double* __restrict__ partials, int nblocks, int kq,
-                                                       long long S, const double* __restrict__ shifts,
-                                                       double* __restrict__ out) {
+// One block of 1024 threads per reduced quantity q.
+__global__ void __launch_bounds__(1024) sdesim_finalize(const double* __restrict__ partials, int nblocks, int kq,
+                                                        long long S, const double* __restrict__ shifts,
+                                                        double* __restrict__ out) {
   const int q = blockIdx.x;
-  Neumaier s1, s2;
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  SdeSum s1, s2;
+#pragma unroll 4
   for (int b = threadIdx.x; b < nblocks; b += blockDim.x) {
-    s1.add(partials[(long long)b * 2 * kq + 2 * q]);
-    s2.add(partials[(long long)b * 2 * kq + 2 * q + 1]);
+    const D2 v = *(const D2*)(partials + ((long long)b * kq + q) * 2);
+    s1.add(v.x);
+    s2.add(v.y);
   }
-  __shared__ double a1[256], c1[256], a2[256], c2[256];
-  a1[threadIdx.x] = s1.s; c1[threadIdx.x] = s1.c;
-  a2[threadIdx.x] = s2.s; c2[threadIdx.x] = s2.c;
-  __syncthreads();
+  __shared__ double sh1[16][2], sh2[16][2];
+  sde_block_sum(s1, sh1);
+  sde_block_sum(s2, sh2);
   if (threadIdx.x == 0) {
-    Neumaier t1, t2;
-    for (int i = 0; i < (int)blockDim.x; ++i) { t1.add(a1[i]); t1.add(c1[i]); t2.add(a2[i]); t2.add(c2[i]); }
     const double n = (double)S;
-    const double m1 = t1.value() / n;
+    const double m1 = s1.value() / n;
     out[2 * q] = shifts[q] + m1;
-    out[2 * q + 1] = S > 1 ? (t2.value() - t1.value() * m1) / (n - 1.0) : 0.0;
+    out[2 * q + 1] = S > 1 ? (s2.value() - s1.value() * m1) / (n - 1.0) : 0.0;
   }
 }
 
@@ -149,7 +140,7 @@ hipError_t sdesim_scratch_address(double** ptr, size_t* bytes) {
 
 hipError_t sdesim_launch_finalize(const double* partials, int nblocks, int kq, long long S, const double* shifts,
                                   double* out, hipStream_t stream) {
-  hipLaunchKernelGGL(sdesim_finalize, dim3(kq), dim3(256), 0, stream, partials, nblocks, kq, S, shifts, out);
+  hipLaunchKernelGGL(sdesim_finalize, dim3(kq), dim3(nblocks > 256 ? 1024 : 256), 0, stream, partials, nblocks, kq, S, shifts, out);
   return hipGetLastError();
 }
 

@@ -29,6 +29,7 @@
 
 #include "device/sdesim_device.hpp"
 #include "adjoint.hpp"
+#include "reduce.hpp"
 
 namespace {
 
@@ -344,32 +345,18 @@ __global__ void __launch_bounds__(256) sdesim_basket_reverse(const BasketArgs a)
       a.partials + (long long)blockIdx.x * NQ);
 }
 
-// Sum of per-block partials per quantity (one block per quantity, Neumaier-compensated).
-__global__ void __launch_bounds__(256) sdesim_sum_partials(const double* __restrict__ partials, int nblocks, int nq,
-                                                           double* __restrict__ out) {
+// Sum of per-block partials per quantity: one block of 1024 threads each, whose loads of 8 bytes
+// from rows of nq values are all in flight together (the quantities' blocks read the same lines
+// through L2).
+__global__ void __launch_bounds__(1024) sdesim_sum_partials(const double* __restrict__ partials, int nblocks, int nq,
+                                                            double* __restrict__ out) {
   const int q = blockIdx.x;
-  double s = 0.0, c = 0.0;
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x) {
-    const double x = partials[(long long)b * nq + q];
-    const double t = s + x;
-    c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
-    s = t;
-  }
-  __shared__ double sh[256], shc[256];
-  sh[threadIdx.x] = s;
-  shc[threadIdx.x] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double S = 0.0, C = 0.0;
-    for (int i = 0; i < (int)blockDim.x; ++i) {
-      for (double x : {sh[i], shc[i]}) {
-        const double t = S + x;
-        C += (fabs(S) >= fabs(x)) ? (S - t) + x : (x - t) + S;
-        S = t;
-      }
-    }
-    out[q] = S + C;
-  }
+  SdeSum a;
+#pragma unroll 8
+  for (int b = threadIdx.x; b < nblocks; b += blockDim.x) a.add(partials[(long long)b * nq + q]);
+  __shared__ double sh[16][2];
+  sde_block_sum(a, sh);
+  if (threadIdx.x == 0) out[q] = a.value();
 }
 
 }  // namespace
@@ -411,11 +398,11 @@ hipError_t sdesim_launch_basket(int f32, int assets, int mode, int grid, const B
   if (!ok) return hipErrorInvalidValue;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(sdesim_sum_partials, dim3(nq), dim3(256), 0, stream, a.partials, grid, nq, sums);
+  hipLaunchKernelGGL(sdesim_sum_partials, dim3(nq), dim3(grid > 256 ? 1024 : 256), 0, stream, a.partials, grid, nq, sums);
   return hipGetLastError();
 }
 
 hipError_t sdesim_launch_sum_partials(const double* partials, int nblocks, int nq, double* out, hipStream_t stream) {
-  hipLaunchKernelGGL(sdesim_sum_partials, dim3(nq), dim3(256), 0, stream, partials, nblocks, nq, out);
+  hipLaunchKernelGGL(sdesim_sum_partials, dim3(nq), dim3(nblocks > 256 ? 1024 : 256), 0, stream, partials, nblocks, nq, out);
   return hipGetLastError();
 }

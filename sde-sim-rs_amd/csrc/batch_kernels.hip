@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include "device/sdesim_device.hpp"
+#include "reduce.hpp"
 
 namespace {
 
@@ -155,30 +156,31 @@ __global__ void sdesim_batch_reset(unsigned int* counter) {
   if (threadIdx.x == 0 && blockIdx.x == 0) counter[0] = 0u;
 }
 
-struct Neumaier {
-  double s = 0.0, c = 0.0;
-  __device__ void add(double x) {
-    const double t = s + x;
-    c += (fabs(s) >= fabs(x)) ? (s - t) + x : (x - t) + s;
-    s = t;
-  }
-};
-
-// One thread per instance: its item slots are [slot0[i], slot0[i+1]).
-__global__ void sdesim_batch_finalize(const SdeInstance* __restrict__ inst, const int* __restrict__ slot0, int n,
-                                      const double* __restrict__ partials, double* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// One wave per instance: its item slots are [slot0[i], slot0[i+1]).
+__global__ void __launch_bounds__(256) sdesim_batch_finalize(const SdeInstance* __restrict__ inst,
+                                                             const int* __restrict__ slot0, int n,
+                                                             const double* __restrict__ partials,
+                                                             double* __restrict__ out) {
+  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), lane = threadIdx.x & 63;
   if (i >= n) return;
-  Neumaier a, b;
-  for (int s = slot0[i]; s < slot0[i + 1]; ++s) {
-    a.add(partials[2 * (long long)s]);
-    b.add(partials[2 * (long long)s + 1]);
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  SdeSum a, b;
+  const int end = slot0[i + 1];
+#pragma unroll 4
+  for (int s = slot0[i] + lane; s < end; s += 64) {
+    const D2 v = *(const D2*)(partials + 2 * (long long)s);
+    a.add(v.x);
+    b.add(v.y);
   }
-  const double S = (double)inst[i].paths;
-  const double s1 = a.s + a.c, s2 = b.s + b.c;
-  const double m1 = s1 / S;
-  out[2 * i] = inst[i].x0 + m1;
-  out[2 * i + 1] = S > 1.0 ? (s2 - s1 * m1) / (S - 1.0) : 0.0;
+  sde_wave_sum(a);
+  sde_wave_sum(b);
+  if (lane == 0) {
+    const double S = (double)inst[i].paths;
+    const double s1 = a.value(), s2 = b.value();
+    const double m1 = s1 / S;
+    out[2 * i] = inst[i].x0 + m1;
+    out[2 * i + 1] = S > 1.0 ? (s2 - s1 * m1) / (S - 1.0) : 0.0;
+  }
 }
 
 }  // namespace
@@ -209,7 +211,7 @@ hipError_t sdesim_launch_batch(int f32, int ppl, int grid, int block, const SdeI
 
 hipError_t sdesim_launch_batch_finalize(const SdeInstance* inst, const int* slot0, int n, const double* partials,
                                         double* out, hipStream_t stream) {
-  hipLaunchKernelGGL(sdesim_batch_finalize, dim3((n + 255) / 256), dim3(256), 0, stream, inst, slot0, n, partials,
+  hipLaunchKernelGGL(sdesim_batch_finalize, dim3((n + 3) / 4), dim3(256), 0, stream, inst, slot0, n, partials,
                      out);
   return hipGetLastError();
 }
