@@ -27,6 +27,8 @@
 //   eps_n = L^-1 Z_n (forward substitution),  Lbar_ik += Zbar_{n,i} eps_{n,k}  (k <= i)
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device/sdesim_device.hpp"
 #include "adjoint.hpp"
 #include "reduce.hpp"
@@ -39,11 +41,10 @@ struct BasketConst {
   static constexpr int NQ = 2 + 3 * D + NL;    // reduced quantities: payoff, payoff^2, gradients
 };
 
-// The words (low, high) of the D f64 draws of step n: draws n*D .. n*D + D - 1 of the path's
-// stream (draw j is words 2j and 2j + 1). PADDED (D = 8 holding A < 8 assets, the rest padding
-// with zero weight): step n uses draws n*A .. n*A + A - 1, as the DSL form with A Wiener
-// increments does; they lie in ChaCha blocks (n*A) / 8 and the next one, and the wave-uniform
-// word offset (n*A) mod 8 selects them (the padding assets take the following draws, unused).
+// Random access to a step's draws, for the checkpoint form, whose segments start at any step: the
+// words (low, high) of draws n*A .. n*A + A - 1 of the path's stream (draw j is words 2j and 2j +
+// 1). They lie in ChaCha blocks (n*A) / 8 and the next one, and the wave-uniform word offset (n*A)
+// mod 8 selects them (the padding assets of a basket of A < 8 = D take the following draws, unused).
 template <int D, bool PADDED>
 __device__ __forceinline__ void basket_draws(const sde_u32 (&key)[8], int n, int A, sde_u32 (&lo)[D],
                                              sde_u32 (&hi)[D]) {
@@ -75,35 +76,62 @@ __device__ __forceinline__ void basket_draws(const sde_u32 (&key)[8], int n, int
       hi[k] = blk[2 * k + 1];
     }
   } else {
+    static_assert(D == 1, "the checkpoint form runs one asset or eight");
+    sde_u32 blk[16];
+    sde_chacha_block<8>(key, (sde_u64)(n >> 3), blk);
+    const int w = n & 7;
+    sde_u32 l = blk[0], h = blk[1];
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-      const long long j = (long long)n * D + k;
-      sde_u32 blk[16];
-      sde_chacha_block<8>(key, (sde_u64)(j >> 3), blk);
-      const int w = (int)(j & 7);
-      sde_u32 l = blk[0], h = blk[1];
-#pragma unroll
-      for (int q = 1; q < 8; ++q) {
-        l = (w == q) ? blk[2 * q] : l;
-        h = (w == q) ? blk[2 * q + 1] : h;
-      }
-      lo[k] = l;
-      hi[k] = h;
+    for (int q = 1; q < 8; ++q) {
+      l = (w == q) ? blk[2 * q] : l;
+      h = (w == q) ? blk[2 * q + 1] : h;
     }
+    lo[0] = l;
+    hi[0] = h;
   }
 }
+
+// f(0), f(1), .. f(N - 1) with the argument a constant.
+template <int I, int N, class F>
+__device__ __forceinline__ void basket_static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    basket_static_for<I + 1, N>(f);
+  }
+}
+
+// The path's normals in order, taken with compile-time positions: draw(j) for j = 0, 1, .. of a chunk
+// of steps that starts on a block. f32 converts a block's eight draws together (one test for rare
+// ones), f64 each on its own (fewer registers).
+template <typename R>
+struct BasketNormals {
+  sde_u32 lo[8], hi[8];
+  float z[8];
+  template <int j>
+  __device__ __forceinline__ R draw(const sde_u32 (&key)[8], sde_u64 block0) {
+    if constexpr (j % 8 == 0) {
+      sde_u32 blk[16];
+      sde_chacha_block<8>(key, block0 + (sde_u64)(j / 8), blk);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        lo[k] = blk[2 * k];
+        hi[k] = blk[2 * k + 1];
+      }
+      if constexpr (sizeof(R) == 4) sde_psi_words<8>(lo, hi, z);
+    }
+    if constexpr (sizeof(R) == 4) return z[j % 8];
+    else return sde_psi_word(lo[j % 8], hi[j % 8]);
+  }
+};
 
 template <typename R, int D>
 struct BasketStep {
   R eps[D], Z[D];
 };
 
-template <typename R, int D, bool PADDED>
-__device__ __forceinline__ void basket_noise(const sde_u32 (&key)[8], int n, int A, const R (&L)[D][D],
-                                             BasketStep<R, D>& st) {
-  sde_u32 lo[D], hi[D];
-  basket_draws<D, PADDED>(key, n, A, lo, hi);
-  sde_psi_words<D>(lo, hi, st.eps);
+// Z = L eps.
+template <typename R, int D>
+__device__ __forceinline__ void basket_correlate(const R (&L)[D][D], BasketStep<R, D>& st) {
 #pragma unroll
   for (int i = 0; i < D; ++i) {
     R z = R(0);
@@ -111,6 +139,15 @@ __device__ __forceinline__ void basket_noise(const sde_u32 (&key)[8], int n, int
     for (int k = 0; k <= i; ++k) z = z + L[i][k] * st.eps[k];
     st.Z[i] = z;
   }
+}
+
+template <typename R, int D, bool PADDED>
+__device__ __forceinline__ void basket_noise(const sde_u32 (&key)[8], int n, int A, const R (&L)[D][D],
+                                             BasketStep<R, D>& st) {
+  sde_u32 lo[D], hi[D];
+  basket_draws<D, PADDED>(key, n, A, lo, hi);
+  sde_psi_words<D>(lo, hi, st.eps);
+  basket_correlate<R, D>(L, st);
 }
 
 template <typename R>
@@ -219,7 +256,7 @@ struct BasketReverse {
   }
 };
 
-// MODE 0: price; 1: price and adjoint with checkpoints and recomputation; 2: the forward pass of
+// MODE 0: price (two partials a block, payoff and payoff^2); 1: price and adjoint with checkpoints and recomputation; 2: the forward pass of
 // the tape form, which writes X_0 .. X_N to the tape and leaves the payoff, the reverse sweep and
 // every partial to sdesim_basket_reverse.
 template <typename R, int D, int SEG, int MODE, bool PADDED>
@@ -252,17 +289,37 @@ __global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
 
   R* ck = (R*)a.states;
   // Forward pass.
-  for (int n = 0; n < N; ++n) {
-    if (TAPE) sde_tape_store<R, D>(a.states, n, S, voff, X);
-    if (MODE == 1 && (n % SEG) == 0 && live) {
-      const long long slot = n / SEG;
+  if constexpr (MODE == 1) {
+    for (int n = 0; n < N; ++n) {
+      if ((n % SEG) == 0 && live) {
+        const long long slot = n / SEG;
 #pragma unroll
-      for (int i = 0; i < D; ++i) ck[(slot * D + i) * S + sid] = X[i];
+        for (int i = 0; i < D; ++i) ck[(slot * D + i) * S + sid] = X[i];
+      }
+      BasketStep<R, D> st;
+      basket_noise<R, D, PADDED>(key, n, a.assets, L, st);
+#pragma unroll
+      for (int i = 0; i < D; ++i) X[i] = X[i] + X[i] * (mu[i] * dt + sig[i] * sdt * st.Z[i]);
     }
-    BasketStep<R, D> st;
-    basket_noise<R, D, PADDED>(key, n, a.assets, L, st);
+  } else {
+    constexpr int U = SdeChunk<D>::U;  // steps in a whole number of ChaCha blocks
+    for (int n0 = 0; n0 < N; n0 += U) {
+      BasketNormals<R> noise;
+      basket_static_for<0, U>([&](auto u_) {
+        constexpr int u = u_;
+        if (U == 1 || n0 + u < N) {
+          if (TAPE) sde_tape_store<R, D>(a.states, n0 + u, S, voff, X);
+          BasketStep<R, D> st;
+          basket_static_for<0, D>([&](auto k_) {
+            constexpr int k = k_;
+            st.eps[k] = noise.template draw<u * D + k>(key, (sde_u64)n0 * D / 8);
+          });
+          basket_correlate<R, D>(L, st);
 #pragma unroll
-    for (int i = 0; i < D; ++i) X[i] = X[i] + X[i] * (mu[i] * dt + sig[i] * sdt * st.Z[i]);
+          for (int i = 0; i < D; ++i) X[i] = X[i] + X[i] * (mu[i] * dt + sig[i] * sdt * st.Z[i]);
+        }
+      });
+    }
   }
   if (TAPE) {
     sde_tape_store<R, D>(a.states, N, S, voff, X);
@@ -274,11 +331,11 @@ __global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
   R pay, dpay;
   basket_payoff<R, D>(X, w, (R)a.strike, (R)a.width, pay, dpay);
 
-  if (MODE == 0) {
-    sde_reduce_store_chunked<NQ>([&](int q) { return !live || q > 1 ? 0.0 : q == 0 ? (double)pay : (double)pay * (double)pay; },
-                            a.partials + (long long)blockIdx.x * NQ);
+  if constexpr (MODE == 0) {
+    sde_reduce_store_chunked<2>([&](int q) { return !live ? 0.0 : q == 0 ? (double)pay : (double)pay * (double)pay; },
+                                a.partials + (long long)blockIdx.x * 2);
   }
-  if (MODE == 1) {
+  if constexpr (MODE == 1) {
     BasketReverse<R, D> rv(a, X, dpay);
     for (int seg = (N + SEG - 1) / SEG - 1; seg >= 0; --seg) {
       const int n0 = seg * SEG;
@@ -361,48 +418,62 @@ __global__ void __launch_bounds__(1024) sdesim_sum_partials(const double* __rest
 
 }  // namespace
 
-// mode: 0 price, 1 adjoint with checkpoints (a.states holds [slots][D][paths], one per 19 steps),
-// 2 adjoint with the tape (a.states holds [steps + 1][D][paths]; a forward and a reverse kernel).
-hipError_t sdesim_launch_basket(int f32, int assets, int mode, int grid, const BasketArgs& a, int nq,
-                                double* sums, hipStream_t stream) {
-  // assets 1 runs the one-asset kernels, 8 the eight-asset ones, and 2-7 the eight-asset ones
-  // padded (their own draw stride).
-#define SDE_BASKET(R, D, MODE, PAD)                                                                        \
-  hipLaunchKernelGGL((sdesim_basket<R, D, 19, MODE, PAD>), dim3(grid), dim3(256), 0, stream, a);              \
-  if (MODE == 2) hipLaunchKernelGGL((sdesim_basket_reverse<R, D>), dim3(grid), dim3(256), 0, stream, a);     \
-  break;
-  bool ok = true;
-  const int shape = assets == 1 ? 1 : assets == 8 ? 8 : (assets >= 2 && assets < 8) ? 9 : 0;
-  switch ((f32 ? 100 : 0) + shape * 3 + mode) {
-    case 100 + 27 + 2: SDE_BASKET(float, 8, 2, true)
-    case 100 + 27 + 1: SDE_BASKET(float, 8, 1, true)
-    case 100 + 27 + 0: SDE_BASKET(float, 8, 0, true)
-    case 100 + 24 + 2: SDE_BASKET(float, 8, 2, false)
-    case 100 + 24 + 1: SDE_BASKET(float, 8, 1, false)
-    case 100 + 24 + 0: SDE_BASKET(float, 8, 0, false)
-    case 100 + 3 + 2: SDE_BASKET(float, 1, 2, false)
-    case 100 + 3 + 1: SDE_BASKET(float, 1, 1, false)
-    case 100 + 3 + 0: SDE_BASKET(float, 1, 0, false)
-    case 27 + 2: SDE_BASKET(double, 8, 2, true)
-    case 27 + 1: SDE_BASKET(double, 8, 1, true)
-    case 27 + 0: SDE_BASKET(double, 8, 0, true)
-    case 24 + 2: SDE_BASKET(double, 8, 2, false)
-    case 24 + 1: SDE_BASKET(double, 8, 1, false)
-    case 24 + 0: SDE_BASKET(double, 8, 0, false)
-    case 3 + 2: SDE_BASKET(double, 1, 2, false)
-    case 3 + 1: SDE_BASKET(double, 1, 1, false)
-    case 3 + 0: SDE_BASKET(double, 1, 0, false)
-    default: ok = false;
-  }
-#undef SDE_BASKET
-  if (!ok) return hipErrorInvalidValue;
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(sdesim_sum_partials, dim3(nq), dim3(grid > 256 ? 1024 : 256), 0, stream, a.partials, grid, nq, sums);
-  return hipGetLastError();
-}
-
 hipError_t sdesim_launch_sum_partials(const double* partials, int nblocks, int nq, double* out, hipStream_t stream) {
   hipLaunchKernelGGL(sdesim_sum_partials, dim3(nq), dim3(nblocks > 256 ? 1024 : 256), 0, stream, partials, nblocks, nq, out);
   return hipGetLastError();
+}
+
+// mode: 0 price, 1 adjoint with checkpoints (a.states holds [slots][D][paths], one per 19 steps, D = 1 or
+// 8), 2 adjoint with the tape (a.states holds [steps + 1][assets][paths]; a forward and a reverse kernel).
+// Price and tape have a kernel per asset count, which draws, correlates and stores no more than the
+// basket's own assets: 5 assets in f64 (30,001 paths x 252) took 745 us forward and 197 us
+// reverse in the 8-asset kernels, padded, each step from two ChaCha blocks (a step's draws do not start on a
+// block) with 15-way selects; 252 and 134 us in their own. The checkpoint form, which must start at any
+// step, keeps the padded 8-asset kernels for 2-7 assets.
+hipError_t sdesim_launch_basket(int f32, int assets, int mode, int grid, const BasketArgs& a, int nq,
+                                double* sums, hipStream_t stream) {
+#define SDE_BASKET(R, D, MODE, PAD) \
+  hipLaunchKernelGGL((sdesim_basket<R, D, 19, MODE, PAD>), dim3(grid), dim3(256), 0, stream, a)
+#define SDE_BASKET_WIDTH(D)                                                                                         \
+  case D:                                                                                                           \
+    if (mode == 0) {                                                                                                \
+      if (f32) SDE_BASKET(float, D, 0, false);                                                                      \
+      else SDE_BASKET(double, D, 0, false);                                                                         \
+    } else if (f32) {                                                                                               \
+      SDE_BASKET(float, D, 2, false);                                                                               \
+      hipLaunchKernelGGL((sdesim_basket_reverse<float, D>), dim3(grid), dim3(256), 0, stream, a);                   \
+    } else {                                                                                                        \
+      SDE_BASKET(double, D, 2, false);                                                                              \
+      hipLaunchKernelGGL((sdesim_basket_reverse<double, D>), dim3(grid), dim3(256), 0, stream, a);                  \
+    }                                                                                                               \
+    break;
+  if (assets < 1 || assets > 8 || mode < 0 || mode > 2) return hipErrorInvalidValue;
+  if (mode == 1) {
+    if (assets == 1) {
+      if (f32) SDE_BASKET(float, 1, 1, false);
+      else SDE_BASKET(double, 1, 1, false);
+    } else if (assets == 8) {
+      if (f32) SDE_BASKET(float, 8, 1, false);
+      else SDE_BASKET(double, 8, 1, false);
+    } else {
+      if (f32) SDE_BASKET(float, 8, 1, true);
+      else SDE_BASKET(double, 8, 1, true);
+    }
+  } else {
+    switch (assets) {
+      SDE_BASKET_WIDTH(1)
+      SDE_BASKET_WIDTH(2)
+      SDE_BASKET_WIDTH(3)
+      SDE_BASKET_WIDTH(4)
+      SDE_BASKET_WIDTH(5)
+      SDE_BASKET_WIDTH(6)
+      SDE_BASKET_WIDTH(7)
+      SDE_BASKET_WIDTH(8)
+    }
+  }
+#undef SDE_BASKET_WIDTH
+#undef SDE_BASKET
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return sdesim_launch_sum_partials(a.partials, grid, nq, sums, stream);
 }

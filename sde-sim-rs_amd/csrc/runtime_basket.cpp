@@ -44,8 +44,8 @@ int guard(F&& f) {
 
 struct sdesim_basket {
   sdesim_basket_spec spec{};
-  int D = 8;          // compiled width (1 or 8)
-  int nq = 0;
+  int D = 8;          // width of the adjoint's kernels: the assets (tape), 1 or 8 (checkpoints)
+  int nq = 0;         // reduced quantities of the adjoint
   long long grid = 0;
   int storage = SDESIM_STORAGE_CHECKPOINTS;  // resolved at creation: TAPE or CHECKPOINTS
   void* states = nullptr;                   // the tape or the checkpoints
@@ -74,18 +74,17 @@ int sdesim_basket_create(const sdesim_basket_spec* spec, sdesim_basket** out) {
       throw BFail{SDESIM_EVALUE, "storage must be SDESIM_STORAGE_AUTO, _TAPE or _CHECKPOINTS"};
     std::unique_ptr<sdesim_basket> b(new sdesim_basket());
     b->spec = s;
-    b->D = s.assets == 1 ? 1 : 8;
-    b->nq = 2 + 3 * b->D + b->D * (b->D + 1) / 2;
+    const int padded = s.assets == 1 ? 1 : 8;
     b->grid = (s.paths + 255) / 256;
     if (b->grid > 0x7fffffffLL) throw BFail{SDESIM_EVALUE, "too many paths"};
     const size_t rb = s.precision == SDESIM_F32 ? 4 : 8;
     const long long slots = (s.steps + kSeg - 1) / kSeg;
-    const size_t ck = (size_t)slots * b->D * (size_t)s.paths * rb;
-    const size_t step_bytes = (size_t)b->D * (size_t)s.paths * rb;  // one step of the tape
-    const size_t tape = step_bytes * ((size_t)s.steps + 1);  // X_0 .. X_N
+    const size_t ck = (size_t)slots * padded * (size_t)s.paths * rb;
+    const size_t tape = (size_t)s.assets * (size_t)s.paths * rb * ((size_t)s.steps + 1);  // X_0 .. X_N
     size_t free_b = 0, total_b = 0;
     bk(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-    const bool tape_addressable = step_bytes < (1ull << 31);  // one buffer resource per step
+    // One buffer resource per step (sized for the padded width, the widest kernels').
+    const bool tape_addressable = (size_t)padded * (size_t)s.paths * rb < (1ull << 31);
     if (s.storage == SDESIM_STORAGE_TAPE) {
       if (!tape_addressable) throw BFail{SDESIM_EVALUE, "the tape needs assets * paths * size < 2^31 bytes per step"};
       if (tape + (64u << 20) > free_b) throw BFail{SDESIM_ERUNTIME, "the tape does not fit in free device memory"};
@@ -99,6 +98,8 @@ int sdesim_basket_create(const sdesim_basket_spec* spec, sdesim_basket** out) {
       if (ck + (64u << 20) > free_b) throw BFail{SDESIM_ERUNTIME, "checkpoints do not fit in free device memory"};
       bk(hipMalloc(&b->states, ck), "hipMalloc(checkpoints)");
     }
+    b->D = b->storage == SDESIM_STORAGE_TAPE ? s.assets : padded;
+    b->nq = 2 + 3 * b->D + b->D * (b->D + 1) / 2;
     bk(sdesim_normal_table(s.precision == SDESIM_F32 ? 1 : 0, &b->normal_tab), "inverse normal table");
     bk(hipMalloc(&b->partials, sizeof(double) * b->nq * b->grid), "hipMalloc(partials)");
     bk(hipMalloc(&b->sums, sizeof(double) * b->nq), "hipMalloc(sums)");
@@ -140,11 +141,12 @@ int sdesim_basket_eval(sdesim_basket* b, const double* x0, const double* mu, con
     a.assets = A;
     a.normal_tab = b->normal_tab;
     hipStream_t st = (hipStream_t)stream;
+    const int nq = adjoint ? b->nq : 2;
     const int mode = !adjoint ? 0 : b->storage == SDESIM_STORAGE_TAPE ? 2 : 1;
-    bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, mode, (int)b->grid, a, b->nq, b->sums, st),
+    bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, mode, (int)b->grid, a, nq, b->sums, st),
        "basket launch");
-    std::vector<double> sums(b->nq);
-    bk(hipMemcpyAsync(sums.data(), b->sums, sizeof(double) * b->nq, hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
+    std::vector<double> sums(nq);
+    bk(hipMemcpyAsync(sums.data(), b->sums, sizeof(double) * nq, hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
     bk(hipStreamSynchronize(st), "hipStreamSynchronize");
     const double n = (double)s.paths;
     const double m1 = sums[0] / n;

@@ -67,7 +67,7 @@ class Basket:
     """Price and adjoint of a weighted basket call on D <= 8 correlated GBM assets.
 
     `storage` picks how the adjoint keeps the forward states: "tape" (every state in device
-    memory, steps * 8 * paths values for D > 1), "checkpoints" (every 19th state, the rest
+    memory, (steps + 1) * assets * paths values), "checkpoints" (every 19th state, the rest
     recomputed during the reverse sweep) or "auto" (the tape when it fits in half of the free
     device memory). `self.storage` is the form in use."""
 
