@@ -491,6 +491,16 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
   s << "  static constexpr int M = " << M << ";\n";
   s << "  static constexpr int NK = " << NK << ";\n";
   s << "  static constexpr bool HAS_PAYOFF = " << (o.payoff.empty() ? "false" : "true") << ";\n";
+  if (o.team > 1) {
+    std::set<int> jumps;
+    for (const ProcessDef& pd : u.processes)
+      for (const Term& t : pd.terms)
+        if (t.kind == IncKind::Jump) jumps.insert(t.index);
+    s << "  static constexpr bool SIGN = " << (o.scheme == 0 ? "false" : "true") << ";\n";
+    s << "  __device__ static constexpr bool is_jump(int k) {\n    return false";
+    for (int k : jumps) s << " || k == " << k;
+    s << ";\n  }\n";
+  }
   s << "  __device__ static __forceinline__ void prologue(real (&X)[P], real (&C)[P], real (&K)[NK], real tc) {\n";
   s << pro;
   s << "  }\n";
@@ -520,8 +530,9 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
   s << "  }\n";
   s << "};\n\n";
   s << "extern \"C\" __global__ void __launch_bounds__(" << o.block << ") " << o.name << "(SimArgs a) {\n";
-  s << "  sde_path_kernel<SdeModel, " << o.rng << ", " << o.out << ", " << o.ppl << ", " << o.nsl << ", "
-    << (o.uniform_grid ? "true" : "false") << ", " << (o.wave_aligned ? "true" : "false") << ">(a);\n";
+  s << "  sde_" << (o.team > 1 ? "team" : "path") << "_kernel<SdeModel, " << o.rng << ", " << o.out << ", "
+    << (o.team > 1 ? o.team : o.ppl) << ", " << o.nsl << ", " << (o.uniform_grid ? "true" : "false") << ", "
+    << (o.wave_aligned ? "true" : "false") << ">(a);\n";
   s << "}\n";
   return s.str();
 }

@@ -18,6 +18,7 @@ struct CodegenOptions {
   int nsl = 1;          // Sobol table slices (Gray-code bits covered: 6 + 8 (nsl - 1))
   bool uniform_grid = false;  // every dt and sqrt(dt) is bitwise equal in the kernel's precision
   bool wave_aligned = false;  // Sobol index of path 0 is a multiple of 64 and blocks hold whole waves
+  int team = 1;         // waves to 64 paths: 1 = sde_path_kernel, else sde_team_kernel
   bool library_f64 = false;   // f64: library logarithm and roots (reaches_root below)
   bool steps = true;    // false when the time grid has a single point (nothing is evaluated)
   std::string payoff;   // expression over process names and t at the last time point

@@ -595,6 +595,41 @@ template <> struct SdeUnifOf<SDE_RNG_SOBOL_XOR, float> { typedef SdeUnifX type; 
 template <> struct SdeUnifOf<SDE_RNG_PSEUDO, float> { typedef SdeUnifW type; };
 template <> struct SdeUnifOf<SDE_RNG_SOBOL_SHIFT, float> { typedef SdeUnifW type; };
 
+// The uniform of one draw: from the Sobol word nx (in XOR mode the complement of the scrambled point)
+// and the stream's two words.
+template <int RNG, typename R, bool LIB>
+__device__ __forceinline__ typename SdeUnifOf<RNG, R>::type sde_uniform(sde_u32 nx, sde_u32 lo, sde_u32 hi,
+                                                                        const float* tail, sde_u32 sm, sde_u32 sm2) {
+  typename SdeUnifOf<RNG, R>::type u;
+  if constexpr (RNG == SDE_RNG_SOBOL_SHIFT && sizeof(R) == 8) {
+    const double y = (double)nx * 0x1.0p-32 + sde_u01_from_words(lo, hi);
+    const double v = __builtin_amdgcn_fract(y);  // y - floor(y), 0 <= y < 2
+    if constexpr (LIB) u = v;
+    else u.u = v;
+  } else if constexpr (LIB && RNG == SDE_RNG_SOBOL_XOR) {
+    u = sde_uval(SdeUnifX{nx, nullptr, 0u, 0u});
+  } else if constexpr (LIB) {
+    u = sde_u01_from_words(lo, hi);
+  } else if constexpr (RNG == SDE_RNG_SOBOL_XOR) {
+    u.yc = nx;
+    u.tail = tail;
+    u.sm = sm;
+    u.sm2 = sm2;
+  } else if constexpr (RNG == SDE_RNG_SOBOL_SHIFT) {
+    // frac(y 2^-32 + shift) as an exact 53-bit fraction: (y 2^21 + (word >> 11)) mod 2^53, held
+    // as the 64-bit word (fraction << 11). The f64 path rounds the sum to 53 bits first when it
+    // exceeds 1, a difference of at most 2^-53 in the uniform.
+    const sde_u64 sh = (((sde_u64)hi << 32) | lo) >> 11;
+    const sde_u64 f = (((sde_u64)nx << 21) + sh) << 11;
+    u.lo = (sde_u32)f;
+    u.hi = (sde_u32)(f >> 32);
+  } else {
+    u.lo = lo;
+    u.hi = hi;
+  }
+  return u;
+}
+
 template <typename R>
 struct SdeGrid {
   R tc, tn, dt, sdt;
@@ -848,47 +883,11 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
         for (int j = 0; j < PPL; ++j) {
 #pragma unroll
           for (int k = 0; k < MM; ++k) {
-            double v = 0.5;
-            if (RNG == SDE_RNG_SOBOL_SHIFT && M > 0) {
-              const int w = 2 * (i * M + k);
-              const double sh = sde_u01_from_words(W[j][USE_CHACHA ? w : 0], W[j][USE_CHACHA ? w + 1 : 0]);
-              const double y = (double)nx[j][k] * 0x1.0p-32 + sh;
-              v = __builtin_amdgcn_fract(y);  // y - floor(y), 0 <= y < 2
-            } else if (USE_INJ) {
-              v = ni[j][k];
-            }
-            if constexpr (LIB) {
-              if constexpr (RNG == SDE_RNG_SOBOL_XOR) {
-                u[j][k] = sde_uval(SdeUnifX{nx[j][k], nullptr, 0u, 0u});
-              } else if constexpr (RNG == SDE_RNG_PSEUDO) {
-                const int w = 2 * (i * M + k);
-                u[j][k] = sde_u01_from_words(W[j][USE_CHACHA ? w : 0], W[j][USE_CHACHA ? w + 1 : 0]);
-              } else {
-                u[j][k] = v;
-              }
-            } else if constexpr (RNG == SDE_RNG_SOBOL_XOR) {
-              u[j][k].yc = nx[j][k];
-              u[j][k].tail = a.tail_tab;
-              u[j][k].sm = smask;
-              u[j][k].sm2 = smask2;
-            } else if constexpr (RNG == SDE_RNG_PSEUDO) {
-              const int w = 2 * (i * M + k);
-              u[j][k].lo = W[j][USE_CHACHA ? w : 0];
-              u[j][k].hi = W[j][USE_CHACHA ? w + 1 : 0];
-            } else if constexpr (RNG == SDE_RNG_SOBOL_SHIFT && sizeof(real) == 4) {
-              // frac(y 2^-32 + shift) as an exact 53-bit fraction: (y 2^21 + (word >> 11)) mod
-              // 2^53, held as the 64-bit word (fraction << 11). The f64 path rounds the sum to
-              // 53 bits first when it exceeds 1, a difference of at most 2^-53 in the uniform.
-              const int w = 2 * (i * M + k);
-              const sde_u64 sh = (((sde_u64)W[j][USE_CHACHA ? w + 1 : 0] << 32) | W[j][USE_CHACHA ? w : 0]) >> 11;
-              const sde_u64 f = (((sde_u64)nx[j][k] << 21) + sh) << 11;
-              u[j][k].lo = (sde_u32)f;
-              u[j][k].hi = (sde_u32)(f >> 32);
-            } else if constexpr (RNG == SDE_RNG_SOBOL_SHIFT) {
-              u[j][k].u = v;
-            } else {
-              u[j][k] = v;
-            }
+            const int w = USE_CHACHA ? 2 * (i * M + k) : 0;
+            if constexpr (USE_INJ) u[j][k] = ni[j][k];
+            else if constexpr (M > 0 && (USE_CHACHA || USE_SOBOL))
+              u[j][k] = sde_uniform<RNG, real, LIB>(nx[j][k], W[j][w], W[j][USE_CHACHA ? w + 1 : 0], a.tail_tab, smask, smask2);
+            else u[j][k] = 0.5;
           }
         }
         // The grid and table words ahead are requested unconditionally (near the end the last
@@ -924,6 +923,233 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
           acc[2 * (KQ - 1)] += v;
           acc[2 * (KQ - 1) + 1] += v * v;
         }
+      }
+    }
+    sde_block_reduce_store<2 * KQ>(acc, a.partials + (long long)blockIdx.x * (2 * KQ));
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// The same paths with several waves to 64 of them
+// ------------------------------------------------------------------------------------------
+// A run of few paths leaves the SIMDs empty: 10,000 paths are 157 waves for 1024 SIMDs, each a serial
+// chain of steps, and most of a step is its noise (ChaCha8 block, inverse normals), which does not
+// depend on the state. Here a block of W waves has 64 paths: waves 0 .. W - 2 produce the noise of
+// successive units of steps (whole ChaCha blocks) into LDS, and the last wave steps the paths through the
+// previous round's noise meanwhile; the two halves of the buffer change roles at a barrier per round. The
+// steps' times go through LDS as well: a scalar load per step, waited for together with the LDS reads, took
+// a fifth of the stepping wave's time. Each value is computed by the operations of sde_path_kernel (in what
+// pairs products and sums are fused can differ, so a last bit can).
+// What bounds it now is the stepping wave's chain. GBM, 10,000 x 252 pseudo-random: 31 us instead of 80; the
+// jump diffusion, 10,000 x 1000: 295 instead of 588; Heston RK, 65,537 x 365, random shift: 302 instead of 388.
+// FP64 only: the FP32 step may be reassociated, and how depends on the code around it.
+//
+// A step's noise as the stepping wave reads it: Psi(u) of a Wiener increment, u of a jump, and (RK) whether
+// the first uniform exceeds 1/2.
+struct SdeUnifP {
+  double z, u;
+  bool gt;
+};
+__device__ __forceinline__ double sde_uval(SdeUnifP u) { return u.u; }
+__device__ __forceinline__ double sde_dw(SdeUnifP u, double sdt) { return sdt * u.z; }
+__device__ __forceinline__ double sde_signed(SdeUnifP u, double sdt) { return sde_negate_if(!u.gt, sdt); }
+
+__device__ __forceinline__ double sde_psi_of(SdeUnifD u) { return sde_inv_normal_d<true>(u.u - 0.5); }
+__device__ __forceinline__ double sde_psi_of(SdeUnifX u) { return sde_psi<double>(u); }
+__device__ __forceinline__ double sde_psi_of(SdeUnifW u) { return sde_psi_word(u.lo, u.hi); }
+
+// A model provides, beyond sde_path_kernel's needs: is_jump(k) (increment k is a jump) and SIGN (the
+// step reads the first uniform's sign).
+template <class Mdl, int RNG, int OUT, int W, int NSL, bool UG, bool AL>
+__device__ __forceinline__ void sde_team_kernel(const SimArgs& a) {
+  typedef double real;
+  static_assert(sizeof(typename Mdl::real) == 8, "FP64 only");
+  constexpr int P = Mdl::P;
+  constexpr int M = Mdl::M;
+  constexpr int NK = Mdl::NK;
+  constexpr bool USE_CHACHA = RNG == SDE_RNG_PSEUDO || RNG == SDE_RNG_SOBOL_SHIFT;
+  constexpr bool USE_SOBOL = RNG == SDE_RNG_SOBOL_SHIFT || RNG == SDE_RNG_SOBOL_XOR;
+  static_assert(M > 0 && (USE_CHACHA || USE_SOBOL), "no noise to share out");
+  constexpr int UNIT = SdeChunk<M>::U;    // steps of a unit: whole ChaCha blocks
+  constexpr int NB = SdeChunk<M>::BLOCKS;
+  constexpr int KQ = P + (Mdl::HAS_PAYOFF ? 1 : 0);
+  constexpr bool FILT = (OUT & SDE_OUT_FILTRATION) != 0;
+  __shared__ double noise[2][(W - 1) * UNIT * M][64];
+  __shared__ double grid[2][(W - 1) * UNIT][4];  // the steps' t, next t, dt and sqrt(dt)
+  __shared__ sde_u64 above[2][(W - 1) * UNIT];  // SIGN: bit l set when lane l's first uniform is > 1/2
+
+  sde_normal_tab_load<real>(a.normal_tab);
+
+  const long long S = a.S;
+  const int N = a.N;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const long long s = (long long)blockIdx.x * 64 + lane;
+  const bool live = s < S;
+  const long long sid = live ? s : 0;
+  const bool steps = wave == W - 1;
+
+  // Producers: the path's stream and table entries, as in sde_path_kernel.
+  sde_u32 key[8];
+  sde_u32 soff[NSL];
+  sde_const_u32* urow[NSL];
+  if (!steps) {
+    if (USE_CHACHA) sde_seed_from_u64(a.seed + (sde_u64)sid, key);
+    if (USE_SOBOL) {
+      const sde_u64 idx = (sde_u64)(a.sobol_first + sid);
+      const sde_u64 g = idx ^ (idx >> 1);
+      if (AL) {
+        soff[0] = (sde_u32)(g & 63u) * (sde_u32)(M * 4);
+#pragma unroll
+        for (int sl = 1; sl < NSL; ++sl) {
+          const sde_u32 e = __builtin_amdgcn_readfirstlane((sde_u32)(g >> (6 + 8 * (sl - 1))) & 255u);
+          urow[sl] = (sde_const_u32*)a.sobol_up + ((size_t)(sl - 1) * 256u + e) * (size_t)a.sobol_dims;
+        }
+      } else {
+        sde_sobol_offsets<NSL>(g, soff);
+#pragma unroll
+        for (int sl = 0; sl < NSL; ++sl) soff[sl] *= 4u;
+      }
+    }
+  }
+  __amdgpu_buffer_rsrc_t tab_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)a.sobol_tab, (short)0, USE_SOBOL ? a.sobol_tab_words * 4 : 0, 0x00020000);
+  auto produce = [&](int half, int q, int n0) {
+    if (lane < UNIT) {
+      const int n = n0 + lane < N ? n0 + lane : N - 1;
+      double* gs = grid[half][q * UNIT + lane];
+      gs[0] = a.times[n];
+      gs[1] = a.times[n + 1];
+      gs[2] = UG ? a.dt_u : a.dts[n];
+      gs[3] = UG ? a.sdt_u : a.sdts[n];
+    }
+    sde_u32 nx[UNIT][M];
+    if (USE_SOBOL) {
+#pragma unroll
+      for (int i = 0; i < UNIT; ++i) {
+        const int n = n0 + i < N ? n0 + i : N - 1;
+        if (AL) {
+          sde_load_words<M>(tab_rsrc, (int)soff[0], n * (64 * M * 4), nx[i]);
+#pragma unroll
+          for (int k = 0; k < M; ++k) {
+#pragma unroll
+            for (int sl = 1; sl < NSL; ++sl) nx[i][k] ^= urow[sl][n * M + k];
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < M; ++k) {
+            const int base = (int)((sde_u32)(n * M + k) * (64u + 256u * (NSL - 1)) * 4u);
+            nx[i][k] = 0u;
+#pragma unroll
+            for (int sl = 0; sl < NSL; ++sl)
+              nx[i][k] ^= (sde_u32)__builtin_amdgcn_raw_buffer_load_b32(tab_rsrc, (int)soff[sl], base, 0);
+          }
+        }
+      }
+    }
+    sde_u32 words[USE_CHACHA ? NB * 16 : 1];
+    if (USE_CHACHA) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        sde_u32 blk[16];
+        sde_chacha_block<8>(key, (sde_u64)n0 * M / 8 + b, blk);
+#pragma unroll
+        for (int w = 0; w < 16; ++w) words[USE_CHACHA ? 16 * b + w : 0] = blk[w];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < UNIT; ++i) {
+#pragma unroll
+      for (int k = 0; k < M; ++k) {
+        const int w = USE_CHACHA ? 2 * (i * M + k) : 0;
+        const auto u = sde_uniform<RNG, real, false>(nx[i][k], words[w], words[USE_CHACHA ? w + 1 : 0], nullptr, 0u, 0u);
+        noise[half][(q * UNIT + i) * M + k][lane] = Mdl::is_jump(k) ? sde_uval(u) : sde_psi_of(u);
+        if (Mdl::SIGN && k == 0) {
+          const sde_u64 gt = __builtin_amdgcn_ballot_w64(sde_gt_half(u));
+          if (lane == 0) above[half][q * UNIT + i] = gt;
+        }
+      }
+    }
+  };
+
+  // The stepping wave: the state, and its rows' stores as in sde_path_kernel.
+  real X[P], C[P], K[NK];
+#pragma unroll
+  for (int p = 0; p < P; ++p) { X[p] = (real)a.x0[p]; C[p] = X[p]; }
+#pragma unroll
+  for (int k = 0; k < NK; ++k) K[k] = real(0);
+  Mdl::prologue(X, C, K, a.times[0]);
+  const long long row_bytes = (long long)P * S * (long long)sizeof(real);
+  const sde_u32 voff = live ? (sde_u32)(sid * (long long)sizeof(real)) : 0x80000000u;
+  auto store_row = [&](int r) {
+    char* base = (char*)a.filtration + (long long)r * row_bytes;
+    __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)row_bytes, 0x00020000);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int soff_p = (int)((long long)p * S * (long long)sizeof(real));
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(SdeU32x2, X[p]), rs, (int)voff, soff_p, 2);
+    }
+  };
+  if (steps) __builtin_amdgcn_s_setprio(3);  // it shares its SIMD with other blocks' producers
+  if (FILT && steps) store_row(0);
+  auto consume = [&](int half, int q, int n0) {
+    double v[UNIT][M];
+    sde_u64 gt[UNIT];
+    double g[UNIT][4];
+#pragma unroll
+    for (int i = 0; i < UNIT; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) g[i][j] = UG && j == 2 ? a.dt_u : UG && j == 3 ? a.sdt_u : grid[half][q * UNIT + i][j];
+      gt[i] = Mdl::SIGN ? above[half][q * UNIT + i] : 0u;
+#pragma unroll
+      for (int k = 0; k < M; ++k) v[i][k] = noise[half][(q * UNIT + i) * M + k][lane];
+    }
+#pragma unroll
+    for (int i = 0; i < UNIT; ++i) {
+      const int n = n0 + i;
+      if (n < N) {
+        SdeUnifP u[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) u[k] = SdeUnifP{v[i][k], v[i][k], ((gt[i] >> lane) & 1u) != 0u};
+        Mdl::step(X, C, K, g[i][0], g[i][1], g[i][2], g[i][3], u);
+        if (FILT) store_row(n + 1);
+      }
+    }
+  };
+
+  // Round r: units r (W - 1) .. are produced, those of round r - 1 stepped through. Every wave passes every
+  // barrier (the trip count is the grid's N, the same for all).
+  const int units = (N + UNIT - 1) / UNIT, rounds = (units + W - 2) / (W - 1);
+  for (int r = 0; r <= rounds; ++r) {
+    if (steps) {
+      if (r > 0) {
+        for (int q = 0; q < W - 1; ++q) {
+          const int n0 = ((r - 1) * (W - 1) + q) * UNIT;
+          if (n0 < N) consume((r - 1) & 1, q, n0);
+        }
+      }
+    } else {
+      const int n0 = (r * (W - 1) + wave) * UNIT;
+      if (r < rounds && n0 < N) produce(r & 1, wave, n0);
+    }
+    __syncthreads();
+  }
+
+  if (OUT & SDE_OUT_TERMINAL) {
+    double acc[2 * KQ];
+#pragma unroll
+    for (int q = 0; q < 2 * KQ; ++q) acc[q] = 0.0;
+    const real tT = a.times[N];
+    if (steps && live) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const double dv = (double)X[p] - a.x0[p];
+        acc[2 * p] += dv;
+        acc[2 * p + 1] += dv * dv;
+      }
+      if (Mdl::HAS_PAYOFF) {
+        const double v = (double)Mdl::payoff(X, tT);
+        acc[2 * (KQ - 1)] += v;
+        acc[2 * (KQ - 1) + 1] += v * v;
       }
     }
     sde_block_reduce_store<2 * KQ>(acc, a.partials + (long long)blockIdx.x * (2 * KQ));

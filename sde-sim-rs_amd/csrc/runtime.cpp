@@ -542,6 +542,31 @@ int32_t sdesim_process_index(const sdesim_universe* u, const char* name) {
   return it == u->u.registry.end() ? -1 : it->second;
 }
 
+// Waves of a block in sde_team_kernel for this plan, or 1: one lane per path, sde_path_kernel. Teams are for
+// runs that leave SIMDs empty or nearly so: four waves, one per SIMD of a CU (five to twelve are no faster
+// even with a CU per block), up to 3/2 waves of paths per SIMD. There (98,304 paths) they still take
+// 62 against 81 us (GBM, XOR) and 152 against 162 (Heston moments); at 2 per SIMD 216 against 185. Three, up
+// to a wave per SIMD, where the buffer of four exceeds a block's 64 KB of LDS. Not for FP32, nor where paths
+// part from any difference in a last bit; nor for fewer steps than one round produces, nor
+// where the partials of 64 paths each would outgrow the scratch array.
+static int team_waves(const sdesim::CodegenOptions& co, long long S, int N, int M, int KQ) {
+  if (M < 1 || co.f32 || co.library_f64 || co.rng == SDE_RNG_NONE || co.rng == SDE_RNG_INJECTED) return 1;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 1;  // no device: the module load reports it, after the source's own errors
+  const long long waves = (S + 63) / 64, simds = 4LL * cus;
+  const bool terminal = (co.out & SDE_OUT_TERMINAL) != 0;
+  if (terminal && (unsigned long long)waves * 2ull * (unsigned long long)KQ * 8ull > SDESIM_SCRATCH_BYTES) return 1;
+  const int unit = M % 8 == 0 ? 1 : M % 4 == 0 ? 2 : M % 2 == 0 ? 4 : 8;  // SdeChunk<M>::U
+  auto lds = [&](int team) {
+    return 2LL * (team - 1) * unit * (M * 512LL + 32 + 8) + 4096 + (terminal ? 256LL * KQ : 0);
+  };
+  const int team = lds(4) <= 65536 ? 4 : 3;
+  if (lds(team) > 65536 || 2 * waves > (team == 4 ? 3 : 2) * simds || N < (team - 1) * unit) return 1;
+  return team;
+}
+
 int sdesim_plan_create(const sdesim_universe* uh, const double* times, int32_t T, const double* x0,
                        int64_t S, const sdesim_options* opt_in, const char* payoff, sdesim_plan** out) {
   return guarded([&] {
@@ -630,6 +655,8 @@ int sdesim_plan_create(const sdesim_universe* uh, const double* times, int32_t T
     if (!x0) x0v.assign(P, 0.0);
     if (x0v.empty()) x0v.push_back(0.0);
     co.library_f64 = !co.f32 && sdesim::reaches_root(U, x0v, tv[0]);
+    if (opt.block_size <= 0 && opt.paths_per_lane <= 0) co.team = team_waves(co, S, N, M, plan->KQ);
+    if (co.team > 1) co.block = plan->block = 64 * co.team;
     co.name = sdesim::kernel_name(co);
     plan->source = sdesim::generate_kernel_source(U, co);
     plan->kname = co.name;
@@ -692,7 +719,8 @@ int sdesim_plan_create(const sdesim_universe* uh, const double* times, int32_t T
     if ((opt.outputs & SDESIM_OUT_FILTRATION) &&
         (long long)P * S * (opt.precision == SDESIM_F32 ? 4 : 8) >= (1LL << 31))
       fail(SDESIM_EVALUE, "one filtration row (processes x scenarios) must be below 2 GiB; split the scenarios");
-    plan->grid = (S + (long long)plan->block * plan->ppl - 1) / ((long long)plan->block * plan->ppl);
+    const long long block_paths = co.team > 1 ? 64 : (long long)plan->block * plan->ppl;
+    plan->grid = (S + block_paths - 1) / block_paths;
     if (plan->grid > 0x7fffffffLL) fail(SDESIM_EVALUE, "too many scenarios for one launch");
     if (opt.outputs & SDESIM_OUT_TERMINAL) {
       hip_check(hipMalloc(&plan->partials, (size_t)plan->grid * 2 * plan->KQ * sizeof(double)), "hipMalloc(partials)");
