@@ -276,16 +276,8 @@ def main():
                "greeks": 52, "adjoint_ms": times[True], "price_ms": times[False],
                "adjoint_over_price": times[True] / times[False],
                "path_steps_per_s_adjoint": AS * AN / (times[True] * 1e-3), "price": r["price"],
-               "storage": bk.storage,
-               "state_bytes": (AN + 1) * 8 * AS * 4 if bk.storage == "tape" else ((AN + 18) // 19) * 8 * AS * 4}
+               "storage": bk.storage, "state_bytes": 0}  # the derivatives are summed on the way forward
         del bk
-        if adj["storage"] == "tape":
-            # The checkpoint form (every 19th state, the rest recomputed in the reverse sweep),
-            # timed the same way for comparison.
-            bk = Basket(8, AN, AS, horizon=1.0, strike=100.0, width=0.5, seed=3, precision="f32", storage="checkpoints")
-            adj["adjoint_ms_checkpoints"] = _time_eval(
-                lambda: bk.evaluate(c["x0"], c["mu"], c["sigma"], c["rho"], adjoint=True), args)
-            del bk
 
     lmm = None
     if "lmm" in legs:

@@ -236,12 +236,13 @@ typedef struct sdesim_basket_spec {
   int32_t storage;    /* adjoint state storage: SDESIM_STORAGE_AUTO, _TAPE or _CHECKPOINTS */
 } sdesim_basket_spec;
 
-/* Adjoint state storage (basket and forward-rate model). TAPE keeps every state in device memory
- * ((steps + 1) * state size * paths values in the path precision, one write and one read each;
- * one step's states must stay below 2^31 bytes). CHECKPOINTS keeps every 19th (basket) or 16th
- * (forward-rate model) state and recomputes the rest during the reverse sweep (one more forward
- * pass of arithmetic, for that factor less memory). AUTO takes the tape when it fits in half of
- * the free device memory at creation, otherwise checkpoints. */
+/* Adjoint state storage. Forward-rate model: TAPE keeps every state in device memory
+ * ((steps + 1) * 40 * paths values in the path precision, one write and one read each);
+ * CHECKPOINTS keeps every 16th state and recomputes the rest during the reverse sweep (one more
+ * forward pass of arithmetic, for that factor less memory); AUTO takes the tape when it fits in half of
+ * the free device memory at creation, otherwise checkpoints. Basket: its adjoint keeps no states, and
+ * the choice is reported and makes no difference; TAPE needs one step's states (at 1 or 8 assets)
+ * below 2^31 bytes, and AUTO is TAPE where that holds. */
 #define SDESIM_STORAGE_AUTO 0
 #define SDESIM_STORAGE_TAPE 1
 #define SDESIM_STORAGE_CHECKPOINTS 2

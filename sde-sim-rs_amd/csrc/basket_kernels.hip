@@ -9,22 +9,18 @@
 // plain call max(B - K, 0) when width == 0.
 //
 // Adjoint (no reference counterpart): pathwise derivatives of the payoff with respect to X0, mu,
-// sigma and L, per path, reduced over paths in f64. The reverse sweep needs every state X_n. Two
-// storage forms:
-//  * tape (MODE 2): the forward pass writes every state to HBM ([step][asset][path], 4 or 8 bytes
-//    each; 49 GB for 8 assets x 365 steps x 2^22 paths in f32) and the reverse sweep reads them
-//    back, one step ahead of its arithmetic;
-//  * checkpoints (MODE 1): the forward pass stores the state every SEG steps ([slot][asset][path]);
-//    the reverse sweep walks the segments backwards, recomputes each segment's states from its
-//    checkpoint into registers and then steps back through it (one more forward pass of
-//    arithmetic, for SEG times less memory).
-// A reverse step reads the step's noise off the two states instead of regenerating it:
-//   g_n = X_{n+1} / X_n = 1 + mu dt + sigma sqrt(dt) Z_n,  d_n = (X_{n+1} - X_n) - X_n mu dt
-// (X_{n+1} - X_n is exact, the two being within a factor 2; forming 1 + mu dt first would round
-// mu dt ~ 2e-4 to the spacing of 1 and bias every recovered Z_n)
-//   Xbar_n = Xbar_{n+1} g_n,  mubar += Xbar_{n+1} X_n dt,  sigmabar += Xbar_{n+1} d_n / sigma
-//   Zbar_n = Xbar_{n+1} X_n sigma sqrt(dt),  Z_n = d_n / (X_n sigma sqrt(dt)),
-//   eps_n = L^-1 Z_n (forward substitution),  Lbar_ik += Zbar_{n,i} eps_{n,k}  (k <= i)
+// sigma and L, per path, reduced over paths in f64, all accumulated on the way forward. With
+//   g_{n,i} = X_{n+1,i} / X_{n,i} = 1 + mu_i dt + sigma_i sqrt(dt) Z_{n,i}
+// the reverse recursion Xbar_n = Xbar_{n+1} g_n makes M_i = Xbar_{n,i} X_{n,i} the same for every n, so it is
+// known from the final state (payoff' w_i X_{N,i}), and what a step adds to a derivative is M_i times a
+// quantity of that step alone:
+//   X0bar_i = M_i / X0_i,  mubar_i = M_i dt sum_n 1 / g_{n,i},
+//   Lbar_ik = M_i sigma_i sqrt(dt) H_ik,  H_ik = sum_n eps_{n,k} / g_{n,i}  (k <= i),
+//   sigmabar_i = M_i sqrt(dt) sum_{k <= i} L_ik H_ik.
+// No state is kept. The reverse sweep that this replaces wrote and read every state (49 GB for 8 assets x
+// 365 steps x 2^22 paths in f32): 26.1 ms for price and Greeks, 18.0 ms now, bound by VALU issue: a step's 8
+// draws are two thirds of it (350 instructions of ChaCha8, 80 of the normals), the 36 sums, 8
+// reciprocals and the step the rest.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -40,56 +36,6 @@ struct BasketConst {
   static constexpr int NL = D * (D + 1) / 2;   // lower-triangular entries of L
   static constexpr int NQ = 2 + 3 * D + NL;    // reduced quantities: payoff, payoff^2, gradients
 };
-
-// Random access to a step's draws, for the checkpoint form, whose segments start at any step: the
-// words (low, high) of draws n*A .. n*A + A - 1 of the path's stream (draw j is words 2j and 2j +
-// 1). They lie in ChaCha blocks (n*A) / 8 and the next one, and the wave-uniform word offset (n*A)
-// mod 8 selects them (the padding assets of a basket of A < 8 = D take the following draws, unused).
-template <int D, bool PADDED>
-__device__ __forceinline__ void basket_draws(const sde_u32 (&key)[8], int n, int A, sde_u32 (&lo)[D],
-                                             sde_u32 (&hi)[D]) {
-  if constexpr (PADDED) {
-    static_assert(D == 8, "padded baskets run the 8-asset kernels");
-    const long long j0 = (long long)n * A;
-    sde_u32 b0[16], b1[16];
-    sde_chacha_block<8>(key, (sde_u64)(j0 >> 3), b0);
-    sde_chacha_block<8>(key, (sde_u64)(j0 >> 3) + 1, b1);
-    const int w0 = (int)(j0 & 7);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int w = w0 + k;  // < 15
-      sde_u32 l = b0[0], h = b0[1];
-#pragma unroll
-      for (int q = 1; q < 16; ++q) {
-        l = (w == q) ? (q < 8 ? b0[2 * q] : b1[2 * q - 16]) : l;
-        h = (w == q) ? (q < 8 ? b0[2 * q + 1] : b1[2 * q - 15]) : h;
-      }
-      lo[k] = l;
-      hi[k] = h;
-    }
-  } else if constexpr (D == 8) {
-    sde_u32 blk[16];
-    sde_chacha_block<8>(key, (sde_u64)n, blk);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      lo[k] = blk[2 * k];
-      hi[k] = blk[2 * k + 1];
-    }
-  } else {
-    static_assert(D == 1, "the checkpoint form runs one asset or eight");
-    sde_u32 blk[16];
-    sde_chacha_block<8>(key, (sde_u64)(n >> 3), blk);
-    const int w = n & 7;
-    sde_u32 l = blk[0], h = blk[1];
-#pragma unroll
-    for (int q = 1; q < 8; ++q) {
-      l = (w == q) ? blk[2 * q] : l;
-      h = (w == q) ? blk[2 * q + 1] : h;
-    }
-    lo[0] = l;
-    hi[0] = h;
-  }
-}
 
 // f(0), f(1), .. f(N - 1) with the argument a constant.
 template <int I, int N, class F>
@@ -124,73 +70,12 @@ struct BasketNormals {
   }
 };
 
-template <typename R, int D>
-struct BasketStep {
-  R eps[D], Z[D];
-};
-
-// Z = L eps.
-template <typename R, int D>
-__device__ __forceinline__ void basket_correlate(const R (&L)[D][D], BasketStep<R, D>& st) {
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-    R z = R(0);
-#pragma unroll
-    for (int k = 0; k <= i; ++k) z = z + L[i][k] * st.eps[k];
-    st.Z[i] = z;
-  }
-}
-
-template <typename R, int D, bool PADDED>
-__device__ __forceinline__ void basket_noise(const sde_u32 (&key)[8], int n, int A, const R (&L)[D][D],
-                                             BasketStep<R, D>& st) {
-  sde_u32 lo[D], hi[D];
-  basket_draws<D, PADDED>(key, n, A, lo, hi);
-  sde_psi_words<D>(lo, hi, st.eps);
-  basket_correlate<R, D>(L, st);
-}
-
-template <typename R>
-__device__ __forceinline__ R basket_recip(R x) {
-  if constexpr (sizeof(R) == 4) return __builtin_amdgcn_rcpf(x);  // v_rcp_f32, 1 ulp
-  else return R(1) / x;
-}
-
-// One reverse step: x = X_n, xp = X_{n+1} (replaced by x on return), with the adjoint state
-// Xb = Xbar_{n+1} (replaced by Xbar_n) and the gradient sums gm, gs (sigma's, times sigma), gL.
-template <typename R, int D>
-__device__ __forceinline__ void basket_reverse_step(const R (&x)[D], R (&xp)[D], R (&Xb)[D], R (&gm)[D], R (&gs)[D],
-                                                    R (&gL)[D * (D + 1) / 2], const R (&L)[D][D], const R (&rLd)[D],
-                                                    const R (&mdt)[D], const R (&rsd)[D], const R (&sig)[D], R sdt,
-                                                    R dt) {
-  R Zb[D], Z[D], eps[D];
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-    const R xb = Xb[i], xi = x[i], xpi = xp[i];
-    const R rx = basket_recip<R>(xi);
-    const R d = (xpi - xi) - xi * mdt[i];
-    gm[i] = gm[i] + xb * xi * dt;
-    gs[i] = gs[i] + xb * d;
-    Zb[i] = xb * xi * sig[i] * sdt;
-    Z[i] = d * rx * rsd[i];
-    Xb[i] = xb * (xpi * rx);
-    xp[i] = xi;
-  }
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-    R r = Z[i];
-#pragma unroll
-    for (int kk = 0; kk < i; ++kk) r = r - L[i][kk] * eps[kk];
-    eps[i] = r * rLd[i];
-  }
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-#pragma unroll
-    for (int kk = 0; kk <= i; ++kk) {
-      const int q = i * (i + 1) / 2 + kk;
-      gL[q] = gL[q] + Zb[i] * eps[kk];
-    }
-  }
+// 1 / x: v_rcp_f32 (1 ulp), or the hardware seed (2^-24) and a third-order step (rounding of the
+// last sum only; x is a growth factor, far from f64's ends).
+__device__ __forceinline__ float basket_recip(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double basket_recip(double x) {
+  const double y = __builtin_amdgcn_rcp(x), e = __builtin_fma(-x, y, 1.0);
+  return __builtin_fma(y, __builtin_fma(e, e, e), y);
 }
 
 template <typename R>
@@ -215,115 +100,65 @@ __device__ __forceinline__ void basket_payoff(const R (&X)[D], const R (&w)[D], 
   }
 }
 
-// The reverse sweep's parameters (wave-uniform) and per-path adjoint state.
-template <typename R, int D>
-struct BasketReverse {
-  static constexpr int NL = BasketConst<D>::NL;
-  R L[D][D], sig[D], mdt[D], rsd[D], rLd[D];  // L, sigma, mu dt, 1 / (sigma sqrt(dt)), 1 / L_ii
-  R dt, sdt;
-  R Xb[D], gm[D], gs[D], gL[NL];
-  R Xp[D];  // the state after the step being reversed: X_N first, then each state stepped back to
+// The step's parameters in the path precision, in scalar registers: mu dt and sigma sqrt(dt) L.
+template <typename R>
+__device__ __forceinline__ R basket_mdt(const BasketArgs& a, int i) {
+  if constexpr (sizeof(R) == 4) return a.mdt_f[i];
+  else return a.mdt[i];
+}
+template <typename R>
+__device__ __forceinline__ R basket_scl(const BasketArgs& a, int i, int k) {
+  if constexpr (sizeof(R) == 4) return a.scl_f[i * 8 + k];
+  else return a.scl[i * 8 + k];
+}
 
-  __device__ __forceinline__ BasketReverse(const BasketArgs& a, const R (&XN)[D], R dpay) {
-    dt = (R)a.dt;
-    sdt = (R)a.sdt;
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-#pragma unroll
-      for (int k = 0; k < D; ++k) L[i][k] = (R)a.chol[i * 8 + k];
-      sig[i] = (R)a.sigma[i];
-      mdt[i] = (R)a.mu[i] * dt;
-      rsd[i] = R(1) / (sig[i] * sdt);
-      rLd[i] = R(1) / L[i][i];
-      Xb[i] = dpay * (R)a.weight[i];
-      gm[i] = R(0);
-      gs[i] = R(0);
-      Xp[i] = XN[i];
-    }
-#pragma unroll
-    for (int q = 0; q < NL; ++q) gL[q] = R(0);
-  }
-  __device__ __forceinline__ void step(const R (&x)[D]) {
-    basket_reverse_step<R, D>(x, Xp, Xb, gm, gs, gL, L, rLd, mdt, rsd, sig, sdt, dt);
-  }
-  // Gradient q of this path, q < 3 D + NL: d/dX0, d/dmu, d/dsigma, d/dL (q a constant after
-  // unrolling).
-  __device__ __forceinline__ double grad(int q) const {
-    if (q < D) return (double)Xb[q];
-    if (q < 2 * D) return (double)gm[q - D];
-    if (q < 3 * D) return (double)(gs[q - 2 * D] / sig[q - 2 * D]);
-    return (double)gL[q - 3 * D];
-  }
-};
-
-// MODE 0: price (two partials a block, payoff and payoff^2); 1: price and adjoint with checkpoints and recomputation; 2: the forward pass of
-// the tape form, which writes X_0 .. X_N to the tape and leaves the payoff, the reverse sweep and
-// every partial to sdesim_basket_reverse.
-template <typename R, int D, int SEG, int MODE, bool PADDED>
+// Price (two partials a block, payoff and payoff^2) or, with ADJ, price and derivatives.
+template <typename R, int D, bool ADJ>
 __global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
-  constexpr bool TAPE = MODE == 2;
+  constexpr int NL = BasketConst<D>::NL, NQ = BasketConst<D>::NQ;
+  constexpr int U = SdeChunk<D>::U;  // steps in a whole number of ChaCha blocks
   sde_normal_tab_load<R>(a.normal_tab);
-  constexpr int NQ = BasketConst<D>::NQ;
   const long long S = a.paths;
   const int N = a.steps;
   const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const bool live = s < S;
-  const long long sid = live ? s : 0;
-  const sde_u32 voff = live ? (sde_u32)(sid * (long long)sizeof(R)) : 0x80000000u;
-
-  R mu[D], sig[D], L[D][D];
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-    mu[i] = (R)a.mu[i];
-    sig[i] = (R)a.sigma[i];
-#pragma unroll
-    for (int k = 0; k < D; ++k) L[i][k] = (R)a.chol[i * 8 + k];
-  }
-  const R dt = (R)a.dt, sdt = (R)a.sdt;
 
   sde_u32 key[8];
-  sde_seed_from_u64(a.seed + (sde_u64)sid, key);
-  R X[D];
+  sde_seed_from_u64(a.seed + (sde_u64)(live ? s : 0), key);
+  R X[D], H[NL], Q[D];  // the state, the sums H of the header and sum_n 1 / g_n
 #pragma unroll
-  for (int i = 0; i < D; ++i) X[i] = (R)a.x0[i];
-
-  R* ck = (R*)a.states;
-  // Forward pass.
-  if constexpr (MODE == 1) {
-    for (int n = 0; n < N; ++n) {
-      if ((n % SEG) == 0 && live) {
-        const long long slot = n / SEG;
-#pragma unroll
-        for (int i = 0; i < D; ++i) ck[(slot * D + i) * S + sid] = X[i];
-      }
-      BasketStep<R, D> st;
-      basket_noise<R, D, PADDED>(key, n, a.assets, L, st);
-#pragma unroll
-      for (int i = 0; i < D; ++i) X[i] = X[i] + X[i] * (mu[i] * dt + sig[i] * sdt * st.Z[i]);
-    }
-  } else {
-    constexpr int U = SdeChunk<D>::U;  // steps in a whole number of ChaCha blocks
-    for (int n0 = 0; n0 < N; n0 += U) {
-      BasketNormals<R> noise;
-      basket_static_for<0, U>([&](auto u_) {
-        constexpr int u = u_;
-        if (U == 1 || n0 + u < N) {
-          if (TAPE) sde_tape_store<R, D>(a.states, n0 + u, S, voff, X);
-          BasketStep<R, D> st;
-          basket_static_for<0, D>([&](auto k_) {
-            constexpr int k = k_;
-            st.eps[k] = noise.template draw<u * D + k>(key, (sde_u64)n0 * D / 8);
-          });
-          basket_correlate<R, D>(L, st);
-#pragma unroll
-          for (int i = 0; i < D; ++i) X[i] = X[i] + X[i] * (mu[i] * dt + sig[i] * sdt * st.Z[i]);
-        }
-      });
-    }
+  for (int i = 0; i < D; ++i) {
+    X[i] = (R)a.x0[i];
+    Q[i] = R(0);
   }
-  if (TAPE) {
-    sde_tape_store<R, D>(a.states, N, S, voff, X);
-    return;
+#pragma unroll
+  for (int q = 0; q < NL; ++q) H[q] = R(0);
+
+  for (int n0 = 0; n0 < N; n0 += U) {
+    BasketNormals<R> noise;
+    basket_static_for<0, U>([&](auto u_) {
+      constexpr int u = u_;
+      if (U == 1 || n0 + u < N) {
+        R eps[D];
+        basket_static_for<0, D>([&](auto k_) {
+          constexpr int k = k_;
+          eps[k] = noise.template draw<u * D + k>(key, (sde_u64)n0 * D / 8);
+        });
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+          R c = basket_mdt<R>(a, i);
+#pragma unroll
+          for (int k = 0; k <= i; ++k) c = c + basket_scl<R>(a, i, k) * eps[k];
+          X[i] = X[i] + X[i] * c;
+          if constexpr (ADJ) {
+            const R r = basket_recip(R(1) + c);
+            Q[i] = Q[i] + r;
+#pragma unroll
+            for (int k = 0; k <= i; ++k) H[i * (i + 1) / 2 + k] = H[i * (i + 1) / 2 + k] + r * eps[k];
+          }
+        }
+      }
+    });
   }
   R w[D];
 #pragma unroll
@@ -331,75 +166,33 @@ __global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
   R pay, dpay;
   basket_payoff<R, D>(X, w, (R)a.strike, (R)a.width, pay, dpay);
 
-  if constexpr (MODE == 0) {
+  if constexpr (ADJ) {
+    R m[D], lh[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      m[i] = dpay * w[i] * X[i];
+      lh[i] = R(0);
+#pragma unroll
+      for (int k = 0; k <= i; ++k) lh[i] = lh[i] + (R)a.chol[i * 8 + k] * H[i * (i + 1) / 2 + k];
+    }
+    const R dt = (R)a.dt, sdt = (R)a.sdt;
+    // Derivative q of this path, q < 3 D + NL: d/dX0, d/dmu, d/dsigma, d/dL (q a constant after
+    // unrolling).
+    auto grad = [&](int q) -> double {
+      if (q < D) return (double)(m[q] / (R)a.x0[q]);
+      if (q < 2 * D) return (double)(m[q - D] * dt * Q[q - D]);
+      if (q < 3 * D) return (double)(m[q - 2 * D] * sdt * lh[q - 2 * D]);
+      int i = 0;
+      while ((i + 1) * (i + 2) / 2 <= q - 3 * D) ++i;
+      return (double)(m[i] * ((R)a.sigma[i] * sdt) * H[q - 3 * D]);
+    };
+    sde_reduce_store_chunked<NQ>(
+        [&](int q) { return !live ? 0.0 : q == 0 ? (double)pay : q == 1 ? (double)pay * (double)pay : grad(q - 2); },
+        a.partials + (long long)blockIdx.x * NQ);
+  } else {
     sde_reduce_store_chunked<2>([&](int q) { return !live ? 0.0 : q == 0 ? (double)pay : (double)pay * (double)pay; },
                                 a.partials + (long long)blockIdx.x * 2);
   }
-  if constexpr (MODE == 1) {
-    BasketReverse<R, D> rv(a, X, dpay);
-    for (int seg = (N + SEG - 1) / SEG - 1; seg >= 0; --seg) {
-      const int n0 = seg * SEG;
-      R Xs[SEG][D];
-      R Xc[D];
-#pragma unroll
-      for (int i = 0; i < D; ++i) Xc[i] = ck[((long long)seg * D + i) * S + sid];
-      // Recompute the segment's states.
-#pragma unroll
-      for (int k = 0; k < SEG; ++k) {
-#pragma unroll
-        for (int i = 0; i < D; ++i) Xs[k][i] = Xc[i];
-        if (n0 + k < N && k + 1 < SEG) {
-          BasketStep<R, D> st;
-          basket_noise<R, D, PADDED>(key, n0 + k, a.assets, L, st);
-#pragma unroll
-          for (int i = 0; i < D; ++i) Xc[i] = Xc[i] + Xc[i] * (mu[i] * dt + sig[i] * sdt * st.Z[i]);
-        }
-      }
-      // Step back through it.
-#pragma unroll
-      for (int k = SEG - 1; k >= 0; --k) {
-        if (n0 + k < N) rv.step(Xs[k]);
-      }
-    }
-    sde_reduce_store_chunked<NQ>(
-        [&](int q) { return !live ? 0.0 : q == 0 ? (double)pay : q == 1 ? (double)pay * (double)pay : rv.grad(q - 2); },
-        a.partials + (long long)blockIdx.x * NQ);
-  }
-}
-
-// Reverse sweep of the tape form: X_N from the tape gives the payoff, then the states X_{N-1} ..
-// X_0 are read back in two alternating register buffers, each requested one reverse step before
-// its use (the requests past step 0 are clamped to step 0 and unused).
-template <typename R, int D>
-__global__ void __launch_bounds__(256) sdesim_basket_reverse(const BasketArgs a) {
-  constexpr int NQ = BasketConst<D>::NQ;
-  const long long S = a.paths;
-  const int N = a.steps;
-  const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = s < S;
-  const sde_u32 voff = live ? (sde_u32)(s * (long long)sizeof(R)) : 0x80000000u;
-
-  R X[D], w[D];
-  sde_tape_load<R, D>(a.states, N, S, voff, X);
-#pragma unroll
-  for (int i = 0; i < D; ++i) w[i] = (R)a.weight[i];
-  R pay, dpay;
-  basket_payoff<R, D>(X, w, (R)a.strike, (R)a.width, pay, dpay);
-
-  BasketReverse<R, D> rv(a, X, dpay);
-  R xa[D], xb[D];
-  sde_tape_load<R, D>(a.states, N - 1, S, voff, xa);
-  int n = N - 1;
-  for (; n >= 1; n -= 2) {
-    sde_tape_load<R, D>(a.states, n - 1, S, voff, xb);
-    rv.step(xa);  // step n
-    sde_tape_load<R, D>(a.states, n >= 2 ? n - 2 : 0, S, voff, xa);
-    rv.step(xb);  // step n - 1
-  }
-  if (n == 0) rv.step(xa);
-  sde_reduce_store_chunked<NQ>(
-      [&](int q) { return !live ? 0.0 : q == 0 ? (double)pay : q == 1 ? (double)pay * (double)pay : rv.grad(q - 2); },
-      a.partials + (long long)blockIdx.x * NQ);
 }
 
 // Sum of per-block partials per quantity: one block of 1024 threads each, whose loads of 8 bytes
@@ -423,53 +216,28 @@ hipError_t sdesim_launch_sum_partials(const double* partials, int nblocks, int n
   return hipGetLastError();
 }
 
-// mode: 0 price, 1 adjoint with checkpoints (a.states holds [slots][D][paths], one per 19 steps, D = 1 or
-// 8), 2 adjoint with the tape (a.states holds [steps + 1][assets][paths]; a forward and a reverse kernel).
-// Price and tape have a kernel per asset count, which draws, correlates and stores no more than the
-// basket's own assets: 5 assets in f64 (30,001 paths x 252) took 745 us forward and 197 us
-// reverse in the 8-asset kernels, padded, each step from two ChaCha blocks (a step's draws do not start on a
-// block) with 15-way selects; 252 and 134 us in their own. The checkpoint form, which must start at any
-// step, keeps the padded 8-asset kernels for 2-7 assets.
-hipError_t sdesim_launch_basket(int f32, int assets, int mode, int grid, const BasketArgs& a, int nq,
+// A kernel per asset count, which draws, correlates and sums no more than the basket's own assets: padded to 8
+// assets, 5 in f64 took three times as long.
+hipError_t sdesim_launch_basket(int f32, int assets, int adjoint, int grid, const BasketArgs& a, int nq,
                                 double* sums, hipStream_t stream) {
-#define SDE_BASKET(R, D, MODE, PAD) \
-  hipLaunchKernelGGL((sdesim_basket<R, D, 19, MODE, PAD>), dim3(grid), dim3(256), 0, stream, a)
-#define SDE_BASKET_WIDTH(D)                                                                                         \
-  case D:                                                                                                           \
-    if (mode == 0) {                                                                                                \
-      if (f32) SDE_BASKET(float, D, 0, false);                                                                      \
-      else SDE_BASKET(double, D, 0, false);                                                                         \
-    } else if (f32) {                                                                                               \
-      SDE_BASKET(float, D, 2, false);                                                                               \
-      hipLaunchKernelGGL((sdesim_basket_reverse<float, D>), dim3(grid), dim3(256), 0, stream, a);                   \
-    } else {                                                                                                        \
-      SDE_BASKET(double, D, 2, false);                                                                              \
-      hipLaunchKernelGGL((sdesim_basket_reverse<double, D>), dim3(grid), dim3(256), 0, stream, a);                  \
-    }                                                                                                               \
+#define SDE_BASKET(R, D, ADJ) hipLaunchKernelGGL((sdesim_basket<R, D, ADJ>), dim3(grid), dim3(256), 0, stream, a)
+#define SDE_BASKET_WIDTH(D)                         \
+  case D:                                           \
+    if (f32 && adjoint) SDE_BASKET(float, D, true); \
+    else if (f32) SDE_BASKET(float, D, false);      \
+    else if (adjoint) SDE_BASKET(double, D, true);  \
+    else SDE_BASKET(double, D, false);              \
     break;
-  if (assets < 1 || assets > 8 || mode < 0 || mode > 2) return hipErrorInvalidValue;
-  if (mode == 1) {
-    if (assets == 1) {
-      if (f32) SDE_BASKET(float, 1, 1, false);
-      else SDE_BASKET(double, 1, 1, false);
-    } else if (assets == 8) {
-      if (f32) SDE_BASKET(float, 8, 1, false);
-      else SDE_BASKET(double, 8, 1, false);
-    } else {
-      if (f32) SDE_BASKET(float, 8, 1, true);
-      else SDE_BASKET(double, 8, 1, true);
-    }
-  } else {
-    switch (assets) {
-      SDE_BASKET_WIDTH(1)
-      SDE_BASKET_WIDTH(2)
-      SDE_BASKET_WIDTH(3)
-      SDE_BASKET_WIDTH(4)
-      SDE_BASKET_WIDTH(5)
-      SDE_BASKET_WIDTH(6)
-      SDE_BASKET_WIDTH(7)
-      SDE_BASKET_WIDTH(8)
-    }
+  switch (assets) {
+    SDE_BASKET_WIDTH(1)
+    SDE_BASKET_WIDTH(2)
+    SDE_BASKET_WIDTH(3)
+    SDE_BASKET_WIDTH(4)
+    SDE_BASKET_WIDTH(5)
+    SDE_BASKET_WIDTH(6)
+    SDE_BASKET_WIDTH(7)
+    SDE_BASKET_WIDTH(8)
+    default: return hipErrorInvalidValue;
   }
 #undef SDE_BASKET_WIDTH
 #undef SDE_BASKET

@@ -75,17 +75,16 @@ struct SdeItem {
 // Correlated GBM basket, price and adjoint (basket_kernels.hip)
 // ------------------------------------------------------------------------------------------
 struct BasketArgs {
-  double x0[8], mu[8], sigma[8], weight[8];
+  double x0[8], sigma[8], weight[8];
   double chol[64];            // lower Cholesky factor of the correlation, row-major 8 x 8
+  double mdt[8], scl[64];     // mu dt, and sigma_i sqrt(dt) chol_ik
+  float mdt_f[8], scl_f[64];  // the same in f32
   double dt, sdt, strike, width;
   sde_u64 seed;               // path s uses seed + s
   long long paths;
-  void* states;               // adjoint storage: the tape [steps][D][paths] real, or checkpoints
-                              // [slots][D][paths] real (one slot per 19 steps)
   double* partials;           // [gridDim.x][NQ]
   const void* normal_tab;     // table of the inverse normal in the kernel's precision
   int steps;
-  int assets;                 // the basket's asset count A: step n uses draws n * A .. n * A + A - 1
 };
 
 // ------------------------------------------------------------------------------------------

@@ -13,15 +13,13 @@
 #include "../../include/sdesim.h"
 #include "device/sdesim_args.hpp"
 
-hipError_t sdesim_launch_basket(int f32, int assets, int mode, int grid, const BasketArgs& a, int nq,
+hipError_t sdesim_launch_basket(int f32, int assets, int adjoint, int grid, const BasketArgs& a, int nq,
                                 double* sums, hipStream_t stream);
 hipError_t sdesim_normal_table(int f32, const void** out);
 int sdesim_set_error(int code, const std::string& msg);
 void sdesim_log(const char* fmt, ...);
 
 namespace {
-constexpr int kSeg = 19;  // checkpoint interval of the compiled reverse sweep
-
 struct BFail {
   int code;
   std::string msg;
@@ -44,16 +42,13 @@ int guard(F&& f) {
 
 struct sdesim_basket {
   sdesim_basket_spec spec{};
-  int D = 8;          // width of the adjoint's kernels: the assets (tape), 1 or 8 (checkpoints)
   int nq = 0;         // reduced quantities of the adjoint
   long long grid = 0;
-  int storage = SDESIM_STORAGE_CHECKPOINTS;  // resolved at creation: TAPE or CHECKPOINTS
-  void* states = nullptr;                   // the tape or the checkpoints
+  int storage = SDESIM_STORAGE_CHECKPOINTS;  // as asked for, or AUTO's choice; neither keeps states
   double* partials = nullptr;
   double* sums = nullptr;
   const void* normal_tab = nullptr;         // the device's shared table of the inverse normal
   ~sdesim_basket() {
-    if (states) (void)hipFree(states);
     if (partials) (void)hipFree(partials);
     if (sums) (void)hipFree(sums);
   }
@@ -74,37 +69,20 @@ int sdesim_basket_create(const sdesim_basket_spec* spec, sdesim_basket** out) {
       throw BFail{SDESIM_EVALUE, "storage must be SDESIM_STORAGE_AUTO, _TAPE or _CHECKPOINTS"};
     std::unique_ptr<sdesim_basket> b(new sdesim_basket());
     b->spec = s;
-    const int padded = s.assets == 1 ? 1 : 8;
     b->grid = (s.paths + 255) / 256;
     if (b->grid > 0x7fffffffLL) throw BFail{SDESIM_EVALUE, "too many paths"};
+    // The derivatives are summed on the way forward: no state is stored under either name. What a tape
+    // was refused for, a step of it (at 1 or 8 assets) of 2^31 bytes or more, still is.
     const size_t rb = s.precision == SDESIM_F32 ? 4 : 8;
-    const long long slots = (s.steps + kSeg - 1) / kSeg;
-    const size_t ck = (size_t)slots * padded * (size_t)s.paths * rb;
-    const size_t tape = (size_t)s.assets * (size_t)s.paths * rb * ((size_t)s.steps + 1);  // X_0 .. X_N
-    size_t free_b = 0, total_b = 0;
-    bk(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-    // One buffer resource per step (sized for the padded width, the widest kernels').
-    const bool tape_addressable = (size_t)padded * (size_t)s.paths * rb < (1ull << 31);
-    if (s.storage == SDESIM_STORAGE_TAPE) {
-      if (!tape_addressable) throw BFail{SDESIM_EVALUE, "the tape needs assets * paths * size < 2^31 bytes per step"};
-      if (tape + (64u << 20) > free_b) throw BFail{SDESIM_ERUNTIME, "the tape does not fit in free device memory"};
-      b->storage = SDESIM_STORAGE_TAPE;
-    } else if (s.storage == SDESIM_STORAGE_AUTO && tape_addressable && tape + (64u << 20) <= free_b / 2) {
-      b->storage = SDESIM_STORAGE_TAPE;
-    }
-    if (b->storage == SDESIM_STORAGE_TAPE) {
-      bk(hipMalloc(&b->states, tape), "hipMalloc(tape)");
-    } else {
-      if (ck + (64u << 20) > free_b) throw BFail{SDESIM_ERUNTIME, "checkpoints do not fit in free device memory"};
-      bk(hipMalloc(&b->states, ck), "hipMalloc(checkpoints)");
-    }
-    b->D = b->storage == SDESIM_STORAGE_TAPE ? s.assets : padded;
-    b->nq = 2 + 3 * b->D + b->D * (b->D + 1) / 2;
+    const bool tape_addressable = (size_t)(s.assets == 1 ? 1 : 8) * (size_t)s.paths * rb < (1ull << 31);
+    if (s.storage == SDESIM_STORAGE_TAPE && !tape_addressable)
+      throw BFail{SDESIM_EVALUE, "the tape needs assets * paths * size < 2^31 bytes per step"};
+    if (s.storage != SDESIM_STORAGE_CHECKPOINTS && tape_addressable) b->storage = SDESIM_STORAGE_TAPE;
+    b->nq = 2 + 3 * s.assets + s.assets * (s.assets + 1) / 2;
     bk(sdesim_normal_table(s.precision == SDESIM_F32 ? 1 : 0, &b->normal_tab), "inverse normal table");
     bk(hipMalloc(&b->partials, sizeof(double) * b->nq * b->grid), "hipMalloc(partials)");
     bk(hipMalloc(&b->sums, sizeof(double) * b->nq), "hipMalloc(sums)");
-    sdesim_log("basket: %d assets, %lld paths, %d steps, adjoint storage %s", s.assets, (long long)s.paths, s.steps,
-               b->storage == SDESIM_STORAGE_TAPE ? "tape" : "checkpoints");
+    sdesim_log("basket: %d assets, %lld paths, %d steps", s.assets, (long long)s.paths, s.steps);
     *out = b.release();
   });
 }
@@ -118,32 +96,34 @@ int sdesim_basket_eval(sdesim_basket* b, const double* x0, const double* mu, con
   return guard([&] {
     if (!b || !x0 || !mu || !sigma || !weight || !chol || !out) throw BFail{SDESIM_EVALUE, "null argument"};
     const sdesim_basket_spec& s = b->spec;
-    const int A = s.assets, D = b->D;
+    const int A = s.assets;
     BasketArgs a;
     std::memset(&a, 0, sizeof a);
-    for (int i = 0; i < 8; ++i) a.chol[i * 8 + i] = 1.0;  // padding assets: identity rows, zero weight
-    for (int i = 0; i < A; ++i) {
-      a.x0[i] = x0[i];
-      a.mu[i] = mu[i];
-      a.sigma[i] = sigma[i];
-      a.weight[i] = weight[i];
-      for (int k = 0; k < A; ++k) a.chol[i * 8 + k] = k <= i ? chol[i * A + k] : 0.0;
-    }
     a.dt = s.horizon / s.steps;
     a.sdt = std::sqrt(a.dt);
+    for (int i = 0; i < A; ++i) {
+      a.x0[i] = x0[i];
+      a.sigma[i] = sigma[i];
+      a.weight[i] = weight[i];
+      a.mdt[i] = mu[i] * a.dt;
+      a.mdt_f[i] = (float)a.mdt[i];
+      for (int k = 0; k <= i; ++k) {
+        const int q = i * 8 + k;
+        a.chol[q] = chol[i * A + k];
+        a.scl[q] = sigma[i] * a.sdt * a.chol[q];
+        a.scl_f[q] = (float)a.scl[q];
+      }
+    }
     a.strike = s.strike;
     a.width = s.width;
     a.seed = s.seed;
     a.paths = s.paths;
     a.steps = s.steps;
-    a.states = b->states;
     a.partials = b->partials;
-    a.assets = A;
     a.normal_tab = b->normal_tab;
     hipStream_t st = (hipStream_t)stream;
     const int nq = adjoint ? b->nq : 2;
-    const int mode = !adjoint ? 0 : b->storage == SDESIM_STORAGE_TAPE ? 2 : 1;
-    bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, mode, (int)b->grid, a, nq, b->sums, st),
+    bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, adjoint != 0, (int)b->grid, a, nq, b->sums, st),
        "basket launch");
     std::vector<double> sums(nq);
     bk(hipMemcpyAsync(sums.data(), b->sums, sizeof(double) * nq, hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
@@ -152,16 +132,8 @@ int sdesim_basket_eval(sdesim_basket* b, const double* x0, const double* mu, con
     const double m1 = sums[0] / n;
     out[0] = m1;
     out[1] = s.paths > 1 ? (sums[1] - sums[0] * m1) / (n - 1.0) : 0.0;
-    if (adjoint) {
-      for (int i = 0; i < A; ++i) {
-        out[2 + i] = sums[2 + i] / n;
-        out[2 + A + i] = sums[2 + D + i] / n;
-        out[2 + 2 * A + i] = sums[2 + 2 * D + i] / n;
-      }
-      int q = 2 + 3 * A;
-      for (int i = 0; i < A; ++i)
-        for (int k = 0; k <= i; ++k) out[q++] = sums[2 + 3 * D + i * (i + 1) / 2 + k] / n;
-    }
+    if (adjoint)
+      for (int q = 2; q < nq; ++q) out[q] = sums[q] / n;
   });
 }
 

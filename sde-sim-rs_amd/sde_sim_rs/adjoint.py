@@ -66,10 +66,9 @@ _STORAGE = {"auto": nat.STORAGE_AUTO, "tape": nat.STORAGE_TAPE, "checkpoints": n
 class Basket:
     """Price and adjoint of a weighted basket call on D <= 8 correlated GBM assets.
 
-    `storage` picks how the adjoint keeps the forward states: "tape" (every state in device
-    memory, (steps + 1) * assets * paths values), "checkpoints" (every 19th state, the rest
-    recomputed during the reverse sweep) or "auto" (the tape when it fits in half of the free
-    device memory). `self.storage` is the form in use."""
+    The adjoint's sums are formed on the way forward, with no state kept: `storage` ("auto", "tape" or
+    "checkpoints") is accepted and reported in `self.storage`, and makes no difference. "tape" is
+    refused where a step's states reach 2^31 bytes; "auto" is then "checkpoints"."""
 
     def __init__(self, assets, steps, paths, horizon=1.0, strike=100.0, width=0.5, seed=0, precision="f32",
                  storage="auto"):
