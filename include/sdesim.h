@@ -236,8 +236,8 @@ typedef struct sdesim_basket_spec {
   int32_t storage;    /* adjoint state storage: SDESIM_STORAGE_AUTO, _TAPE or _CHECKPOINTS */
 } sdesim_basket_spec;
 
-/* Adjoint state storage. Forward-rate model: TAPE keeps every state in device memory
- * ((steps + 1) * 40 * paths values in the path precision, one write and one read each);
+/* Adjoint state storage. Forward-rate model: TAPE keeps every second state in device memory
+ * (((steps + 1) / 2 + 1) * 40 * paths values in the path precision, one write and one read each);
  * CHECKPOINTS keeps every 16th state and recomputes the rest during the reverse sweep (one more
  * forward pass of arithmetic, for that factor less memory); AUTO takes the tape when it fits in half of
  * the free device memory at creation, otherwise checkpoints. Basket: its adjoint keeps no states, and

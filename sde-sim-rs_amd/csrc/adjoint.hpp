@@ -1,8 +1,8 @@
-// adjoint.hpp -- pieces shared by the adjoint kernels (basket_kernels.hip, lmm_kernels.hip): the
-// state tape of the reverse sweeps and a chunked per-block reduction of the per-path results.
+// adjoint.hpp -- the state tape of the forward-rate model's reverse sweep; a reciprocal and a chunked
+// per-block reduction of per-path results, shared with the basket.
 //
-// Tape layout [step][row][path]: row r of step n holds one state variable of every path. The ROWS rows
-// of a step sit under one buffer resource of ROWS * S * sizeof(R) bytes (below 2^31, checked by
+// Tape layout [slot][row][path]: row r of a slot holds one state variable of every path. The ROWS rows
+// of a slot sit under one buffer resource of ROWS * S * sizeof(R) bytes (below 2^31, checked by
 // the host); the path's byte offset is the vector offset and the row's the scalar offset. Lanes
 // past the last path pass vector offset 2^31, beyond the resource: their stores are dropped and
 // their loads return 0, so no exec-masked branch surrounds the accesses. Both directions use the
@@ -11,47 +11,62 @@
 
 #include "device/sdesim_device.hpp"
 
+// 1 / x: v_rcp_f32 (1 ulp), or the hardware seed (2^-24) and a third-order step (rounding of the
+// last sum only; x is a growth or discount factor, far from f64's ends).
+__device__ __forceinline__ float sde_recip(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double sde_recip(double x) {
+  const double y = __builtin_amdgcn_rcp(x), e = __builtin_fma(-x, y, 1.0);
+  return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
+
+// One slot: its resource and a row's bytes. The latter is opaque to the compiler, which otherwise forms the
+// ROWS row offsets once for the kernel, has no scalar registers for them and reads each from a vector
+// register's lane at its use.
+struct SdeTapeSlot {
+  __amdgpu_buffer_rsrc_t rs;
+  int row_bytes;
+};
+
 // n is wave-uniform; readfirstlane keeps the resource in scalar registers even where the index
 // was formed by a vector instruction (a clamped subtraction, say), which would otherwise make
 // the compiler wrap every access in a loop over distinct resources.
 template <typename R, int ROWS>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t sde_tape_rsrc(void* tape, int n, long long S) {
+__device__ __forceinline__ SdeTapeSlot sde_tape_slot(void* tape, int n, long long S) {
   n = __builtin_amdgcn_readfirstlane(n);
-  const long long step_bytes = (long long)ROWS * S * (long long)sizeof(R);
-  return __builtin_amdgcn_make_buffer_rsrc((void*)((char*)tape + (long long)n * step_bytes), (short)0, (int)step_bytes,
+  const long long slot_bytes = (long long)ROWS * S * (long long)sizeof(R);
+  SdeTapeSlot t;
+  t.rs = __builtin_amdgcn_make_buffer_rsrc((void*)((char*)tape + (long long)n * slot_bytes), (short)0, (int)slot_bytes,
                                            0x00020000);
+  t.row_bytes = (int)(S * (long long)sizeof(R));
+  asm volatile("" : "+s"(t.row_bytes));
+  return t;
 }
 
 template <typename R>
-__device__ __forceinline__ void sde_tape_put(__amdgpu_buffer_rsrc_t rs, sde_u32 voff, int row, long long S, R v) {
-  const int soff = (int)((long long)row * S * (long long)sizeof(R));
+__device__ __forceinline__ R sde_tape_get(const SdeTapeSlot& t, sde_u32 voff, int row) {
   if constexpr (sizeof(R) == 4)
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(sde_u32, (float)v), rs, (int)voff, soff, 2);
+    return __builtin_bit_cast(float, (sde_u32)__builtin_amdgcn_raw_buffer_load_b32(t.rs, (int)voff, row * t.row_bytes, 2));
   else
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(SdeU32x2, (double)v), rs, (int)voff, soff, 2);
-}
-
-template <typename R>
-__device__ __forceinline__ R sde_tape_get(__amdgpu_buffer_rsrc_t rs, sde_u32 voff, int row, long long S) {
-  const int soff = (int)((long long)row * S * (long long)sizeof(R));
-  if constexpr (sizeof(R) == 4)
-    return __builtin_bit_cast(float, (sde_u32)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)voff, soff, 2));
-  else
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, (int)voff, soff, 2));
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(t.rs, (int)voff, row * t.row_bytes, 2));
 }
 
 template <typename R, int ROWS>
 __device__ __forceinline__ void sde_tape_store(void* tape, int n, long long S, sde_u32 voff, const R (&X)[ROWS]) {
-  const __amdgpu_buffer_rsrc_t rs = sde_tape_rsrc<R, ROWS>(tape, n, S);
+  const SdeTapeSlot t = sde_tape_slot<R, ROWS>(tape, n, S);
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i) sde_tape_put<R>(rs, voff, i, S, X[i]);
+  for (int i = 0; i < ROWS; ++i) {
+    if constexpr (sizeof(R) == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(sde_u32, (float)X[i]), t.rs, (int)voff, i * t.row_bytes, 2);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(SdeU32x2, (double)X[i]), t.rs, (int)voff, i * t.row_bytes, 2);
+  }
 }
 
 template <typename R, int ROWS>
 __device__ __forceinline__ void sde_tape_load(void* tape, int n, long long S, sde_u32 voff, R (&X)[ROWS]) {
-  const __amdgpu_buffer_rsrc_t rs = sde_tape_rsrc<R, ROWS>(tape, n, S);
+  const SdeTapeSlot t = sde_tape_slot<R, ROWS>(tape, n, S);
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i) X[i] = sde_tape_get<R>(rs, voff, i, S);
+  for (int i = 0; i < ROWS; ++i) X[i] = sde_tape_get<R>(t, voff, i);
 }
 
 // One partial per block of each of the NQ per-path values get(q): a butterfly over the wave's

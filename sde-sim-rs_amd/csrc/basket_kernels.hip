@@ -70,14 +70,6 @@ struct BasketNormals {
   }
 };
 
-// 1 / x: v_rcp_f32 (1 ulp), or the hardware seed (2^-24) and a third-order step (rounding of the
-// last sum only; x is a growth factor, far from f64's ends).
-__device__ __forceinline__ float basket_recip(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double basket_recip(double x) {
-  const double y = __builtin_amdgcn_rcp(x), e = __builtin_fma(-x, y, 1.0);
-  return __builtin_fma(y, __builtin_fma(e, e, e), y);
-}
-
 template <typename R>
 __device__ __forceinline__ R basket_softplus(R x) {
   // log(1 + e^x) without overflow: max(x, 0) + log1p(exp(-|x|))
@@ -151,7 +143,7 @@ __global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
           for (int k = 0; k <= i; ++k) c = c + basket_scl<R>(a, i, k) * eps[k];
           X[i] = X[i] + X[i] * c;
           if constexpr (ADJ) {
-            const R r = basket_recip(R(1) + c);
+            const R r = sde_recip(R(1) + c);
             Q[i] = Q[i] + r;
 #pragma unroll
             for (int k = 0; k <= i; ++k) H[i * (i + 1) / 2 + k] = H[i * (i + 1) / 2 + k] + r * eps[k];

@@ -92,14 +92,15 @@ struct BasketArgs {
 // ------------------------------------------------------------------------------------------
 struct LmmArgs {
   double L0[40];                      // initial forwards
-  const double* pard;                 // device [40] volatilities then [40][3] loadings (f64)
-  const float* parf;                  // the same in f32
+  const void* rows;                   // device [41][8] real, the forward step's parameter rows and a row of zeros
+  const void* rows_back;              // the step back's
   double dt, sdt, tau, strike;
   long long paths;
   const sde_u32* sobol_tab;           // slice 0 as [steps][64][3], the mask complements folded in
   const sde_u32* sobol_up;            // slices 1-2 as [2][256][steps * 3]
   void* checkpoints;                  // [slots][40][paths] real, one slot per 16 steps
-  void* tape;                         // [16][40][paths] real, the states of one segment
+  void* tape;                         // [16][40][paths] real, the states of one segment; or the state
+                                      // tape [(steps + 1) / 2 + 1][40][paths]: L_0, L_2, .. and L_N
   double* partials;                   // [gridDim.x][42]
   const void* normal_tab;             // table of the f64 inverse normal
   int steps;
@@ -107,5 +108,4 @@ struct LmmArgs {
   int expiry_index;
   int sobol_tab_words;
   int sobol_dims;                     // steps * 3, the row length of sobol_up
-  int zero;                           // always 0: makes per-step parameter reads step-dependent
 };

@@ -14,17 +14,22 @@
 // fixed rate K: V = max(K A - (1 - P_{NF-1}), 0) / N, P_j = prod_{k=e..j} 1 / (1 + tau L_k),
 // A = tau sum_{j=e..NF-1} P_j, numeraire N = prod_{k<e} (1 + tau L_k).
 //
-// Adjoint: the reverse sweep needs every state L_n. Two storage forms:
-//  * state tape (MODE 2): the forward pass writes L_0 .. L_N to HBM ([n][i][path], 27 GB for
-//    161 states x 40 forwards x 2^20 paths in f32) and a second kernel reads them back;
+// Adjoint: in logarithms. With M_i = Lbar_i L_i (the derivative with respect to ln L_i) and
+// a_j = tau sig_j L_j / (1 + tau L_j), one step back is, L the state before it,
+//   G_f(j) = sum_{i >= j} M'_i sig_i B_if (a suffix sum),
+//   M_j = M'_j + dt (sum_f B_jf G_f(j)) tau sig_j L_j / (1 + tau L_j)^2,
+// which needs neither the state after the step nor a quotient of the two. The states come from
+//  * the state tape (MODE 2): the forward pass writes every second state, L_0, L_2, .. and L_N, to HBM
+//    ([slot][i][path], 13.6 GB for 160 steps x 40 forwards x 2^20 paths in f32); a second kernel reads them
+//    back and recomputes the states between;
 //  * checkpoints (MODE 1): the forward pass stores L every SEG steps ([slot][i][path]); the
 //    reverse sweep takes the segments last to first, recomputes a segment's states once from its
 //    checkpoint into the segment tape ([k][i][path], rewritten per segment) and then steps back
 //    through them.
-// For one step, with a_j = tau sig_j L_j / (1 + tau L_j) and
-// E_i = L'_i / L_i (read as the ratio of the stored states, so the reverse step needs no exp):
-//   Cbar_f(i) = Lbar'_i L'_i dt sig_i B_if,   G_f(j) = sum_{i >= j} Cbar_f(i)  (a suffix sum),
-//   Lbar_j = Lbar'_j E_j + (sum_f B_jf G_f(j)) tau sig_j / (1 + tau L_j)^2.
+// Price and sensitivities at that size, f32: 6.8 ms, VALU issue and the chains within a step (forward kernel
+// 2.9, reverse 3.9); 9.7 with every state on the tape and a step back in Lbar, which holds the states on both
+// sides of it: both kernels then waited for HBM. The price alone: 2.55, and 2.7 with three more operations
+// per forward and parameters from LDS.
 #include <hip/hip_runtime.h>
 
 #include "device/sdesim_device.hpp"
@@ -69,149 +74,149 @@ __device__ __forceinline__ void lmm_noise(__amdgpu_buffer_rsrc_t rsrc, const Lmm
   }
 }
 
-// Model parameters: the workgroup stages them once from the device buffer ([40] volatilities
-// then [40][3] loadings) into LDS, one 8-value row per forward with the step's constant products
-// precomputed, so a forward's parameters are two broadcast LDS reads. Each step reads them at
-// index i + off, where off = step * a.zero is 0 at run time but not known to the compiler: the
-// reads repeat per step (issued ahead of use within the step) instead of 320 loop-invariant
-// values being hoisted into registers for the whole kernel.
+// Model parameters: one 8-value row per forward with the step's constant products precomputed, in device
+// memory, read with scalar loads so that a row's values are scalar operands of the arithmetic. Each
+// step reads them at a pointer the compiler cannot see through: the reads repeat per step (and hit the
+// scalar cache) instead of 320 loop-invariant values being hoisted and spilled. From LDS, two
+// broadcast reads per forward took as long as the forward's arithmetic (16 cycles of the CU's LDS for a
+// wave, against 60 of one of its four SIMDs).
 template <typename R>
-struct LmmParRow {
-  R ts;           // tau sigma_i
-  R b0, b1, b2;   // loadings B_i0..B_i2
-  R q0, q1, q2;   // sigma_i B_i0..B_i2
-  R h;            // -sigma_i^2 dt / 2 (f32: times log2 e)
-};
-
+using LmmRow = R __attribute__((ext_vector_type(8)));  // ts, b0, b1, b2, q0, q1, q2, h:
+//          forward rows              step back
+//   ts     tau sigma_i sqrt(dt)      tau sigma_i dt
+//   b      loadings B_if             loadings B_if
+//   q      sigma_i B_if sqrt(dt) un  sigma_i B_if
+//   h      -sigma_i^2 dt / 2 un
+// un is 1, or log2 e for f32, whose exponential has base 2. (sqrt(dt) is in each row's values, rounded once
+// there: as a factor of its own its rounding would be common to every forward and step.)
 template <typename R>
-struct LmmPar {
-  const LmmParRow<R>* rows;  // LDS, already advanced by the step's offset
-  __device__ __forceinline__ LmmParRow<R> row(int i) const { return rows[i]; }
-};
-
-// The step's view of the parameter rows: rows + off, with the offset moved into a vector register
-// the compiler cannot see through, so the LDS address is formed once per step and each forward's
-// reads use it with constant offsets (with the offset in a scalar register the compiler copies
-// the address into a vector register again in every forward's branch).
+using LmmRows = __attribute__((address_space(4))) const LmmRow<R>*;
 template <typename R>
-__device__ __forceinline__ LmmPar<R> lmm_par(const LmmParRow<R>* rows, int off) {
-  asm volatile("" : "+v"(off));
-  return LmmPar<R>{rows + off};
+__device__ __forceinline__ LmmRows<R> lmm_rows(const void* rows) {
+  sde_u64 p = (sde_u64)rows;
+  asm volatile("" : "+s"(p));
+  return (LmmRows<R>)p;
 }
 
-template <typename R>
-__device__ __forceinline__ R lmm_recip(R x) {
-  if constexpr (sizeof(R) == 4) return __builtin_amdgcn_rcpf(x);  // v_rcp_f32, 1 ulp
-  else return R(1) / x;
-}
-
-// One log-Euler step of all alive forwards (forwards below `eta` are dead and unchanged). The
-// exponent (sigma_i (B_i.C) - sigma_i^2 / 2) dt + sigma_i sqrt(dt) (B_i.eps) is formed as
-// q_i.(dt C + sqrt(dt) eps) + h_i with q_i = sigma_i B_i: the step's sqrt(dt) eps is shared by all
-// forwards. dtu and sdtu are dt and sqrt(dt) in the exponent's unit (log2 e for f32).
-template <typename R>
-__device__ __forceinline__ void lmm_step(const LmmPar<R>& tab, R (&L)[NF], const R (&eps)[F], int eta, R dtu, R sdtu,
-                                         R tau) {
-  R C[F] = {R(0), R(0), R(0)};
-  const R se0 = sdtu * eps[0], se1 = sdtu * eps[1], se2 = sdtu * eps[2];
+// f(i, row) for the alive forwards i >= eta, upwards or downwards. A group of four with no dead forward has
+// no branch inside, so the forwards' chains overlap, and loads its rows together. The second test is on a copy of
+// eta that the compiler does not know to be one: joined into an if and else, the two sides' results would
+// meet in copies of all the state.
+template <typename R, bool DOWN, class Fn>
+__device__ __forceinline__ void lmm_alive(LmmRows<R> rows, int eta, const Fn& f) {
+  int eta2 = eta;
+  asm volatile("" : "+s"(eta2));
 #pragma unroll
-  for (int i = 0; i < NF; ++i) {
-    if (i >= eta) {
-      const LmmParRow<R> pr = tab.row(i);
-      const R ai = pr.ts * L[i] * lmm_recip<R>(R(1) + tau * L[i]);
-      C[0] = C[0] + ai * pr.b0;
-      C[1] = C[1] + ai * pr.b1;
-      C[2] = C[2] + ai * pr.b2;
-      const R x = pr.q0 * (dtu * C[0] + se0) + pr.q1 * (dtu * C[1] + se1) + pr.q2 * (dtu * C[2] + se2) + pr.h;
-      L[i] = L[i] * lmm_exp_row<R>(x);
+  for (int g = 0; g < NF / 4; ++g) {
+    const int i0 = 4 * (DOWN ? NF / 4 - 1 - g : g);
+    if (i0 >= eta) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = DOWN ? i0 + 3 - j : i0 + j;
+        const LmmRow<R> r = rows[i];
+        f(i, r);
+      }
+    }
+    if (i0 < eta2 && i0 + 3 >= eta2) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = DOWN ? i0 + 3 - j : i0 + j;
+        if (i >= eta2) {
+          const LmmRow<R> r = rows[i];
+          f(i, r);
+        }
+      }
     }
   }
 }
 
-// Adjoint of one forward's part of lmm_step, forwards taken from the last down: Li and Lpi are
-// L_i before and after the step, Lbi the adjoint of Lp_i on entry and of L_i on exit, G the
-// running sums over the forwards above. Forwards are positive, so E_i = Lp_i / L_i.
+// One log-Euler step of all alive forwards (forwards below `eta` are dead: Lp is L, or left alone). With
+// D_f = eps_f + sqrt(dt) C_f, kept as one running sum, the exponent is sqrt(dt) q_i.D + h_i, q_i = sigma_i B_i.
 template <typename R>
-__device__ __forceinline__ void lmm_forward_adjoint(const LmmParRow<R>& pr, R Li, R Lpi, R& Lbi, R (&G)[F], R dt,
-                                                    R tau) {
-  const R b0 = pr.b0, b1 = pr.b1, b2 = pr.b2;
-  const R db = Lbi * Lpi * dt;
-  G[0] = G[0] + db * pr.q0;
-  G[1] = G[1] + db * pr.q1;
-  G[2] = G[2] + db * pr.q2;
-  const R ab = b0 * G[0] + b1 * G[1] + b2 * G[2];
-  const R rop = lmm_recip<R>(R(1) + tau * Li);
-  Lbi = Lbi * (Lpi * lmm_recip<R>(Li)) + ab * pr.ts * (rop * rop);
+__device__ __forceinline__ void lmm_step(LmmRows<R> rows, const R (&L)[NF], R (&Lp)[NF], const R (&eps)[F], int eta,
+                                         R tau) {
+  R D[F] = {eps[0], eps[1], eps[2]};
+  lmm_alive<R, false>(rows, eta, [&](int i, const LmmRow<R>& r) {
+    const R ai = r[0] * L[i] * sde_recip(R(1) + tau * L[i]);
+#pragma unroll
+    for (int f = 0; f < F; ++f) D[f] = D[f] + ai * r[1 + f];
+    Lp[i] = L[i] * lmm_exp_row<R>(r[4] * D[0] + r[5] * D[1] + r[6] * D[2] + r[7]);
+  });
 }
 
-// Adjoint of lmm_step: L is the state before the step and Lp the state after it; on entry Lb is
-// the adjoint of Lp, on exit the adjoint of L.
+// One step back: L is the state before the step; M on entry that of the state after it.
 template <typename R>
-__device__ __forceinline__ void lmm_step_adjoint(const LmmPar<R>& tab, const R (&L)[NF], const R (&Lp)[NF],
-                                                 R (&Lb)[NF], int eta, R dt, R tau) {
+__device__ __forceinline__ void lmm_step_back(LmmRows<R> rows, const R (&L)[NF], R (&M)[NF], int eta, R tau) {
   R G[F] = {R(0), R(0), R(0)};
+  lmm_alive<R, true>(rows, eta, [&](int i, const LmmRow<R>& r) {
 #pragma unroll
-  for (int i = NF - 1; i >= 0; --i) {
-    if (i >= eta) lmm_forward_adjoint<R>(tab.row(i), L[i], Lp[i], Lb[i], G, dt, tau);
-  }
+    for (int f = 0; f < F; ++f) G[f] = G[f] + M[i] * r[4 + f];
+    const R ab = r[1] * G[0] + r[2] * G[1] + r[3] * G[2];
+    const R rop = sde_recip(R(1) + tau * L[i]);
+    M[i] = M[i] + ab * (r[0] * L[i] * rop * rop);
+  });
 }
 
-// Payoff at the final forwards L (discounted by the spot numeraire) and, with GRAD, its
-// derivatives dV/dL_k in Lb: the numeraire part for k < e, the swap part for k >= e (only when
-// in the money).
+// Payoff at the final forwards L (discounted by the spot numeraire) and, with GRAD, its derivatives
+// dV/d ln L_k in M: the numeraire part for k < e, the swap part for k >= e (only when in the money). In f64
+// for f32 paths too: 36 rounded discount factors left the swap's value 3e-7 off, which decided on the wrong
+// side for a path or two in 2^20, each 1e-6 of a sensitivity. It is one part in 100 of the path's work.
 template <typename R, bool GRAD>
-__device__ __forceinline__ R lmm_payoff(const R (&L)[NF], int e, R tau, R K, R (&Lb)[NF]) {
-  R numer = R(1);
+__device__ __forceinline__ double lmm_payoff(const LmmArgs& a, const R (&L)[NF], R (&M)[NF]) {
+  const int e = a.expiry_index;
+  const double tau = a.tau, K = a.strike;
+  double numer = 1.0, P = 1.0, A = 0.0;
 #pragma unroll
-  for (int k = 0; k < NF; ++k)
-    if (k < e) numer = numer * (R(1) + tau * L[k]);
-  R P = R(1), A = R(0);
-  R Pj[NF];
-#pragma unroll
-  for (int j = 0; j < NF; ++j) {
-    Pj[j] = R(0);
-    if (j >= e) {
-      P = P / (R(1) + tau * L[j]);
-      Pj[j] = P;
+  for (int k = 0; k < NF; ++k) {
+    const double op = 1.0 + tau * (double)L[k];
+    if (k < e) {
+      numer = numer * op;
+    } else {
+      P = P * sde_recip(op);
       A = A + tau * P;
     }
   }
-  const R U = K * A - (R(1) - P);
-  const R V = U > R(0) ? U / numer : R(0);
+  const double U = K * A - (1.0 - P), rn = sde_recip(numer);
+  const double V = U > 0.0 ? U * rn : 0.0;
   if (GRAD) {
-    R tail = R(0);  // sum_{j >= k} P_j, built from the end
+    const double itm = U > 0.0 ? rn : 0.0;
+    double Pk = P, tail = 0.0;  // P_k, and sum_{j >= k} P_j from the end
 #pragma unroll
     for (int k = NF - 1; k >= 0; --k) {
-      if (k >= e) tail = tail + Pj[k];
-      const R op = R(1) + tau * L[k];
+      const double op = 1.0 + tau * (double)L[k], x = tau * (double)L[k] * sde_recip(op);
       if (k < e) {
-        Lb[k] = -V * tau / op;
+        M[k] = (R)(-V * x);
       } else {
-        Lb[k] = U > R(0) ? (-K * tau * tau * tail - tau * P) / (op * numer) : R(0);
+        tail = tail + Pk;
+        M[k] = (R)((-K * tau * tail - P) * itm * x);
+        Pk = Pk * op;
       }
     }
   }
   return V;
 }
 
-// Model parameters staged into LDS by the first NF threads of the workgroup.
-template <typename R>
-__device__ __forceinline__ void lmm_stage_params(const LmmArgs& a, LmmParRow<R>* par_rows) {
-  if (threadIdx.x < NF) {
-    const R dt = (R)a.dt, tau = (R)a.tau;
-    const R* par = sizeof(R) == 4 ? (const R*)(const void*)a.parf : (const R*)(const void*)a.pard;
-    const int i = (int)threadIdx.x;
-    const R sig = par[i];
-    const R un = sizeof(R) == 4 ? R(1.4426950408889634) : R(1);  // exponent unit: log2 e for f32
-    const R b0 = par[NF + i * F], b1 = par[NF + i * F + 1], b2 = par[NF + i * F + 2];
-    par_rows[i] = LmmParRow<R>{tau * sig, b0, b1, b2, sig * b0, sig * b1, sig * b2, R(-0.5) * sig * sig * dt * un};
+// The lane's Sobol entry and the wave's rows. Point index = path index; blocks of 256 make every wave one
+// aligned run of 64 indices. Lane 0 has the wave's smallest index: if it is past the last path so is every
+// lane of the wave, whose values are then never used.
+__device__ __forceinline__ LmmSobol lmm_sobol(const LmmArgs& a, long long sid) {
+  LmmSobol sb;
+  const sde_u64 g = (sde_u64)sid ^ ((sde_u64)sid >> 1);
+  sb.voff0 = (sde_u32)(g & 63u) * (sde_u32)(F * 4);
+#pragma unroll
+  for (int sl = 1; sl < NSL; ++sl) {
+    const sde_u32 e = __builtin_amdgcn_readfirstlane((sde_u32)(g >> (6 + 8 * (sl - 1))) & 255u);
+    sb.urow[sl - 1] = (sde_const_u32*)a.sobol_up + ((size_t)(sl - 1) * 256u + e) * (size_t)a.sobol_dims;
   }
-  __syncthreads();
+  return sb;
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t lmm_sobol_rsrc(const LmmArgs& a) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)a.sobol_tab, (short)0, a.sobol_tab_words * 4, 0x00020000);
 }
 
 // MODE 0: price; 1: price and adjoint with checkpoints, the reverse sweep recomputing each
-// segment into the segment tape; 2: the forward pass of the tape form, which writes L_0 .. L_N to
-// the state tape and leaves the payoff, the reverse sweep and every partial to
+// segment into the segment tape; 2: the forward pass of the tape form, which writes every second state and
+// L_N to the state tape and leaves the payoff, the reverse sweep and every partial to
 // sdesim_lmm_reverse. The f32 checkpoint adjoint is held to 3 waves per SIMD (168 VGPRs): the
 // extra wave hides the tape and LDS latency of its reverse sweep.
 template <typename R, int MODE>
@@ -225,36 +230,18 @@ sdesim_lmm(const LmmArgs a) {
   const bool live = s < S;
   const long long sid = live ? s : 0;
   const sde_u32 voff = live ? (sde_u32)(sid * (long long)sizeof(R)) : 0x80000000u;
-  const R dt = (R)a.dt, tau = (R)a.tau, K = (R)a.strike;
-  const R un = sizeof(R) == 4 ? R(1.4426950408889634) : R(1);  // exponent unit: log2 e for f32
-  const R dtu = (R)a.dt * un, sdtu = (R)a.sdt * un;
-  const int e = a.expiry_index;
+  const R tau = (R)a.tau;
 
-  __shared__ LmmParRow<R> par_rows[NF];
-  lmm_stage_params<R>(a, par_rows);
-
-  LmmSobol sb;
-  {
-    // Point index = path index; blocks of 256 make every wave one aligned run of 64 indices.
-    // Lane 0 has the wave's smallest index: if it is past the last path so is every lane of the
-    // wave, whose values are then never used.
-    const sde_u64 g = (sde_u64)sid ^ ((sde_u64)sid >> 1);
-    sb.voff0 = (sde_u32)(g & 63u) * (sde_u32)(F * 4);
-#pragma unroll
-    for (int sl = 1; sl < NSL; ++sl) {
-      const sde_u32 e = __builtin_amdgcn_readfirstlane((sde_u32)(g >> (6 + 8 * (sl - 1))) & 255u);
-      sb.urow[sl - 1] = (sde_const_u32*)a.sobol_up + ((size_t)(sl - 1) * 256u + e) * (size_t)a.sobol_dims;
-    }
-  }
-  __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)a.sobol_tab, (short)0, a.sobol_tab_words * 4, 0x00020000);
+  const LmmSobol sb = lmm_sobol(a, sid);
+  const __amdgpu_buffer_rsrc_t rsrc = lmm_sobol_rsrc(a);
 
   R L[NF];
 #pragma unroll
   for (int i = 0; i < NF; ++i) L[i] = (R)a.L0[i];
   R* ck = (R*)a.checkpoints;
+  int eta = 1, left = a.steps_per_period;  // n / steps_per_period + 1, without the division
   for (int n = 0; n < N; ++n) {
-    if (MODE == 2) sde_tape_store<R, NF>(a.tape, n, S, voff, L);
+    if (MODE == 2 && (n & 1) == 0) sde_tape_store<R, NF>(a.tape, n >> 1, S, voff, L);
     if (MODE == 1 && (n % SEG) == 0 && live) {
       const long long slot = n / SEG;
 #pragma unroll
@@ -262,20 +249,20 @@ sdesim_lmm(const LmmArgs a) {
     }
     R eps[F];
     lmm_noise<R>(rsrc, sb, n, eps);
-    lmm_step<R>(lmm_par<R>(par_rows, n * a.zero), L, eps, n / a.steps_per_period + 1, dtu, sdtu, tau);
+    lmm_step<R>(lmm_rows<R>(a.rows), L, L, eps, eta, tau);
+    if (--left == 0) {
+      left = a.steps_per_period;
+      ++eta;
+    }
   }
   if (MODE == 2) {
-    sde_tape_store<R, NF>(a.tape, N, S, voff, L);
+    sde_tape_store<R, NF>(a.tape, (N + 1) >> 1, S, voff, L);
     return;
   }
 
-  R Lb[NF];
-  const R V = lmm_payoff<R, MODE == 1>(L, e, tau, K, Lb);
-  if (MODE == 1) {
-    // Lp holds the state after the step being reversed: L_N first, then each state read back.
-    R Lp[NF];
-#pragma unroll
-    for (int i = 0; i < NF; ++i) Lp[i] = L[i];
+  R M[NF];
+  const double V = lmm_payoff<R, MODE == 1>(a, L, M);
+  if constexpr (MODE == 1) {
     R* tape = (R*)a.tape;
     const int nseg = (N + SEG - 1) / SEG;
     for (int seg = nseg - 1; seg >= 0; --seg) {
@@ -292,73 +279,76 @@ sdesim_lmm(const LmmArgs a) {
         }
         R eps[F];
         lmm_noise<R>(rsrc, sb, n0 + k, eps);
-        lmm_step<R>(lmm_par<R>(par_rows, (n0 + k) * a.zero), Xc, eps, (n0 + k) / a.steps_per_period + 1, dtu, sdtu,
-                    tau);
+        lmm_step<R>(lmm_rows<R>(a.rows), Xc, Xc, eps, (n0 + k) / a.steps_per_period + 1, tau);
       }
       for (int k = len - 1; k >= 0; --k) {
         if (k + 1 < len) {
 #pragma unroll
           for (int i = 0; i < NF; ++i) Xc[i] = tape[((long long)k * NF + i) * S + sid];
         }
-        lmm_step_adjoint<R>(lmm_par<R>(par_rows, (n0 + k) * a.zero), Xc, Lp, Lb, (n0 + k) / a.steps_per_period + 1,
-                            dt, tau);
-#pragma unroll
-        for (int i = 0; i < NF; ++i) Lp[i] = Xc[i];
+        lmm_step_back<R>(lmm_rows<R>(a.rows_back), Xc, M, (n0 + k) / a.steps_per_period + 1, tau);
       }
     }
   }
   sde_reduce_store_chunked<NQ>(
       [&](int q) {
-        return !live ? 0.0 : q == 0 ? (double)V : q == 1 ? (double)V * (double)V : MODE == 1 ? (double)Lb[q - 2] : 0.0;
+        return !live ? 0.0 : q == 0 ? V : q == 1 ? V * V : MODE == 1 ? (double)(M[q - 2] / (R)a.L0[q - 2]) : 0.0;
       },
       a.partials + (long long)blockIdx.x * NQ);
 }
 
-// Reverse sweep of the tape form. L_N from the tape gives the payoff; then, for each step from
-// the last, the adjoint runs over the forwards from the last down, and as soon as forward i of
-// the state is used its register is refilled with forward i of the previous step's state (the
-// request after step 0 re-reads step 0 and is unused). The loads are issued in the order in
-// which the next step consumes them, so each has the rest of the step to arrive. The f32 kernel is
-// held to 3 waves per SIMD (168 VGPRs; it needs 169 unconstrained).
+// Reverse sweep of the tape form. L_N from the tape gives the payoff; then, two steps at a time from the
+// last, A = L_n (n even) gives L_{n+1} in B, whose step back frees B for the tape's previous state while A's
+// own step back runs (after step 0, step 0's again, unused). The next pair's normals are formed before that
+// request: loads return in order, so their table words, asked for afterwards, would wait for the whole
+// state. The f32 kernel is held to 3 waves per SIMD.
 template <typename R>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 3 : 1)))
 sdesim_lmm_reverse(const LmmArgs a) {
   constexpr int NQ = 2 + NF;
+  if constexpr (sizeof(R) == 8) sde_normal_tab_load<R>(a.normal_tab);
   const long long S = a.paths;
   const int N = a.steps;
   const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const bool live = s < S;
   const sde_u32 voff = live ? (sde_u32)(s * (long long)sizeof(R)) : 0x80000000u;
-  const R dt = (R)a.dt, tau = (R)a.tau, K = (R)a.strike;
+  const R tau = (R)a.tau;
 
-  __shared__ LmmParRow<R> par_rows[NF];
-  lmm_stage_params<R>(a, par_rows);
+  const LmmSobol sb = lmm_sobol(a, live ? s : 0);
+  const __amdgpu_buffer_rsrc_t rsrc = lmm_sobol_rsrc(a);
 
-  R L[NF], Lb[NF], Lp[NF];
-  sde_tape_load<R, NF>(a.tape, N, S, voff, Lp);
-  const R V = lmm_payoff<R, true>(Lp, a.expiry_index, tau, K, Lb);
-  sde_tape_load<R, NF>(a.tape, N - 1, S, voff, L);
-  for (int n = N - 1; n >= 0; --n) {
-    const LmmPar<R> tab = lmm_par<R>(par_rows, n * a.zero);
-    const int eta = n / a.steps_per_period + 1;
-    const __amdgpu_buffer_rsrc_t rs = sde_tape_rsrc<R, NF>(a.tape, n > 0 ? n - 1 : 0, S);
-    R G[F] = {R(0), R(0), R(0)};
-#pragma unroll
-    for (int i = NF - 1; i >= 0; --i) {
-      if (i >= eta) lmm_forward_adjoint<R>(tab.row(i), L[i], Lp[i], Lb[i], G, dt, tau);
-      Lp[i] = L[i];
-      L[i] = sde_tape_get<R>(rs, voff, i, S);
+  R A[NF], B[NF], M[NF];
+  sde_tape_load<R, NF>(a.tape, (N + 1) >> 1, S, voff, A);
+  const double V = lmm_payoff<R, true>(a, A, M);
+  int n = (N - 1) & ~1;
+  R eps[F];
+  lmm_noise<R>(rsrc, sb, n, eps);
+  sde_tape_load<R, NF>(a.tape, n >> 1, S, voff, A);
+  int eta = n / a.steps_per_period + 1, pos = n % a.steps_per_period;  // of step n; pos its place in its period
+  for (; n >= 0; n -= 2) {
+    if (n + 1 < N) {
+      lmm_step<R>(lmm_rows<R>(a.rows), A, B, eps, eta, tau);
+      lmm_step_back<R>(lmm_rows<R>(a.rows_back), B, M, eta + (pos + 1 == a.steps_per_period ? 1 : 0), tau);
     }
+    const int before = n > 0 ? n - 2 : 0;
+    lmm_noise<R>(rsrc, sb, before, eps);
+    sde_tape_load<R, NF>(a.tape, before >> 1, S, voff, B);
+    lmm_step_back<R>(lmm_rows<R>(a.rows_back), A, M, eta, tau);
+#pragma unroll
+    for (int i = 0; i < NF; ++i) A[i] = B[i];
+    for (pos -= 2; pos < 0; pos += a.steps_per_period) --eta;
   }
   sde_reduce_store_chunked<NQ>(
-      [&](int q) { return !live ? 0.0 : q == 0 ? (double)V : q == 1 ? (double)V * (double)V : (double)Lb[q - 2]; },
+      [&](int q) {
+        return !live ? 0.0 : q == 0 ? V : q == 1 ? V * V : (double)(M[q - 2] / (R)a.L0[q - 2]);
+      },
       a.partials + (long long)blockIdx.x * NQ);
 }
 
 }  // namespace
 
 // mode: 0 price, 1 adjoint with checkpoints and the segment tape, 2 adjoint with the state tape
-// (a.tape holds [steps + 1][40][paths]; a forward and a reverse kernel).
+// (a.tape holds [(steps + 1) / 2 + 1][40][paths]; a forward and a reverse kernel).
 hipError_t sdesim_launch_lmm(int f32, int mode, int grid, const LmmArgs& a, hipStream_t stream) {
 #define SDE_LMM(R, MODE)                                                                                  \
   hipLaunchKernelGGL((sdesim_lmm<R, MODE>), dim3(grid), dim3(256), 0, stream, a);                            \

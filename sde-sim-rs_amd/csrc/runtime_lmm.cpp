@@ -41,6 +41,24 @@ int guard(F&& f) {
     return sdesim_set_error(SDESIM_ERUNTIME, e.what());
   }
 }
+// The kernels' parameter rows (ts, b0..b2, q0..q2, h; lmm_kernels.hip says what they hold): the forward
+// step's, `unit` the unit of its exponent, then the step back's; a row of zeros after each.
+template <class R>
+const void* parameter_rows(std::vector<R>& out, const double* vol, const double* loadings, double dt, double tau,
+                           double unit) {
+  out.assign(2 * (kNF + 1) * 8, R(0));
+  for (int back = 0; back < 2; ++back)
+    for (int i = 0; i < kNF; ++i) {
+      R* r = &out[(size_t)(back * (kNF + 1) + i) * 8];
+      r[0] = (R)(tau * vol[i] * (back ? dt : std::sqrt(dt)));
+      for (int f = 0; f < kF; ++f) {
+        r[1 + f] = (R)loadings[i * kF + f];
+        r[4 + f] = (R)(vol[i] * loadings[i * kF + f] * (back ? 1.0 : std::sqrt(dt) * unit));
+      }
+      r[7] = back ? R(0) : (R)(-0.5 * vol[i] * vol[i] * dt * unit);
+    }
+  return out.data();
+}
 }  // namespace
 
 struct sdesim_lmm {
@@ -52,13 +70,12 @@ struct sdesim_lmm {
   int storage = SDESIM_STORAGE_CHECKPOINTS;  // resolved at creation: TAPE or CHECKPOINTS
   void* ckpt = nullptr;                      // checkpoints (CHECKPOINTS)
   void* tape = nullptr;                      // the segment tape (CHECKPOINTS) or the state tape (TAPE)
-  double* pard = nullptr;
-  float* parf = nullptr;
+  void* rows = nullptr;                      // parameter rows [2][41][8] (forward, back) in the path precision
   double* partials = nullptr;
   double* sums = nullptr;
   const void* normal_tab = nullptr;  // f64: the device's shared table of the inverse normal
   ~sdesim_lmm() {
-    for (void* p : {(void*)tab, (void*)tabup, ckpt, tape, (void*)pard, (void*)parf, (void*)partials, (void*)sums})
+    for (void* p : {(void*)tab, (void*)tabup, ckpt, tape, rows, (void*)partials, (void*)sums})
       if (p) (void)hipFree(p);
   }
 };
@@ -113,7 +130,7 @@ int sdesim_lmm_create(const sdesim_lmm_spec* spec, sdesim_lmm** out) {
     const size_t slots = (size_t)(s.steps + kSeg - 1) / kSeg;
     // One step of the state tape is 40 * paths * rb <= 1.34 GB (paths <= 2^22): one buffer
     // resource always covers it.
-    const size_t tape = (size_t)kNF * (size_t)s.paths * rb * ((size_t)s.steps + 1);  // L_0 .. L_N
+    const size_t tape = (size_t)kNF * (size_t)s.paths * rb * (((size_t)s.steps + 1) / 2 + 1);  // L_0, L_2, .. and L_N
     size_t free_b = 0, total_b = 0;
     lk(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
     if (s.storage == SDESIM_STORAGE_TAPE) {
@@ -128,8 +145,7 @@ int sdesim_lmm_create(const sdesim_lmm_spec* spec, sdesim_lmm** out) {
       lk(hipMalloc(&m->ckpt, slots * kNF * (size_t)s.paths * rb), "hipMalloc(checkpoints)");
       lk(hipMalloc(&m->tape, (size_t)kSeg * kNF * (size_t)s.paths * rb), "hipMalloc(segment tape)");
     }
-    lk(hipMalloc(&m->pard, sizeof(double) * kNF * (1 + kF)), "hipMalloc(parameters)");
-    lk(hipMalloc(&m->parf, sizeof(float) * kNF * (1 + kF)), "hipMalloc(parameters)");
+    lk(hipMalloc(&m->rows, rb * 2 * (kNF + 1) * 8), "hipMalloc(parameters)");
     if (s.precision != SDESIM_F32) lk(sdesim_normal_table(0, &m->normal_tab), "inverse normal table");
     lk(hipMalloc(&m->partials, sizeof(double) * kNQ * m->grid), "hipMalloc(partials)");
     lk(hipMalloc(&m->sums, sizeof(double) * kNQ), "hipMalloc(sums)");
@@ -150,26 +166,23 @@ int sdesim_lmm_eval(sdesim_lmm* m, const double* L0, const double* vol, const do
     const sdesim_lmm_spec& s = m->spec;
     LmmArgs a;
     std::memset(&a, 0, sizeof a);
-    std::vector<double> pd(kNF * (1 + kF));
-    std::vector<float> pf(kNF * (1 + kF));
-    for (int i = 0; i < kNF; ++i) {
-      a.L0[i] = L0[i];
-      pd[i] = vol[i];
-      for (int f = 0; f < kF; ++f) pd[kNF + i * kF + f] = loadings[i * kF + f];
-    }
-    for (size_t q = 0; q < pd.size(); ++q) pf[q] = (float)pd[q];
+    for (int i = 0; i < kNF; ++i) a.L0[i] = L0[i];
     hipStream_t st = (hipStream_t)stream;
-    // Ordered before the launch on the same stream; the host vectors outlive the synchronous
-    // wait at the end of this call.
-    lk(hipMemcpyAsync(m->pard, pd.data(), sizeof(double) * pd.size(), hipMemcpyHostToDevice, st), "hipMemcpyAsync");
-    lk(hipMemcpyAsync(m->parf, pf.data(), sizeof(float) * pf.size(), hipMemcpyHostToDevice, st), "hipMemcpyAsync");
-    a.pard = m->pard;
-    a.parf = m->parf;
     const double T = s.tenor * s.expiry_index;
     a.dt = T / s.steps;
     a.sdt = std::sqrt(a.dt);
     a.tau = s.tenor;
     a.strike = s.strike;
+    std::vector<double> rd;
+    std::vector<float> rf;
+    const void* rows = s.precision == SDESIM_F32 ? parameter_rows(rf, vol, loadings, a.dt, a.tau, std::log2(std::exp(1.0)))
+                                                 : parameter_rows(rd, vol, loadings, a.dt, a.tau, 1.0);
+    const size_t row_bytes = (s.precision == SDESIM_F32 ? sizeof(float) : sizeof(double)) * (kNF + 1) * 8;
+    // Ordered before the launch on the same stream; the host vector outlives the synchronous wait at
+    // the end of this call.
+    lk(hipMemcpyAsync(m->rows, rows, 2 * row_bytes, hipMemcpyHostToDevice, st), "hipMemcpyAsync");
+    a.rows = m->rows;
+    a.rows_back = (const char*)m->rows + row_bytes;
     a.paths = s.paths;
     a.sobol_tab = m->tab;
     a.sobol_tab_words = m->tab_words;
