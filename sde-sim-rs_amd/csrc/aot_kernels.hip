@@ -60,8 +60,11 @@ __global__ void __launch_bounds__(1024) sdesim_finalize(const double* __restrict
 // Among the layouts measured on 2050 x 2^20 values (64 x 128 up to 512 x 16 tiles, 8- or 16-byte
 // stores, default or non-temporal policy, scenario- or row-tile-fastest order, one tile per block
 // or a block walking all row tiles of its scenarios) this one moved the most bytes per second.
-// Tiles that are not whole (the last rows or scenarios), or data whose rows are not 16-byte aligned
-// (S not a multiple of the vector width, an odd row count), take element-wise guarded accesses.
+// An odd row count (whose output rows are not 16-byte aligned) has each lane store a row of its own, 512
+// adjacent bytes a wave: 3003 rows x 10,000 f64 took 132 us as pairs of 8-byte stores 16 bytes apart, 100 so
+// (4.8 TB/s); 1025 rows x 2^18 f32 1144 and 696.
+// The last scenarios' tile, and data whose rows are not 16-byte aligned (S not a multiple of the vector
+// width), take element-wise guarded loads.
 template <typename T>
 __global__ void __launch_bounds__(256) sdesim_to_long(const T* __restrict__ in, long long S, int rows, int ny,
                                                       double* __restrict__ out) {
@@ -73,7 +76,7 @@ __global__ void __launch_bounds__(256) sdesim_to_long(const T* __restrict__ in, 
   const long long b = blockIdx.x;
   const long long s0 = (b / ny) * W;
   const int r0 = (int)(b % ny) * RT;
-  const bool whole = r0 + RT <= rows && s0 + W <= S && S % VEC == 0;
+  const bool vector = s0 + W <= S && S % VEC == 0;
 #pragma unroll
   for (int pass = 0; pass < RT / 32; ++pass) {
     const int r = pass * 32 + (t >> 3);  // 32 rows per pass, 8 lanes per row
@@ -81,9 +84,10 @@ __global__ void __launch_bounds__(256) sdesim_to_long(const T* __restrict__ in, 
     const int row = r0 + r;
     const long long s = s0 + c;
     T v[VEC];
-    if (whole) {
+    if (vector) {
       typedef T TV __attribute__((ext_vector_type(VEC)));
-      const TV x = __builtin_nontemporal_load((const TV*)(in + (long long)row * S + s));
+      TV x = {};
+      if (row < rows) x = __builtin_nontemporal_load((const TV*)(in + (long long)row * S + s));
 #pragma unroll
       for (int e = 0; e < VEC; ++e) v[e] = x[e];
     } else {
@@ -96,20 +100,24 @@ __global__ void __launch_bounds__(256) sdesim_to_long(const T* __restrict__ in, 
   __syncthreads();
   typedef double D2 __attribute__((ext_vector_type(2)));
   const int wave = t >> 6, lane = t & 63;
-  const bool pairs = whole && rows % 2 == 0;
+  const bool pairs = rows % 2 == 0;
   for (int c = wave; c < W; c += 4) {
     const long long s = s0 + c;
+    if (s >= S) break;
+    if (pairs) {
 #pragma unroll
-    for (int k = 0; k < RT / 128; ++k) {
-      const int r = k * 128 + 2 * lane;
-      const int row = r0 + r;
-      if (pairs) {
-        const D2 v = {(double)tile[r][c], (double)tile[r + 1][c]};
-        __builtin_nontemporal_store(v, (D2*)(out + s * rows + row));
-      } else {
+      for (int k = 0; k < RT / 128; ++k) {
+        const int r = k * 128 + 2 * lane;
+        if (r0 + r < rows) {  // and r0 + r + 1 is too
+          const D2 v = {(double)tile[r][c], (double)tile[r + 1][c]};
+          __builtin_nontemporal_store(v, (D2*)(out + s * rows + r0 + r));
+        }
+      }
+    } else {
 #pragma unroll
-        for (int e = 0; e < 2; ++e)
-          if (row + e < rows && s < S) __builtin_nontemporal_store((double)tile[r + e][c], out + s * rows + row + e);
+      for (int k = 0; k < RT / 64; ++k) {
+        const int r = k * 64 + lane;
+        if (r0 + r < rows) __builtin_nontemporal_store((double)tile[r][c], out + s * rows + r0 + r);
       }
     }
   }
