@@ -23,13 +23,11 @@ namespace {
 
 // One Euler step of a built-in model. FP64 adds the terms to the state one at a time, in the
 // reference's order (src/sim/euler.rs:20-27: the drift term, then the Wiener term), which keeps it
-// bitwise equal to the DSL form's kernel. FP32 sums the step's terms first and adds the sum to the
-// state once, as the generated FP32 kernels do: added alone, a drift of a few ulps of x per step
-// (GBM with mu dt ~ 3e-7) is rounded to whole ulps at every step in the same direction, which
-// biased a 1000-step GBM mean by 1.5e-5.
-template <typename R, bool LIB>
-__device__ __forceinline__ R sde_euler_builtin(int kind, R x, R p0, R p1, R p2, R dt, R sdt, R z) {
-  R v0, v1;
+// bitwise equal to the DSL form's kernel.
+template <bool LIB>
+__device__ __forceinline__ double sde_euler_builtin(int kind, double x, double p0, double p1, double p2, double dt,
+                                                    double sdt, double z) {
+  double v0, v1;
   if (kind == 0) {
     v0 = p0 * x;
     v1 = p1 * x;
@@ -37,48 +35,83 @@ __device__ __forceinline__ R sde_euler_builtin(int kind, R x, R p0, R p1, R p2, 
     v0 = p0 * (p1 + (-x));
     v1 = p2;
   } else {
-    v0 = p0 * (p1 + (-sde_fmax(x, R(0))));
-    if constexpr (LIB) v1 = p2 * sqrt(sde_fmax(x, R(0)));
-    else v1 = p2 * sde_sqrt(sde_fmax(x, R(0)));
+    v0 = p0 * (p1 + (-sde_fmax(x, 0.0)));
+    if constexpr (LIB) v1 = p2 * sqrt(sde_fmax(x, 0.0));
+    else v1 = p2 * sde_sqrt(sde_fmax(x, 0.0));
   }
-  if constexpr (sizeof(R) == 4) {
-    return x + (v0 * dt + v1 * (sdt * z));
-  } else {
-    R a0 = x;
-    a0 = a0 + v0 * dt;
-    a0 = a0 + v1 * (sdt * z);
-    return a0;
-  }
+  double a0 = x;
+  a0 = a0 + v0 * dt;
+  a0 = a0 + v1 * (sdt * z);
+  return a0;
+}
+// FP32 sums the step's terms first and adds the sum to the state once, as the generated FP32 kernels do: added
+// alone, a drift of a few ulps of x per step (GBM with mu dt ~ 3e-7) is rounded to whole ulps at every step in
+// the same direction, which biased a 1000-step GBM mean by 1.5e-5. The products with dt and sqrt(dt) are
+// the host's (f64, rounded once): GBM a = mu dt, b = sigma sqrt(dt); OU and CIR a = kappa dt, b = sigma
+// sqrt(dt), and theta. 2, 4 and 8 operations instead of 6, 6 and 9.
+template <int KIND>
+__device__ __forceinline__ float sde_euler_builtin_f32(float x, float a, float b, float theta, float z) {
+  if (KIND == 0) return x + x * (a + b * z);
+  if (KIND == 1) return x + (a * (theta - x) + b * z);
+  const float xp = sde_fmax(x, 0.0f);
+  return x + (a * (theta - xp) + b * sde_sqrt(xp) * z);
 }
 
-// All steps of a wave's 64 * PPL paths.
-template <typename R, int PPL, bool LIB>
-__device__ __forceinline__ void batch_steps(const sde_u32 (&key)[PPL][8], int N, int kind, R (&x)[PPL], R p0, R p1, R p2,
-                                            R dt, R sdt) {
+// All steps of a wave's 64 * PPL paths in f64.
+template <int PPL, bool LIB>
+__device__ __forceinline__ void batch_steps(const sde_u32 (&key)[PPL][8], int N, int kind, double (&x)[PPL], double p0,
+                                            double p1, double p2, double dt, double sdt) {
   for (int n0 = 0; n0 < N; n0 += 8) {
-    sde_u32 lo[PPL][8], hi[PPL][8];
-    R z[PPL][8];
+    sde_u32 blk[PPL][16];
 #pragma unroll
-    for (int j = 0; j < PPL; ++j) {
-      sde_u32 blk[16];
-      sde_chacha_block<8>(key[j], (sde_u64)(n0 / 8), blk);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        lo[j][i] = blk[2 * i];
-        hi[j][i] = blk[2 * i + 1];
-      }
-      // f32: one test for rare draws per ChaCha block. f64 draws are taken one by one below (100
-      // registers; all eight at once take 138).
-      if constexpr (sizeof(R) == 4) sde_psi_words<8>(lo[j], hi[j], z[j]);
-    }
+    for (int j = 0; j < PPL; ++j) sde_chacha_block<8>(key[j], (sde_u64)(n0 / 8), blk[j]);
+    // The draws are taken one by one (100 registers; all eight at once take 138).
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       if (n0 + i < N) {
 #pragma unroll
         for (int j = 0; j < PPL; ++j) {
-          if constexpr (LIB) z[j][i] = sde_inv_normal(sde_u01_from_words(lo[j][i], hi[j][i]));
-          else if constexpr (sizeof(R) == 8) z[j][i] = sde_psi_word(lo[j][i], hi[j][i]);
-          x[j] = sde_euler_builtin<R, LIB>(kind, x[j], p0, p1, p2, dt, sdt, z[j][i]);
+          const sde_u32 lo = blk[j][2 * i], hi = blk[j][2 * i + 1];
+          double z;
+          if constexpr (LIB) z = sde_inv_normal(sde_u01_from_words(lo, hi));
+          else z = sde_psi_word(lo, hi);
+          x[j] = sde_euler_builtin<LIB>(kind, x[j], p0, p1, p2, dt, sdt, z);
+        }
+      }
+    }
+  }
+}
+
+// All steps of a wave's 64 * PPL paths in f32: a loop per model, and whole ChaCha blocks' eight steps without
+// a test between them.
+template <int KIND, int PPL>
+__device__ __forceinline__ void batch_steps_f32(const sde_u32 (&key)[PPL][8], int N, float (&x)[PPL], float a, float b,
+                                                float theta) {
+  for (int n0 = 0; n0 < N; n0 += 8) {
+    float z[PPL][8];
+#pragma unroll
+    for (int j = 0; j < PPL; ++j) {
+      sde_u32 blk[16], lo[8], hi[8];
+      sde_chacha_block<8>(key[j], (sde_u64)(n0 / 8), blk);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        lo[i] = blk[2 * i];
+        hi[i] = blk[2 * i + 1];
+      }
+      sde_psi_words<8>(lo, hi, z[j]);
+    }
+    if (n0 + 8 <= N) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int j = 0; j < PPL; ++j) x[j] = sde_euler_builtin_f32<KIND>(x[j], a, b, theta, z[j][i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 7; ++i) {
+        if (n0 + i < N) {
+#pragma unroll
+          for (int j = 0; j < PPL; ++j) x[j] = sde_euler_builtin_f32<KIND>(x[j], a, b, theta, z[j][i]);
         }
       }
     }
@@ -104,9 +137,6 @@ __global__ void __launch_bounds__(256) sdesim_batch(const SdeInstance* __restric
     if (k >= n_items) break;
     const SdeItem it = items[k];
     const SdeInstance I = inst[it.instance];
-    const R p0 = (R)I.p0, p1 = (R)I.p1, p2 = (R)I.p2;
-    const R dt = sizeof(R) == 4 ? (R)I.dtf : (R)I.dt;
-    const R sdt = sizeof(R) == 4 ? (R)I.sdtf : (R)I.sdt;
     const int N = I.steps;
     const int kind = I.kind;
     R x[PPL];
@@ -121,14 +151,16 @@ __global__ void __launch_bounds__(256) sdesim_batch(const SdeInstance* __restric
       x[j] = (R)I.x0;
       sde_seed_from_u64(I.seed + (sde_u64)sid[j], key[j]);
     }
-    // A CIR instance whose rounding differences grow (4 kappa theta < sigma^2: reaches_root in
-    // codegen.hpp) keeps the library's logarithm, root and division in f64.
-    bool lib = false;
-    if constexpr (sizeof(R) == 8) lib = kind == 2 && 4.0 * (I.p0 * I.p1) < I.p2 * I.p2;
-    if (lib) {
-      if constexpr (sizeof(R) == 8) batch_steps<R, PPL, true>(key, N, kind, x, p0, p1, p2, dt, sdt);
+    if constexpr (sizeof(R) == 4) {
+      if (kind == 0) batch_steps_f32<0, PPL>(key, N, x, I.af, I.bf, I.thetaf);
+      else if (kind == 1) batch_steps_f32<1, PPL>(key, N, x, I.af, I.bf, I.thetaf);
+      else batch_steps_f32<2, PPL>(key, N, x, I.af, I.bf, I.thetaf);
+    } else if (kind == 2 && 4.0 * (I.p0 * I.p1) < I.p2 * I.p2) {
+      // A CIR instance whose rounding differences grow (reaches_root in codegen.hpp) keeps the
+      // library's logarithm, root and division.
+      batch_steps<PPL, true>(key, N, kind, x, I.p0, I.p1, I.p2, I.dt, I.sdt);
     } else {
-      batch_steps<R, PPL, false>(key, N, kind, x, p0, p1, p2, dt, sdt);
+      batch_steps<PPL, false>(key, N, kind, x, I.p0, I.p1, I.p2, I.dt, I.sdt);
     }
     double acc[2] = {0.0, 0.0};
 #pragma unroll

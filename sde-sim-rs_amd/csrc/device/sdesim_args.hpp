@@ -55,7 +55,7 @@ struct SdeInstance {
   double p0, p1, p2;   // GBM: mu, sigma; OU / CIR: kappa, theta, sigma
   double x0;
   double dt, sdt;      // f64 grid
-  float dtf, sdtf;     // f32 grid
+  float af, bf, thetaf;  // f32 step constants: GBM mu dt, sigma sqrt(dt); OU / CIR kappa dt, sigma sqrt(dt), theta
   sde_u64 seed;        // path s uses seed + s
   long long paths;
   int kind;            // 0 GBM, 1 OU, 2 CIR

@@ -235,10 +235,10 @@ __device__ __forceinline__ float sde_inv_normal_f32_words(sde_u32 lo, sde_u32 hi
 // 15 octaves are 16 KB, so eight blocks of 256 still fit a CU; below 2^-15 (one draw in
 // 32768) the rational and its f64 tail take over. Error of z against the f64 formula: at most 4.8e-7
 // anywhere, rms 3.5e-8 relative to max(|z|, 0.05); the rational's 7.1e-7 and 1.5e-7.
-// 4096 batched instances take 66.0 instead of 76.1 ms, the price and Greeks of the 8-asset basket
-// (2^22 x 365) 26.6 instead of 28.8.
+// 4096 batched instances take 66.0 instead of 76.1 ms (62.9 with the step constants of batch_kernels.hip), the 8-asset basket with the
+// reverse sweep it then had 26.6 instead of 28.8.
 struct __attribute__((aligned(16))) SdePsi {
-  float c, a0, a1, a2;  // |z| = a0 + r (a1 + r a2), r = v - c, c the segment's middle
+  float c, a0, a1, a2;  // |z| = a0 + r (a1 + r a2), r = 2^31 v - c, c the segment's middle
 };
 __device__ __forceinline__ SdePsi* sde_psi_tab() {
   __shared__ SdePsi tab[1024];
@@ -250,28 +250,28 @@ __device__ __forceinline__ void sde_psi_tab_load(const void* __restrict__ src) {
   for (int i = threadIdx.x; i < 1024; i += blockDim.x) tab[i] = ((const SdePsi*)src)[i];
   __syncthreads();
 }
-// v is taken from the draw's words unfolded: as a signed integer, hi + lo 2^-32 is 2^32 u when bit 31
+// 2^31 v is taken from the draw's words unfolded: as a signed integer, hi + lo 2^-32 is 2^32 u when bit 31
 // of hi is clear and -2^32 (1 - u) when it is set (u here the 64-bit fraction, at most 2^-53 from
-// rand's). A segment's number is the low 4 exponent bits and the top 6 mantissa bits of v, so any v
+// rand's). A segment's number is the low 4 exponent bits and the top 6 mantissa bits, so any v
 // reads inside the table, but only |v| in [2^-15, 1] its own segment. One test covers the N
 // draws (a wave of 64 lanes enters the block once in 500 / N calls), so the gathers are issued
 // together and no branch lies between them.
 template <int N>
 __device__ __forceinline__ void sde_psi_words_mag(const sde_u32 (&lo)[N], const sde_u32 (&hi)[N], float (&x)[N]) {
-  float v[N], least = 1.0f;
+  float v[N], least = 0x1.0p31f;
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    v[k] = __builtin_fmaf((float)(int)hi[k], 0x1.0p-31f, (float)lo[k] * 0x1.0p-63f);
+    v[k] = __builtin_fmaf((float)lo[k], 0x1.0p-32f, (float)(int)hi[k]);
     const SdePsi e = sde_psi_tab()[(__builtin_bit_cast(sde_u32, v[k]) >> 17) & 1023u];
     const float r = __builtin_fabsf(v[k]) - e.c;
     x[k] = __builtin_fmaf(__builtin_fmaf(e.a2, r, e.a1), r, e.a0);
     least = __builtin_fminf(least, __builtin_fabsf(v[k]));
   }
-  if (least < 0x1.0p-15f) {
+  if (least < 0x1.0p16f) {
     asm volatile("");
 #pragma unroll
     for (int k = 0; k < N; ++k)
-      if (__builtin_fabsf(v[k]) < 0x1.0p-15f) x[k] = __builtin_fabsf(sde_inv_normal_f32_words(lo[k], hi[k]));
+      if (__builtin_fabsf(v[k]) < 0x1.0p16f) x[k] = __builtin_fabsf(sde_inv_normal_f32_words(lo[k], hi[k]));
   }
 }
 

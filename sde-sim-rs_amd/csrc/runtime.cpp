@@ -416,17 +416,19 @@ const float* tail_table() {
 // The tables behind the device's inverse normal (SdeLn, SdePsi in sdesim_device.hpp) on the current
 // device: 4 KB (f64) and 16 KB (f32), one copy of each per device, kept until exit.
 static std::vector<float> psi_table_f32() {
-  // Segment k: the low 4 bits of v's exponent (112 .. 127 biased) and the top 6 of its mantissa.
-  // The quadratic through the segment's Chebyshev points, its middle among them.
+  // Segment k of v = 2 min(u, 1 - u): octave 2^-15 .. 2^0 and the top 6 bits of the mantissa; the quadratic
+  // through its Chebyshev points, its middle among them. The kernels hold v 2^31, of which an entry's place is
+  // the low 4 bits of the exponent and those 6.
   std::vector<float> h(1024 * 4);
   for (int k = 0; k < 1024; ++k) {
     const double octave = std::ldexp(1.0, (112 + k / 64) - 127), width = octave / 64.0;
     const double c = octave + (k % 64 + 0.5) * width, s = std::sqrt(0.75) * 0.5 * width;
     const double f0 = inv_normal_mag(0.5 * c), fp = inv_normal_mag(0.5 * (c + s)), fm = inv_normal_mag(0.5 * (c - s));
-    h[4 * k] = (float)c;
-    h[4 * k + 1] = (float)f0;
-    h[4 * k + 2] = (float)((fp - fm) / (2.0 * s));
-    h[4 * k + 3] = (float)((fp + fm - 2.0 * f0) / (2.0 * s * s));
+    float* e = &h[4 * (((k / 64 + 112 + 31) % 16) * 64 + k % 64)];
+    e[0] = (float)std::ldexp(c, 31);
+    e[1] = (float)f0;
+    e[2] = (float)std::ldexp((fp - fm) / (2.0 * s), -31);
+    e[3] = (float)std::ldexp((fp + fm - 2.0 * f0) / (2.0 * s * s), -62);
   }
   return h;
 }

@@ -224,8 +224,9 @@ int sdesim_batch_create(const sdesim_instance* inst, int32_t n, int32_t precisio
       h.x0 = a.x0;
       h.dt = a.horizon / (double)a.steps;
       h.sdt = std::sqrt(h.dt);
-      h.dtf = (float)h.dt;
-      h.sdtf = (float)h.sdt;
+      h.af = (float)(a.p0 * h.dt);
+      h.bf = (float)((a.kind == 0 ? a.p1 : a.p2) * h.sdt);
+      h.thetaf = (float)a.p1;
       h.seed = a.seed;
       b->term_off[i + 1] = b->term_off[i] + a.paths;
       mix((unsigned long long)a.kind); mix((unsigned long long)a.steps); mix((unsigned long long)a.paths);
