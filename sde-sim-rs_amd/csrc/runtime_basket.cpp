@@ -13,7 +13,7 @@
 #include "../../include/sdesim.h"
 #include "device/sdesim_args.hpp"
 
-hipError_t sdesim_launch_basket(int f32, int assets, int adjoint, int grid, const BasketArgs& a, int nq,
+hipError_t sdesim_launch_basket(int f32, int assets, int adjoint, int team, int grid, const BasketArgs& a, int nq,
                                 double* sums, hipStream_t stream);
 hipError_t sdesim_normal_table(int f32, const void** out);
 int sdesim_set_error(int code, const std::string& msg);
@@ -44,6 +44,7 @@ struct sdesim_basket {
   sdesim_basket_spec spec{};
   int nq = 0;         // reduced quantities of the adjoint
   long long grid = 0;
+  bool team = false;  // blocks of four waves to 64 paths (few paths), else a path per lane
   int storage = SDESIM_STORAGE_CHECKPOINTS;  // as asked for, or AUTO's choice; neither keeps states
   double* partials = nullptr;
   double* sums = nullptr;
@@ -69,7 +70,14 @@ int sdesim_basket_create(const sdesim_basket_spec* spec, sdesim_basket** out) {
       throw BFail{SDESIM_EVALUE, "storage must be SDESIM_STORAGE_AUTO, _TAPE or _CHECKPOINTS"};
     std::unique_ptr<sdesim_basket> b(new sdesim_basket());
     b->spec = s;
-    b->grid = (s.paths + 255) / 256;
+    // Teams up to two blocks per CU (32,768 paths): 0.225 instead of 0.30 ms for a call there (8 assets with Greeks,
+    // f64, 100 steps); at twice as many paths they gain nothing (0.32 against 0.29).
+    int dev = 0, cus = 0;
+    bk(hipGetDevice(&dev), "hipGetDevice");
+    bk(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
+    const long long waves = (s.paths + 63) / 64;
+    b->team = waves <= 2LL * cus;
+    b->grid = b->team ? waves : (s.paths + 255) / 256;
     if (b->grid > 0x7fffffffLL) throw BFail{SDESIM_EVALUE, "too many paths"};
     // The derivatives are summed on the way forward: no state is stored under either name. What a tape
     // was refused for, a step of it (at 1 or 8 assets) of 2^31 bytes or more, still is.
@@ -123,7 +131,7 @@ int sdesim_basket_eval(sdesim_basket* b, const double* x0, const double* mu, con
     a.normal_tab = b->normal_tab;
     hipStream_t st = (hipStream_t)stream;
     const int nq = adjoint ? b->nq : 2;
-    bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, adjoint != 0, (int)b->grid, a, nq, b->sums, st),
+    bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, adjoint != 0, b->team, (int)b->grid, a, nq, b->sums, st),
        "basket launch");
     std::vector<double> sums(nq);
     bk(hipMemcpyAsync(sums.data(), b->sums, sizeof(double) * nq, hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
