@@ -18,7 +18,7 @@
 //   Lbar_ik = M_i sigma_i sqrt(dt) H_ik,  H_ik = sum_n eps_{n,k} / g_{n,i}  (k <= i),
 //   sigmabar_i = M_i sqrt(dt) sum_{k <= i} L_ik H_ik.
 // No state is kept. The reverse sweep that this replaces wrote and read every state (49 GB for 8 assets x
-// 365 steps x 2^22 paths in f32): 26.1 ms for price and Greeks, 18.0 ms now, bound by VALU issue: a step's 8
+// 365 steps x 2^22 paths in f32): 26.1 ms for price and Greeks, 17.6 ms now, bound by VALU issue: a step's 8
 // draws are two thirds of it (350 instructions of ChaCha8, 80 of the normals), the 36 sums, 8
 // reciprocals and the step the rest.
 #include <hip/hip_runtime.h>
@@ -175,9 +175,11 @@ struct BasketPath {
   }
 };
 
-// One path per lane.
+// One path per lane. f32 is held to 4 waves per SIMD (128 VGPRs; 8 assets with Greeks take 139 unconstrained and
+// 17.95 instead of 17.63 ms).
 template <typename R, int D, bool ADJ>
-__global__ void __launch_bounds__(256) sdesim_basket(const BasketArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
+sdesim_basket(const BasketArgs a) {
   constexpr int U = SdeChunk<D>::U;  // steps in a whole number of ChaCha blocks
   sde_normal_tab_load<R>(a.normal_tab);
   const int N = a.steps;

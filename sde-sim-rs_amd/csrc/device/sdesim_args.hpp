@@ -94,7 +94,7 @@ struct LmmArgs {
   double L0[40];                      // initial forwards
   const void* rows;                   // device [41][8] real, the forward step's parameter rows and a row of zeros
   const void* rows_back;              // the step back's
-  double dt, sdt, tau, strike;
+  double tau, strike;
   long long paths;
   const sde_u32* sobol_tab;           // slice 0 as [steps][64][3], the mask complements folded in
   const sde_u32* sobol_up;            // slices 1-2 as [2][256][steps * 3]

@@ -235,8 +235,8 @@ __device__ __forceinline__ float sde_inv_normal_f32_words(sde_u32 lo, sde_u32 hi
 // 15 octaves are 16 KB, so eight blocks of 256 still fit a CU; below 2^-15 (one draw in
 // 32768) the rational and its f64 tail take over. Error of z against the f64 formula: at most 4.8e-7
 // anywhere, rms 3.5e-8 relative to max(|z|, 0.05); the rational's 7.1e-7 and 1.5e-7.
-// 4096 batched instances take 66.0 instead of 76.1 ms (62.9 with the step constants of batch_kernels.hip), the 8-asset basket with the
-// reverse sweep it then had 26.6 instead of 28.8.
+// 4096 batched instances take 66.0 instead of 76.1 ms (62.9 with the step constants of
+// batch_kernels.hip), the 8-asset basket with the reverse sweep it then had 26.6 instead of 28.8.
 struct __attribute__((aligned(16))) SdePsi {
   float c, a0, a1, a2;  // |z| = a0 + r (a1 + r a2), r = 2^31 v - c, c the segment's middle
 };
@@ -944,7 +944,8 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
 // a fifth of the stepping wave's time. Each value is computed by the operations of sde_path_kernel (in what
 // pairs products and sums are fused can differ, so a last bit can).
 // What bounds it now is the stepping wave's chain. GBM, 10,000 x 252 pseudo-random: 31 us instead of 80; the
-// jump diffusion, 10,000 x 1000: 295 instead of 588 (193 with its jumps' short cut); Heston RK, 65,537 x 365, random shift: 302 instead of 388.
+// jump diffusion, 10,000 x 1000: 295 instead of 588 (193 with its jumps' short cut); Heston RK, 65,537 x
+// 365, random shift: 302 instead of 388.
 // FP64 only: the FP32 step may be reassociated, and how depends on the code around it.
 //
 // A step's noise as the stepping wave reads it: Psi(u) of a Wiener increment, u of a jump, and (RK) whether

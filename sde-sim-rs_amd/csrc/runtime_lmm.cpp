@@ -169,14 +169,13 @@ int sdesim_lmm_eval(sdesim_lmm* m, const double* L0, const double* vol, const do
     for (int i = 0; i < kNF; ++i) a.L0[i] = L0[i];
     hipStream_t st = (hipStream_t)stream;
     const double T = s.tenor * s.expiry_index;
-    a.dt = T / s.steps;
-    a.sdt = std::sqrt(a.dt);
+    const double dt = T / s.steps;
     a.tau = s.tenor;
     a.strike = s.strike;
     std::vector<double> rd;
     std::vector<float> rf;
-    const void* rows = s.precision == SDESIM_F32 ? parameter_rows(rf, vol, loadings, a.dt, a.tau, std::log2(std::exp(1.0)))
-                                                 : parameter_rows(rd, vol, loadings, a.dt, a.tau, 1.0);
+    const void* rows = s.precision == SDESIM_F32 ? parameter_rows(rf, vol, loadings, dt, a.tau, std::log2(std::exp(1.0)))
+                                                 : parameter_rows(rd, vol, loadings, dt, a.tau, 1.0);
     const size_t row_bytes = (s.precision == SDESIM_F32 ? sizeof(float) : sizeof(double)) * (kNF + 1) * 8;
     // Ordered before the launch on the same stream; the host vector outlives the synchronous wait at
     // the end of this call.

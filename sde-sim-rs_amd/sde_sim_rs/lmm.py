@@ -35,10 +35,10 @@ class ForwardRateModel:
     """Receiver swaption on the swap [T_e, T_40] (e = expiry_index), fixed rate `strike`,
     priced under the spot measure with `steps` log-Euler steps to T_e.
 
-    `storage` picks how the adjoint keeps the forward states: "tape" (all steps + 1 states of the
-    40 forwards in device memory), "checkpoints" (every 16th state, each segment recomputed once
-    during the reverse sweep) or "auto" (the tape when it fits in half of the free device
-    memory). `self.storage` is the form in use."""
+    `storage` picks how the adjoint keeps the forward states: "tape" (every second state of the
+    40 forwards in device memory, the others recomputed during the reverse sweep), "checkpoints"
+    (every 16th state, each segment recomputed once during the reverse sweep) or "auto" (the tape
+    when it fits in half of the free device memory). `self.storage` is the form in use."""
 
     def __init__(self, steps=160, paths=1 << 20, expiry_index=4, strike=0.03, tenor=0.25, scramble_seed=5,
                  precision="f32", storage="auto"):
