@@ -175,8 +175,8 @@ struct BasketPath {
   }
 };
 
-// One path per lane. f32 is held to 4 waves per SIMD (128 VGPRs; 8 assets with Greeks take 139 unconstrained and
-// 17.95 instead of 17.63 ms).
+// One path per lane. f32 is held to 4 waves per SIMD (128 VGPRs): 8 assets with Greeks take 139 unconstrained;
+// with 11 values spilled (a load or store of each a step) they take 17.63 instead of 17.95 ms.
 template <typename R, int D, bool ADJ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
 sdesim_basket(const BasketArgs a) {
