@@ -4,6 +4,7 @@
 // Cholesky factors are written into the coefficients.
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -13,8 +14,8 @@
 #include "../../include/sdesim.h"
 #include "device/sdesim_args.hpp"
 
-hipError_t sdesim_launch_basket(int f32, int assets, int adjoint, int team, int grid, const BasketArgs& a, int nq,
-                                double* sums, hipStream_t stream);
+hipError_t sdesim_launch_basket(int f32, int assets, int adjoint, int team, int again, int grid, const BasketArgs& a,
+                                int nq, double* sums, hipStream_t stream);
 hipError_t sdesim_normal_table(int f32, const void** out);
 int sdesim_set_error(int code, const std::string& msg);
 void sdesim_log(const char* fmt, ...);
@@ -131,11 +132,17 @@ int sdesim_basket_eval(sdesim_basket* b, const double* x0, const double* mu, con
     a.normal_tab = b->normal_tab;
     hipStream_t st = (hipStream_t)stream;
     const int nq = adjoint ? b->nq : 2;
-    bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, adjoint != 0, b->team, (int)b->grid, a, nq, b->sums, st),
-       "basket launch");
     std::vector<double> sums(nq);
-    bk(hipMemcpyAsync(sums.data(), b->sums, sizeof(double) * nq, hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
-    bk(hipStreamSynchronize(st), "hipStreamSynchronize");
+    auto run = [&](int again) {
+      bk(sdesim_launch_basket(s.precision == SDESIM_F32 ? 1 : 0, A, adjoint != 0, b->team, again, (int)b->grid, a, nq,
+                              b->sums, st),
+         "basket launch");
+      bk(hipMemcpyAsync(sums.data(), b->sums, sizeof(double) * nq, hipMemcpyDeviceToHost, st), "hipMemcpyAsync");
+      bk(hipStreamSynchronize(st), "hipStreamSynchronize");
+    };
+    run(0);
+    // Derivatives that are not finite: a path with a growth factor of 0 (or inputs that give no others).
+    if (adjoint && !std::all_of(sums.begin() + 2, sums.end(), [](double v) { return std::isfinite(v); })) run(1);
     const double n = (double)s.paths;
     const double m1 = sums[0] / n;
     out[0] = m1;
