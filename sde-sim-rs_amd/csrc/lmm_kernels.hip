@@ -196,6 +196,14 @@ __device__ __forceinline__ double lmm_payoff(const LmmArgs& a, const R (&L)[NF],
   return V;
 }
 
+// dV/dL_i of the initial curve from M_i, the derivative with respect to ln L_i. Forward 0 is dead at every step: its
+// derivative is the numeraire factor's, which a forward of 0 has too.
+template <typename R>
+__device__ __forceinline__ double lmm_dL0(const LmmArgs& a, const R (&M)[NF], double V, int i) {
+  if (i == 0) return -V * (a.tau * sde_recip(1.0 + a.tau * (double)(R)a.L0[0]));
+  return (double)(M[i] / (R)a.L0[i]);
+}
+
 // The lane's Sobol entry and the wave's rows. Point index = path index; blocks of 256 make every wave one
 // aligned run of 64 indices. Lane 0 has the wave's smallest index: if it is past the last path so is every
 // lane of the wave, whose values are then never used.
@@ -292,7 +300,7 @@ sdesim_lmm(const LmmArgs a) {
   }
   sde_reduce_store_chunked<NQ>(
       [&](int q) {
-        return !live ? 0.0 : q == 0 ? V : q == 1 ? V * V : MODE == 1 ? (double)(M[q - 2] / (R)a.L0[q - 2]) : 0.0;
+        return !live ? 0.0 : q == 0 ? V : q == 1 ? V * V : MODE == 1 ? lmm_dL0<R>(a, M, V, q - 2) : 0.0;
       },
       a.partials + (long long)blockIdx.x * NQ);
 }
@@ -340,7 +348,7 @@ sdesim_lmm_reverse(const LmmArgs a) {
   }
   sde_reduce_store_chunked<NQ>(
       [&](int q) {
-        return !live ? 0.0 : q == 0 ? V : q == 1 ? V * V : (double)(M[q - 2] / (R)a.L0[q - 2]);
+        return !live ? 0.0 : q == 0 ? V : q == 1 ? V * V : lmm_dL0<R>(a, M, V, q - 2);
       },
       a.partials + (long long)blockIdx.x * NQ);
 }
