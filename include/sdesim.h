@@ -144,7 +144,7 @@ const char* sdesim_plan_source(const sdesim_plan* plan);
  * no kernel. No reference counterpart. */
 uint64_t sdesim_plan_code_hash(const sdesim_plan* plan);
 
-/* Host-only helpers (no device needed): the kernel source a plan would generate for a time grid
+/* Host-only helpers (no device needed): the kernel source a plan of many paths would generate for a time grid
  * of n_times points, and a gfx950 compile of a source through hipRTC. `needed` receives the
  * buffer size including the terminating NUL. */
 int sdesim_generate_source(const sdesim_universe* u, int32_t n_times, const sdesim_options* opt, const char* payoff,

@@ -26,6 +26,8 @@
 //     terms r * ((sum_k c_k) * sk * sqrt(dt));
 //   * an increment whose every use is such a group member with one constant c > 0 is formed as
 //     sqrt(dt) * c * Psi(u) directly (the multiplier takes its sign from u, so c must be > 0).
+#include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <map>
 #include <set>
@@ -537,36 +539,111 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
   return s.str();
 }
 
-bool reaches_root(const Universe& u, const std::vector<double>& x0, double t0) {
-  std::map<std::string, double> ns;
-  for (const auto& kv : u.registry) ns[kv.first] = kv.second < (int)x0.size() ? x0[kv.second] : 0.0;
-  ns.emplace("t", t0);
-  // Sum of process p's terms of one kind at the point (squared for noise).
-  auto sum = [&](const ProcessDef& pd, IncKind kind, double x) {
-    ns[pd.name] = x;
-    double v = 0.0;
-    for (const Term& t : pd.terms) {
-      if (t.kind != kind) continue;
-      const double c = eval_host(*t.coef, ns);
-      v += kind == IncKind::Time ? c : c * c;
-    }
-    return v;
-  };
-  for (const ProcessDef& pd : u.processes) {
-    if (!pd.levy) continue;
-    const double own = ns[pd.name];
-    try {
-      const double at0 = sum(pd, IncKind::Wiener, 0.0);
-      const double s2 = sum(pd, IncKind::Wiener, 0x1.0p-40) * 0x1.0p40;
-      const double closer = sum(pd, IncKind::Wiener, 0x1.0p-42) * 0x1.0p42;
-      if (at0 == 0.0 && s2 > 0.0 && closer >= 0.99 * s2 && 4.0 * sum(pd, IncKind::Time, 0.0) < s2) return true;
-    } catch (const std::exception&) {
-      // A coefficient that does not evaluate fails where the kernel is generated.
-    }
-    ns[pd.name] = own;
+namespace {
+
+// The roots among the noise coefficients of a universe: powers below 1 and other functions whose slope is
+// unbounded at a finite argument, of an argument that depends on a Levy process, directly or through
+// algebraic processes.
+class NoiseRoots {
+ public:
+  explicit NoiseRoots(const Universe& u) : u_(u) {}
+
+  // Whether any of them may let rounding differences grow.
+  bool any() {
+    for (const ProcessDef& pd : u_.processes)
+      for (const Term& t : pd.terms)
+        if (t.kind != IncKind::Time && unsafe(*t.coef)) return true;
+    return false;
   }
-  return false;
-}
+
+ private:
+  const Universe& u_;
+  std::set<int> open_;  // algebraic processes being followed
+
+  const ProcessDef* process(const Expr& e) const {
+    if (e.op != Op::Var && !(e.op == Op::Call && e.fn == Fn::Lookup)) return nullptr;
+    auto it = u_.registry.find(e.name);
+    return it == u_.registry.end() ? nullptr : &u_.processes[it->second];
+  }
+
+  // f(expression) of the algebraic process pd, false where that is being followed already.
+  template <class F>
+  bool follow(const ProcessDef& pd, const F& f) {
+    const int k = (int)(&pd - u_.processes.data());
+    if (!open_.insert(k).second) return false;
+    const bool r = f(*pd.expr);
+    open_.erase(k);
+    return r;
+  }
+
+  bool random(const Expr& e) {
+    if (const ProcessDef* pd = process(e))
+      return pd->levy || follow(*pd, [&](const Expr& x) { return random(x); });
+    if (e.op == Op::Call && e.fn == Fn::Lookup) return false;
+    for (const ExprPtr& a : e.args)
+      if (random(*a)) return true;
+    return false;
+  }
+
+  bool unsafe(const Expr& e) {
+    if (const ProcessDef* pd = process(e))
+      return !pd->levy && follow(*pd, [&](const Expr& x) { return unsafe(x); });
+    if (e.op == Op::Call && e.fn == Fn::Lookup) return false;
+    if (e.op == Op::Pow) {
+      const Expr& p = *e.args[1];
+      // A whole power (quotients and negative ones among them, where the noise itself is unbounded and carries
+      // the path away) and one above 1 are no roots.
+      const bool whole = p.op == Op::Const && (p.value >= 1.0 || p.value == std::floor(p.value));
+      if (!whole && random(*e.args[0]) && !(p.op == Op::Const && p.value == 0.5 && steadied(*e.args[0]))) return true;
+    }
+    if (e.op == Op::Call && (e.fn == Fn::Log || e.fn == Fn::Asin || e.fn == Fn::Acos || e.fn == Fn::Acosh || e.fn == Fn::Atanh))
+      for (const ExprPtr& a : e.args)
+        if (random(*a)) return true;
+    for (const ExprPtr& a : e.args)
+      if (unsafe(*a)) return true;
+    return false;
+  }
+
+  // Whether the root's argument is a process x or max(x, 0) whose own drift a and noise b near 0, functions of x
+  // alone, have b^2 / x -> s^2 and 4 a >= s^2.
+  bool steadied(const Expr& arg) {
+    const Expr* v = &arg;
+    if (arg.op == Op::Call && arg.fn == Fn::Max && arg.args.size() == 2)
+      for (int k = 0; k < 2; ++k)
+        if (arg.args[1 - k]->op == Op::Const && arg.args[1 - k]->value == 0.0) v = arg.args[k].get();
+    const ProcessDef* pd = v->op == Op::Var ? process(*v) : nullptr;
+    if (!pd || !pd->levy) return false;
+    for (const ProcessDef& other : u_.processes)
+      if (&other != pd && other.name == pd->name) return false;
+    for (const Term& t : pd->terms) {
+      std::vector<std::string> names;
+      collect_names(*t.coef, names);
+      if (t.kind == IncKind::Jump || !std::all_of(names.begin(), names.end(), [&](const std::string& n) { return n == pd->name; }))
+        return false;
+    }
+    // Sum of the process's coefficients of one kind at x (squared for noise).
+    auto sum = [&](IncKind kind, double x) {
+      double r = 0.0;
+      for (const Term& t : pd->terms) {
+        if (t.kind != kind) continue;
+        const double c = eval_host(*t.coef, {{pd->name, x}});
+        r += kind == IncKind::Time ? c : c * c;
+      }
+      return r;
+    };
+    try {
+      const double s2 = sum(IncKind::Wiener, 0x1.0p-40) * 0x1.0p40, closer = sum(IncKind::Wiener, 0x1.0p-42) * 0x1.0p42;
+      return sum(IncKind::Wiener, 0.0) == 0.0 && s2 > 0.0 && closer >= 0.99 * s2 && closer <= 1.01 * s2 &&
+             4.0 * sum(IncKind::Time, 0.0) >= s2;
+    } catch (const std::exception&) {
+      return false;  // a coefficient that does not evaluate fails where the kernel is generated
+    }
+  }
+};
+
+}  // namespace
+
+bool reaches_root(const Universe& u) { return NoiseRoots(u).any(); }
 
 std::string kernel_name(const CodegenOptions& o) {
   static const char* rng[] = {"pseudo", "sobolshift", "sobolxor", "injected", "none"};

@@ -42,15 +42,17 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o);
 // Descriptive entry point name: sdesim_<em|rk>_<f32|f64>_<rng>_<filt|term|filt_term>.
 std::string kernel_name(const CodegenOptions& o);
 
-// Whether a process of the universe has noise that vanishes at 0 like a root and a drift there too weak
-// to keep rounding differences from growing: with b(x)^2 / x -> s^2 and drift a as x -> 0 (the
-// other processes at x0, time t0), 4 a < s^2. An Euler path that steps out of 0 lands at about
-// a dt, where its next increment changes by s sqrt(dt) / (2 sqrt(a dt)) = s / (2 sqrt(a)) of any
-// difference: above 1, two copies of a path that differ in one last bit drift apart without bound
-// (CIR with 2 a / s^2 = 0.09: 0.1 apart after 1550 steps), below 1 they come together (Heston's
-// variance at 0.64: 1e-15 after 1024). The f64 kernels of such universes, and the batch kernel's
-// CIR instances, keep the library's logarithm, root and division, so that their paths stay bit for bit
+// Whether the noise of the universe holds a root that may let rounding differences grow. With noise s sqrt(x)
+// and drift a at x = 0, an Euler path that steps out of 0 lands at about a dt, where its next increment changes
+// by s sqrt(dt) / (2 sqrt(a dt)) = s / (2 sqrt(a)) of any difference: above 1, two copies of a path that
+// differ in one last bit drift apart without bound (CIR with 4 a / s^2 = 0.18: 0.1 apart after 1550 steps),
+// below 1 they come together (Heston's variance at 1.28: 1e-15 after 1024). Any other root has such a place too,
+// wherever its argument vanishes (0.8 sqrt(x (1 - x)) at 1 with a drift of 0.015 to it: 0.67 after 1550). So the
+// only roots of a Levy process in a noise coefficient that are taken to be harmless are those of a process x, or
+// max(x, 0), whose own drift and noise depend on x alone and have 4 a >= s^2 at 0; every other power below 1,
+// logarithm or inverse function counts. The f64 kernels of such universes, and the batch kernel's CIR
+// instances with 4 a < s^2, keep the library's logarithm, root and division, so that their paths stay bit for bit
 // those of the general inverse normal.
-bool reaches_root(const Universe& u, const std::vector<double>& x0, double t0);
+bool reaches_root(const Universe& u);
 
 }  // namespace sdesim

@@ -656,7 +656,7 @@ int sdesim_plan_create(const sdesim_universe* uh, const double* times, int32_t T
     std::vector<double> x0v(x0 ? x0 : nullptr, x0 ? x0 + P : nullptr);
     if (!x0) x0v.assign(P, 0.0);
     if (x0v.empty()) x0v.push_back(0.0);
-    co.library_f64 = !co.f32 && sdesim::reaches_root(U, x0v, tv[0]);
+    co.library_f64 = !co.f32 && sdesim::reaches_root(U);
     if (opt.block_size <= 0 && opt.paths_per_lane <= 0) co.team = team_waves(co, S, N, M, plan->KQ);
     if (co.team > 1) co.block = plan->block = 64 * co.team;
     co.name = sdesim::kernel_name(co);
@@ -910,6 +910,7 @@ int sdesim_generate_source(const sdesim_universe* u, int32_t n_times, const sdes
     co.uniform_grid = true;
     const long long first = opt.sobol_first >= 0 ? opt.sobol_first : (co.rng == SDE_RNG_SOBOL_XOR ? 0 : 5);
     co.wave_aligned = co.rng == SDE_RNG_SOBOL_XOR && first % 64 == 0 && co.block % 64 == 0;
+    co.library_f64 = !co.f32 && sdesim::reaches_root(u->u);
     co.name = sdesim::kernel_name(co);
     co.steps = n_times > 1;
     co.payoff = payoff ? payoff : "";
