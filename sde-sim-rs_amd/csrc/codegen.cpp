@@ -404,7 +404,15 @@ class StepEmitter {
     for (int p = 0; p < P; ++p) {
       const ProcessDef& pd = u_.processes[p];
       if (!pd.levy) continue;
+      int wiener = 0;
+      for (const Term& t : pd.terms) wiener += t.kind == IncKind::Wiener;
       std::string pe = "pe" + std::to_string(p);
+      if (!o_.f32 && wiener == 1) {  // in y's own statement, for its FMA
+        for (const Term& t : pd.terms)
+          if (t.kind == IncKind::Wiener) pe = eval(*t.coef, false) + " * sks";
+        line(y(p) + " = X[" + std::to_string(p) + "] + k1_" + std::to_string(p) + " + " + pe + ";");
+        continue;
+      }
       line(R_ + " " + pe + " = " + R_ + "(0);");
       bool first = true;
       std::set<int> done;
@@ -503,8 +511,13 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
     for (int k : jumps) s << " || k == " << k;
     s << ";\n  }\n";
   }
+  // FP64 kernels fuse a product into a sum of the same statement only, which is settled by the source: fused
+  // across statements as well, which product of two it is depends on what the kernel around the step makes of
+  // them, and the last bit of a path on the kernel (path or team) that the path count picks. Not where
+  // paths are to stay those of the library form, which was always compiled with free fusing.
+  const char* const fuse = o.f32 || o.library_f64 ? "" : SDE_FUSE_IN_STATEMENTS "\n";
   s << "  __device__ static __forceinline__ void prologue(real (&X)[P], real (&C)[P], real (&K)[NK], real tc) {\n";
-  s << pro;
+  s << fuse << pro;
   s << "  }\n";
   s << "  template <class UT>\n";
   s << "  __device__ static __forceinline__ void step(real (&X)[P], real (&C)[P], real (&K)[NK], real tc, real tn,\n";
@@ -512,9 +525,10 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
   // FP32 kernels let the compiler reassociate the step's arithmetic (for example 2 * (a - v)
   // into one FMA); FP64 kernels keep the reference's evaluation order.
   if (o.f32) s << "#pragma clang fp reassociate(on)\n";
+  s << fuse;
   s << body << tail.str();
   s << "  }\n";
-  s << "  __device__ static __forceinline__ real payoff(const real (&X)[P], real tt) {\n";
+  s << "  __device__ static __forceinline__ real payoff(const real (&X)[P], real tt) {\n" << fuse;
   if (!o.payoff.empty()) {
     ExprPtr pe = parse_expression(o.payoff);
     EmitEnv env;

@@ -5,6 +5,10 @@
 
 #include "universe.hpp"
 
+// In a generated function body: products are fused into sums of their own statement only. Sources that have it are
+// compiled with the option under which clang honours it.
+#define SDE_FUSE_IN_STATEMENTS "#pragma clang fp contract(on)"
+
 namespace sdesim {
 
 struct CodegenOptions {

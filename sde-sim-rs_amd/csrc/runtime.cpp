@@ -104,8 +104,11 @@ struct CompiledKernel {
 std::mutex g_cache_mu;
 std::map<std::pair<int, std::string>, CompiledKernel> g_kernels;
 
-const char* const kRtcOptions[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast",
-                                   "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
+std::vector<const char*> rtc_options(const std::string& src) {
+  return {"--offload-arch=gfx950", "-O3", "-std=c++17",
+          src.find(SDE_FUSE_IN_STATEMENTS) == std::string::npos ? "-ffp-contract=fast" : "-ffp-contract=fast-honor-pragmas",
+          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
+}
 
 // The device header the run-time kernels compile against: the copy embedded at build time.
 const std::string& device_header_text() {
@@ -120,7 +123,8 @@ std::vector<char> rtc_compile(const std::string& src) {
   const char* names[] = {"sdesim_device.hpp", "sdesim_args.hpp"};
   if (hiprtcCreateProgram(&prog, src.c_str(), "sdesim_kernel.hip", 2, hdrs, names) != HIPRTC_SUCCESS)
     fail(SDESIM_ERUNTIME, "hiprtcCreateProgram failed");
-  hiprtcResult r = hiprtcCompileProgram(prog, (int)(sizeof(kRtcOptions) / sizeof(kRtcOptions[0])), kRtcOptions);
+  std::vector<const char*> options = rtc_options(src);
+  hiprtcResult r = hiprtcCompileProgram(prog, (int)options.size(), options.data());
   if (r != HIPRTC_SUCCESS) {
     size_t n = 0;
     hiprtcGetProgramLogSize(prog, &n);
@@ -162,7 +166,7 @@ uint64_t code_key(const std::string& src) {
   const std::string& hdr = device_header_text();
   h = fnv1a(hdr.data(), hdr.size(), h);
   h = fnv1a(sdesim_embedded_args_header, std::strlen(sdesim_embedded_args_header), h);
-  for (const char* o : kRtcOptions) h = fnv1a(o, std::strlen(o) + 1, h);
+  for (const char* o : rtc_options(src)) h = fnv1a(o, std::strlen(o) + 1, h);
   const int ver[2] = {major, minor};
   return fnv1a(ver, sizeof ver, h);
 }
