@@ -216,7 +216,7 @@ __device__ __forceinline__ float sde_inv_normal_f32_words(sde_u32 lo, sde_u32 hi
   const float q = __builtin_fmaf((float)(hi ^ m), 0x1.0p-32f, (float)(lo ^ m) * 0x1.0p-64f);
   float x;
   if (q < 2.87e-7f) {
-    const double p = sde_u01_from_words(lo, hi);
+    const double p = (double)((((sde_u64)hi << 32) | lo) >> 11) * 0x1.0p-53;
     x = sde_inv_normal_tail(p < 0.5 ? p : 1.0 - p);
   } else {
     const float t = __builtin_amdgcn_sqrtf(-1.3862943611198906f * __builtin_amdgcn_logf(q));
@@ -426,9 +426,16 @@ template <> __device__ __forceinline__ float sde_psi<float>(SdeUnifX u) { return
 
 __device__ __forceinline__ double sde_dw(double u, double sdt) { return sdt * sde_inv_normal(u); }
 __device__ __forceinline__ float sde_dw(double u, float sdt) { return sdt * sde_inv_normal_f32(u); }
+// SDE_LIBRARY_F64 (defined by the generated source of a universe whose paths part from any difference in a last bit,
+// reaches_root in codegen.hpp): f64 kernels take the general inverse normal of the uniform's f64 value.
+#ifdef SDE_LIBRARY_F64
+template <class U>
+__device__ __forceinline__ double sde_dw(U u, double sdt) { return sdt * sde_inv_normal(sde_uval(u)); }
+#else
 __device__ __forceinline__ double sde_dw(SdeUnifD u, double sdt) { return sdt * sde_inv_normal_d<true>(u.u - 0.5); }
 __device__ __forceinline__ double sde_dw(SdeUnifX u, double sdt) { return sdt * sde_psi<double>(u); }
 __device__ __forceinline__ double sde_dw(SdeUnifW u, double sdt) { return sdt * sde_psi_word(u.lo, u.hi); }
+#endif
 __device__ __forceinline__ float sde_dw(SdeUnifW u, float sdt) { return sdt * sde_inv_normal_f32_words(u.lo, u.hi); }
 __device__ __forceinline__ float sde_dw(SdeUnifX u, float sdt) {
   return sde_sign_select(u.yc, sdt * (float)SDE_PSI_C, u.sm) * sde_inv_normal_f32_x_scaled(u.yc, u.tail);
@@ -585,34 +592,21 @@ typedef sde_u32 SdeU32x2 __attribute__((ext_vector_type(2)));
 // The uniform a step consumes: pseudo-random draws (and, in FP32, Sobol points with the random
 // shift) as two 32-bit words of a 53-bit fraction, XOR-scrambled Sobol points as their word,
 // otherwise an f64 value.
-// SDE_LIBRARY_F64 (defined by the generated source of a universe whose paths part from any difference
-// in a last bit, reaches_root in codegen.hpp): f64 kernels keep the uniform's f64 value, and with
-// it the general inverse normal.
 template <int RNG, typename R> struct SdeUnifOf { typedef double type; };
-#ifndef SDE_LIBRARY_F64
-template <> struct SdeUnifOf<SDE_RNG_SOBOL_XOR, double> { typedef SdeUnifX type; };
-template <> struct SdeUnifOf<SDE_RNG_PSEUDO, double> { typedef SdeUnifW type; };
+template <typename R> struct SdeUnifOf<SDE_RNG_SOBOL_XOR, R> { typedef SdeUnifX type; };
+template <typename R> struct SdeUnifOf<SDE_RNG_PSEUDO, R> { typedef SdeUnifW type; };
 template <> struct SdeUnifOf<SDE_RNG_SOBOL_SHIFT, double> { typedef SdeUnifD type; };
-#endif
-template <> struct SdeUnifOf<SDE_RNG_SOBOL_XOR, float> { typedef SdeUnifX type; };
-template <> struct SdeUnifOf<SDE_RNG_PSEUDO, float> { typedef SdeUnifW type; };
 template <> struct SdeUnifOf<SDE_RNG_SOBOL_SHIFT, float> { typedef SdeUnifW type; };
 
 // The uniform of one draw: from the Sobol word nx (in XOR mode the complement of the scrambled point)
 // and the stream's two words.
-template <int RNG, typename R, bool LIB>
+template <int RNG, typename R>
 __device__ __forceinline__ typename SdeUnifOf<RNG, R>::type sde_uniform(sde_u32 nx, sde_u32 lo, sde_u32 hi,
                                                                         const float* tail, sde_u32 sm, sde_u32 sm2) {
   typename SdeUnifOf<RNG, R>::type u;
   if constexpr (RNG == SDE_RNG_SOBOL_SHIFT && sizeof(R) == 8) {
     const double y = (double)nx * 0x1.0p-32 + sde_u01_from_words(lo, hi);
-    const double v = __builtin_amdgcn_fract(y);  // y - floor(y), 0 <= y < 2
-    if constexpr (LIB) u = v;
-    else u.u = v;
-  } else if constexpr (LIB && RNG == SDE_RNG_SOBOL_XOR) {
-    u = sde_uval(SdeUnifX{nx, nullptr, 0u, 0u});
-  } else if constexpr (LIB) {
-    u = sde_u01_from_words(lo, hi);
+    u.u = __builtin_amdgcn_fract(y);  // y - floor(y), 0 <= y < 2
   } else if constexpr (RNG == SDE_RNG_SOBOL_XOR) {
     u.yc = nx;
     u.tail = tail;
@@ -889,7 +883,7 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
             const int w = USE_CHACHA ? 2 * (i * M + k) : 0;
             if constexpr (USE_INJ) u[j][k] = ni[j][k];
             else if constexpr (M > 0 && (USE_CHACHA || USE_SOBOL))
-              u[j][k] = sde_uniform<RNG, real, LIB>(nx[j][k], W[j][w], W[j][USE_CHACHA ? w + 1 : 0], a.tail_tab, smask, smask2);
+              u[j][k] = sde_uniform<RNG, real>(nx[j][k], W[j][w], W[j][USE_CHACHA ? w + 1 : 0], a.tail_tab, smask, smask2);
             else u[j][k] = 0.5;
           }
         }
@@ -1065,7 +1059,7 @@ __device__ __forceinline__ void sde_team_kernel(const SimArgs& a) {
 #pragma unroll
       for (int k = 0; k < M; ++k) {
         const int w = USE_CHACHA ? 2 * (i * M + k) : 0;
-        const auto u = sde_uniform<RNG, real, false>(nx[i][k], words[w], words[USE_CHACHA ? w + 1 : 0], nullptr, 0u, 0u);
+        const auto u = sde_uniform<RNG, real>(nx[i][k], words[w], words[USE_CHACHA ? w + 1 : 0], nullptr, 0u, 0u);
         noise[half][(q * UNIT + i) * M + k][lane] = Mdl::is_jump(k) ? sde_uval(u) : sde_psi_of(u);
         if (Mdl::SIGN && k == 0) {
           const sde_u64 gt = __builtin_amdgcn_ballot_w64(sde_gt_half(u));
