@@ -501,11 +501,12 @@ std::string generate_kernel_source(const Universe& u, const CodegenOptions& o) {
   s << "  static constexpr int M = " << M << ";\n";
   s << "  static constexpr int NK = " << NK << ";\n";
   s << "  static constexpr bool HAS_PAYOFF = " << (o.payoff.empty() ? "false" : "true") << ";\n";
+  std::set<int> jumps;
+  for (const ProcessDef& pd : u.processes)
+    for (const Term& t : pd.terms)
+      if (t.kind == IncKind::Jump) jumps.insert(t.index);
+  s << "  static constexpr bool WIENER = " << ((int)jumps.size() < M ? "true" : "false") << ";\n";
   if (o.team > 1) {
-    std::set<int> jumps;
-    for (const ProcessDef& pd : u.processes)
-      for (const Term& t : pd.terms)
-        if (t.kind == IncKind::Jump) jumps.insert(t.index);
     s << "  static constexpr bool SIGN = " << (o.scheme == 0 ? "false" : "true") << ";\n";
     s << "  __device__ static constexpr bool is_jump(int k) {\n    return false";
     for (int k : jumps) s << " || k == " << k;

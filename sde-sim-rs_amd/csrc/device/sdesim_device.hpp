@@ -707,7 +707,7 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
   constexpr bool LIB = false;
 #endif
 
-  if constexpr (sizeof(real) == 8 && (USE_CHACHA || USE_SOBOL) && !LIB) sde_normal_tab_load<real>(a.normal_tab);
+  if constexpr (sizeof(real) == 8 && (USE_CHACHA || USE_SOBOL) && Mdl::WIENER && !LIB) sde_normal_tab_load<real>(a.normal_tab);
 
   const long long S = a.S;
   const int N = a.N;
@@ -978,7 +978,7 @@ __device__ __forceinline__ void sde_team_kernel(const SimArgs& a) {
   __shared__ double grid[2][(W - 1) * UNIT][4];  // the steps' t, next t, dt and sqrt(dt)
   __shared__ sde_u64 above[2][(W - 1) * UNIT];  // SIGN: bit l set when lane l's first uniform is > 1/2
 
-  sde_normal_tab_load<real>(a.normal_tab);
+  if constexpr (Mdl::WIENER) sde_normal_tab_load<real>(a.normal_tab);
 
   const long long S = a.S;
   const int N = a.N;
