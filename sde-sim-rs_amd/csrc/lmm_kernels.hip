@@ -181,9 +181,13 @@ __device__ __forceinline__ double lmm_payoff(const LmmArgs& a, const R (&L)[NF],
   if (GRAD) {
     const double itm = U > 0.0 ? rn : 0.0;
     double Pk = P, tail = 0.0;  // P_k, and sum_{j >= k} P_j from the end
+    // A tau the compiler does not know to be the first loop's: it would keep that loop's 40 factors and their
+    // reciprocals for this one, 160 registers, and spilled 180 of them in the f32 kernels.
+    double tau2 = tau;
+    asm volatile("" : "+v"(tau2));
 #pragma unroll
     for (int k = NF - 1; k >= 0; --k) {
-      const double op = 1.0 + tau * (double)L[k], x = tau * (double)L[k] * sde_recip(op);
+      const double op = 1.0 + tau2 * (double)L[k], x = tau2 * (double)L[k] * sde_recip(op);
       if (k < e) {
         M[k] = (R)(-V * x);
       } else {
