@@ -16,6 +16,8 @@
 // three launches can be captured into one hipGraph and replayed.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "device/sdesim_device.hpp"
 #include "reduce.hpp"
 
@@ -188,30 +190,37 @@ __global__ void sdesim_batch_reset(unsigned int* counter) {
   if (threadIdx.x == 0 && blockIdx.x == 0) counter[0] = 0u;
 }
 
-// One wave per instance: its item slots are [slot0[i], slot0[i+1]).
+// G lanes per instance, whose item slots are [slot0[i], slot0[i+1]): a wave, or a thread where no instance has more than
+// a few. (A wave each whatever the slots took 140 us more of 300,000 instances of one slot than a thread each; a
+// thread each took 222 us of 4.2 ms where 4096 instances have hundreds.) Any number of blocks.
+template <int G>
 __global__ void __launch_bounds__(256) sdesim_batch_finalize(const SdeInstance* __restrict__ inst,
                                                              const int* __restrict__ slot0, int n,
                                                              const double* __restrict__ partials,
                                                              double* __restrict__ out) {
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), lane = threadIdx.x & 63;
-  if (i >= n) return;
+  const long long stride = (long long)gridDim.x * blockDim.x / G;
+  const int lane = threadIdx.x & (G - 1);
   typedef double D2 __attribute__((ext_vector_type(2)));
-  SdeSum a, b;
-  const int end = slot0[i + 1];
+  for (long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / G; i < n; i += stride) {
+    SdeSum a, b;
+    const int end = slot0[i + 1];
 #pragma unroll 4
-  for (int s = slot0[i] + lane; s < end; s += 64) {
-    const D2 v = *(const D2*)(partials + 2 * (long long)s);
-    a.add(v.x);
-    b.add(v.y);
-  }
-  sde_wave_sum(a);
-  sde_wave_sum(b);
-  if (lane == 0) {
-    const double S = (double)inst[i].paths;
-    const double s1 = a.value(), s2 = b.value();
-    const double m1 = s1 / S;
-    out[2 * i] = inst[i].x0 + m1;
-    out[2 * i + 1] = S > 1.0 ? (s2 - s1 * m1) / (S - 1.0) : 0.0;
+    for (int s = slot0[i] + lane; s < end; s += G) {
+      const D2 v = *(const D2*)(partials + 2 * (long long)s);
+      a.add(v.x);
+      b.add(v.y);
+    }
+    if constexpr (G == 64) {
+      sde_wave_sum(a);
+      sde_wave_sum(b);
+    }
+    if (lane == 0) {
+      const double S = (double)inst[i].paths;
+      const double s1 = a.value(), s2 = b.value();
+      const double m1 = s1 / S;
+      out[2 * i] = inst[i].x0 + m1;
+      out[2 * i + 1] = S > 1.0 ? (s2 - s1 * m1) / (S - 1.0) : 0.0;
+    }
   }
 }
 
@@ -241,10 +250,15 @@ hipError_t sdesim_launch_batch(int f32, int ppl, int grid, int block, const SdeI
   return hipErrorInvalidValue;
 }
 
-hipError_t sdesim_launch_batch_finalize(const SdeInstance* inst, const int* slot0, int n, const double* partials,
-                                        double* out, hipStream_t stream) {
-  hipLaunchKernelGGL(sdesim_batch_finalize, dim3((n + 3) / 4), dim3(256), 0, stream, inst, slot0, n, partials,
-                     out);
+// most_slots: the largest number of slots of an instance. Up to 8, two rounds of a thread's loads in flight.
+hipError_t sdesim_launch_batch_finalize(const SdeInstance* inst, const int* slot0, int n, int most_slots,
+                                        const double* partials, double* out, hipStream_t stream) {
+  const long long threads = most_slots <= 8 ? n : 64LL * n;
+  const int grid = (int)std::min<long long>((threads + 255) / 256, 1 << 20);
+  if (most_slots <= 8)
+    hipLaunchKernelGGL(sdesim_batch_finalize<1>, dim3(grid), dim3(256), 0, stream, inst, slot0, n, partials, out);
+  else
+    hipLaunchKernelGGL(sdesim_batch_finalize<64>, dim3(grid), dim3(256), 0, stream, inst, slot0, n, partials, out);
   return hipGetLastError();
 }
 

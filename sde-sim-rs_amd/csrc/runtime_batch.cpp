@@ -30,8 +30,8 @@ hipError_t sdesim_launch_batch(int f32, int ppl, int grid, int block, const SdeI
                                int n_items, unsigned int* counter, double* partials, void* terminal,
                                const long long* term_offset, const void* normal_tab, hipStream_t stream);
 hipError_t sdesim_normal_table(int f32, const void** out);
-hipError_t sdesim_launch_batch_finalize(const SdeInstance* inst, const int* slot0, int n, const double* partials,
-                                        double* out, hipStream_t stream);
+hipError_t sdesim_launch_batch_finalize(const SdeInstance* inst, const int* slot0, int n, int most_slots,
+                                        const double* partials, double* out, hipStream_t stream);
 hipError_t sdesim_batch_occupancy(int f32, int ppl, int block, int* blocks_per_cu);
 
 // Error plumbing shared with runtime.cpp.
@@ -111,6 +111,7 @@ void tune_store(const std::string& key, int ppl, int block, double ms) {
 struct sdesim_batch {
   int n = 0, f32 = 0;
   int ppl = 0, block = 0, grid = 0, n_items = 0;
+  int most_slots = 0;  // of an instance, in the work queue
   std::vector<SdeInstance> host;
   std::vector<long long> term_off;
   long long total_paths = 0;
@@ -158,10 +159,12 @@ struct sdesim_batch {
     ppl = new_ppl;
     block = new_block;
     std::vector<int> slot0(n + 1, 0);
+    most_slots = 0;
     std::vector<SdeItem> items;
     for (int i = 0; i < n; ++i) {
       const long long chunks = (host[i].paths + per_item - 1) / per_item;
       slot0[i + 1] = slot0[i] + (int)chunks;
+      most_slots = std::max(most_slots, (int)chunks);
       for (long long c = 0; c < chunks; ++c) items.push_back(SdeItem{i, (int)c, slot0[i] + (int)c, 0});
     }
     // Longest processing time first: an item costs `steps` wave-steps whatever its live lanes.
@@ -191,7 +194,7 @@ struct sdesim_batch {
     bcheck(sdesim_launch_batch(f32, ppl, grid, block, d_inst, d_items, n_items, d_counter, d_partials,
                                keep_terminal ? d_terminal : nullptr, d_term_off, normal_tab, s),
            "batch launch");
-    bcheck(sdesim_launch_batch_finalize(d_inst, d_slot0, n, d_partials, d_moments, s), "batch finalize");
+    bcheck(sdesim_launch_batch_finalize(d_inst, d_slot0, n, most_slots, d_partials, d_moments, s), "batch finalize");
   }
 };
 
