@@ -5,6 +5,7 @@ table scipy ships) into a generated source, compile the host runtime with g++, t
 ahead-of-time kernels with hipcc for gfx950, and link. Run `python build.py` or call build().
 """
 import concurrent.futures
+import hashlib
 import os
 import subprocess
 import sys
@@ -57,6 +58,15 @@ def _ln_table():
     return np.stack([cand[at, best], (grid[at, best] * np.longdouble(2.0 ** -45)).astype(np.float64)], axis=1)
 
 
+def _batch_code_id():
+    """16 hex digits of everything the batch kernels' code depends on: remembered launch configurations hold for it."""
+    h = hashlib.sha256(" ".join(HIP_FLAGS).encode())
+    for f in ("batch_kernels.hip", "reduce.hpp", "device/sdesim_device.hpp", "device/sdesim_args.hpp"):
+        h.update(open(os.path.join(CSRC, f), "rb").read())
+    h.update(_run([HIPCC, "--version"]).encode())
+    return h.hexdigest()[:16]
+
+
 def _raw(s, tag="SDEHDR"):
     assert (")" + tag + '"') not in s
     return 'R"' + tag + "(" + s + ")" + tag + '"'
@@ -76,8 +86,10 @@ def generate_embedded(path):
              'extern const unsigned int sdesim_jk_poly[];',
              'extern const unsigned int sdesim_jk_vinit[];',
              'extern const double sdesim_ln_table[];',
+             'extern const char* sdesim_batch_code_id;',
              'const char* sdesim_embedded_device_header = ' + _raw(dev) + ";",
              'const char* sdesim_embedded_args_header = ' + _raw(args) + ";",
+             'const char* sdesim_batch_code_id = "' + _batch_code_id() + '";',
              'const int sdesim_jk_dims = %d;' % len(poly),
              'const unsigned int sdesim_jk_poly[] = {']
     lines.append(",".join(str(int(v)) for v in poly) + "};")

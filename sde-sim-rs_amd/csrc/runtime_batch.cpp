@@ -34,6 +34,8 @@ hipError_t sdesim_launch_batch_finalize(const SdeInstance* inst, const int* slot
                                         const double* partials, double* out, hipStream_t stream);
 hipError_t sdesim_batch_occupancy(int f32, int ppl, int block, int* blocks_per_cu);
 
+extern "C" const char* sdesim_batch_code_id;  // made by build.py from the batch kernels' sources and flags
+
 // Error plumbing shared with runtime.cpp.
 int sdesim_set_error(int code, const std::string& msg);
 void sdesim_log(const char* fmt, ...);
@@ -239,9 +241,14 @@ int sdesim_batch_create(const sdesim_instance* inst, int32_t n, int32_t precisio
     for (int i = 0; i < n; ++i) items1 += (inst[i].paths + 63) / 64;
     if (items1 > (long long)INT32_MAX)
       throw BatchFailure{SDESIM_EVALUE, "too many work items (paths / (64 * paths_per_lane) summed over the batch)"};
+    // The autotuner's choice holds for this workload shape, these kernels (an upgrade times again) and this device.
+    hipDeviceProp_t prop;
+    int dev = 0;
+    bcheck(hipGetDevice(&dev), "hipGetDevice");
+    bcheck(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
     char kb[64];
     std::snprintf(kb, sizeof kb, "%s-%d-%016llx", b->f32 ? "f32" : "f64", n, sig);
-    b->key = kb;
+    b->key = std::string(kb) + "-" + sdesim_batch_code_id + "-" + prop.gcnArchName + "-" + std::to_string(prop.multiProcessorCount);
     bcheck(sdesim_normal_table(b->f32, &b->normal_tab), "inverse normal table");
     bcheck(hipMalloc(&b->d_inst, sizeof(SdeInstance) * n), "hipMalloc(instances)");
     bcheck(hipMemcpy(b->d_inst, b->host.data(), sizeof(SdeInstance) * n, hipMemcpyHostToDevice), "hipMemcpy");
