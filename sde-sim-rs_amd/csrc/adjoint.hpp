@@ -50,16 +50,20 @@ __device__ __forceinline__ R sde_tape_get(const SdeTapeSlot& t, sde_u32 voff, in
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(t.rs, (int)voff, row * t.row_bytes, 2));
 }
 
+// Row `row` of a slot, with cache policy AUX.
+template <typename R, int AUX>
+__device__ __forceinline__ void sde_tape_put(const SdeTapeSlot& t, sde_u32 voff, int row, R x) {
+  if constexpr (sizeof(R) == 4)
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(sde_u32, (float)x), t.rs, (int)voff, row * t.row_bytes, AUX);
+  else
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(SdeU32x2, (double)x), t.rs, (int)voff, row * t.row_bytes, AUX);
+}
+
 template <typename R, int ROWS>
 __device__ __forceinline__ void sde_tape_store(void* tape, int n, long long S, sde_u32 voff, const R (&X)[ROWS]) {
   const SdeTapeSlot t = sde_tape_slot<R, ROWS>(tape, n, S);
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i) {
-    if constexpr (sizeof(R) == 4)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(sde_u32, (float)X[i]), t.rs, (int)voff, i * t.row_bytes, 2);
-    else
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(SdeU32x2, (double)X[i]), t.rs, (int)voff, i * t.row_bytes, 2);
-  }
+  for (int i = 0; i < ROWS; ++i) sde_tape_put<R, 2>(t, voff, i, X[i]);
 }
 
 template <typename R, int ROWS>

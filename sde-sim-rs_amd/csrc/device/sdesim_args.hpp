@@ -90,17 +90,20 @@ struct BasketArgs {
 // ------------------------------------------------------------------------------------------
 // Forward-rate model, price and curve sensitivities (lmm_kernels.hip); 40 forwards, 3 factors
 // ------------------------------------------------------------------------------------------
+// The root of log2 e as an f32 number, the unit of the f32 kernels' normals (LmmRow in lmm_kernels.hip).
+#define SDE_LMM_ROOT_LOG2E 0x1.337cc2p+0f
+
 struct LmmArgs {
-  double L0[40];                      // initial forwards
-  const void* rows;                   // device [41][8] real, the forward step's parameter rows and a row of zeros
+  const void* rows;                   // device [40][8] real, the forward step's parameter rows (lmm_kernels.hip)
   const void* rows_back;              // the step back's
+  const double* tau_L0;               // device [40], tau times the initial forwards
   double tau, strike;
   long long paths;
   const sde_u32* sobol_tab;           // slice 0 as [steps][64][3], the mask complements folded in
   const sde_u32* sobol_up;            // slices 1-2 as [2][256][steps * 3]
-  void* checkpoints;                  // [slots][40][paths] real, one slot per 16 steps
-  void* tape;                         // [16][40][paths] real, the states of one segment; or the state
-                                      // tape [(steps + 1) / 2 + 1][40][paths]: L_0, L_2, .. and L_N
+  void* checkpoints;                  // [slots][40][paths] real, one slot per 16 steps: states
+  void* tape;                         // [16][40][paths] real, H (lmm_kernels.hip) in one segment; or the state
+                                      // tape [(steps + 1) / 2 + 1][40][paths]: H_0, H_2, .. and H_N
   double* partials;                   // [gridDim.x][42]
   const void* normal_tab;             // table of the f64 inverse normal
   int steps;

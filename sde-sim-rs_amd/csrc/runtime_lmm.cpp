@@ -41,23 +41,25 @@ int guard(F&& f) {
     return sdesim_set_error(SDESIM_ERUNTIME, e.what());
   }
 }
-// The kernels' parameter rows (ts, b0..b2, q0..q2, h; lmm_kernels.hip says what they hold): the forward
-// step's, `unit` the unit of its exponent, then the step back's; a row of zeros after each.
+// The kernels' parameter rows (LmmRow in lmm_kernels.hip says what they hold): the forward step's, `unit` being the
+// unit of its exponent and `s` the kernels' root of it, then the step back's.
 template <class R>
-const void* parameter_rows(std::vector<R>& out, const double* vol, const double* loadings, double dt, double tau,
-                           double unit) {
-  out.assign(2 * (kNF + 1) * 8, R(0));
-  for (int back = 0; back < 2; ++back)
-    for (int i = 0; i < kNF; ++i) {
-      R* r = &out[(size_t)(back * (kNF + 1) + i) * 8];
-      r[0] = (R)(tau * vol[i] * (back ? dt : std::sqrt(dt)));
-      for (int f = 0; f < kF; ++f) {
-        r[1 + f] = (R)loadings[i * kF + f];
-        r[4 + f] = (R)(vol[i] * loadings[i * kF + f] * (back ? 1.0 : std::sqrt(dt) * unit));
-      }
-      r[7] = back ? R(0) : (R)(-0.5 * vol[i] * vol[i] * dt * unit);
+void parameter_rows(R* out, const double* L0, const double* vol, const double* loadings, double dt, double tau,
+                    double unit, double s) {
+  const bool f32 = sizeof(R) == 4;
+  for (int i = 0; i < kNF; ++i) {
+    R* r = out + (size_t)i * 8;
+    R* back = out + (size_t)(kNF + i) * 8;
+    r[0] = back[0] = (R)(tau * L0[i]);
+    for (int f = 0; f < kF; ++f) {
+      const double b = loadings[i * kF + f];
+      r[1 + f] = (R)(vol[i] * b * std::sqrt(dt) * (unit / s));
+      back[1 + f] = (R)b;
+      back[4 + f] = (R)((f32 ? L0[i] : 1.0) * vol[i] * b);
     }
-  return out.data();
+    r[4] = (R)(-0.5 * vol[i] * vol[i] * dt * unit);
+    back[7] = (R)((f32 ? tau : 1.0) * vol[i] * dt);
+  }
 }
 }  // namespace
 
@@ -70,7 +72,7 @@ struct sdesim_lmm {
   int storage = SDESIM_STORAGE_CHECKPOINTS;  // resolved at creation: TAPE or CHECKPOINTS
   void* ckpt = nullptr;                      // checkpoints (CHECKPOINTS)
   void* tape = nullptr;                      // the segment tape (CHECKPOINTS) or the state tape (TAPE)
-  void* rows = nullptr;                      // parameter rows [2][41][8] (forward, back) in the path precision
+  void* rows = nullptr;                      // parameter rows [2][40][8] (forward, back) in the path precision, then tau L0 [40] in f64
   double* partials = nullptr;
   double* sums = nullptr;
   const void* normal_tab = nullptr;  // f64: the device's shared table of the inverse normal
@@ -145,7 +147,7 @@ int sdesim_lmm_create(const sdesim_lmm_spec* spec, sdesim_lmm** out) {
       lk(hipMalloc(&m->ckpt, slots * kNF * (size_t)s.paths * rb), "hipMalloc(checkpoints)");
       lk(hipMalloc(&m->tape, (size_t)kSeg * kNF * (size_t)s.paths * rb), "hipMalloc(segment tape)");
     }
-    lk(hipMalloc(&m->rows, rb * 2 * (kNF + 1) * 8), "hipMalloc(parameters)");
+    lk(hipMalloc(&m->rows, rb * 2 * kNF * 8 + sizeof(double) * kNF), "hipMalloc(parameters)");
     if (s.precision != SDESIM_F32) lk(sdesim_normal_table(0, &m->normal_tab), "inverse normal table");
     lk(hipMalloc(&m->partials, sizeof(double) * kNQ * m->grid), "hipMalloc(partials)");
     lk(hipMalloc(&m->sums, sizeof(double) * kNQ), "hipMalloc(sums)");
@@ -166,22 +168,25 @@ int sdesim_lmm_eval(sdesim_lmm* m, const double* L0, const double* vol, const do
     const sdesim_lmm_spec& s = m->spec;
     LmmArgs a;
     std::memset(&a, 0, sizeof a);
-    for (int i = 0; i < kNF; ++i) a.L0[i] = L0[i];
     hipStream_t st = (hipStream_t)stream;
     const double T = s.tenor * s.expiry_index;
     const double dt = T / s.steps;
     a.tau = s.tenor;
     a.strike = s.strike;
-    std::vector<double> rd;
-    std::vector<float> rf;
-    const void* rows = s.precision == SDESIM_F32 ? parameter_rows(rf, vol, loadings, dt, a.tau, std::log2(std::exp(1.0)))
-                                                 : parameter_rows(rd, vol, loadings, dt, a.tau, 1.0);
-    const size_t row_bytes = (s.precision == SDESIM_F32 ? sizeof(float) : sizeof(double)) * (kNF + 1) * 8;
+    const bool f32 = s.precision == SDESIM_F32;
+    const size_t row_bytes = (f32 ? sizeof(float) : sizeof(double)) * kNF * 8;
+    std::vector<double> rows(2 * row_bytes / sizeof(double) + kNF, 0.0);  // the rows, then tau L0
+    // A forward of 0 in f64, whose derivative is a quotient by it, is a forward too small to change any sum.
+    auto l0 = [&](int i) { return f32 || L0[i] != 0.0 ? L0[i] : 1e-200; };
+    for (int i = 0; i < kNF; ++i) rows[rows.size() - kNF + i] = a.tau * l0(i);
+    if (f32) parameter_rows((float*)rows.data(), L0, vol, loadings, dt, a.tau, std::log2(std::exp(1.0)), SDE_LMM_ROOT_LOG2E);
+    else parameter_rows(rows.data(), L0, vol, loadings, dt, a.tau, 1.0, 1.0);
     // Ordered before the launch on the same stream; the host vector outlives the synchronous wait at
     // the end of this call.
-    lk(hipMemcpyAsync(m->rows, rows, 2 * row_bytes, hipMemcpyHostToDevice, st), "hipMemcpyAsync");
+    lk(hipMemcpyAsync(m->rows, rows.data(), rows.size() * sizeof(double), hipMemcpyHostToDevice, st), "hipMemcpyAsync");
     a.rows = m->rows;
     a.rows_back = (const char*)m->rows + row_bytes;
+    a.tau_L0 = (const double*)((const char*)m->rows + 2 * row_bytes);
     a.paths = s.paths;
     a.sobol_tab = m->tab;
     a.sobol_tab_words = m->tab_words;
@@ -204,7 +209,7 @@ int sdesim_lmm_eval(sdesim_lmm* m, const double* L0, const double* vol, const do
     out[0] = sums[0] / n;
     out[1] = s.paths > 1 ? (sums[1] - sums[0] * out[0]) / (n - 1.0) : 0.0;
     if (adjoint)
-      for (int i = 0; i < kNF; ++i) out[2 + i] = sums[2 + i] / n;
+      for (int i = 0; i < kNF; ++i) out[2 + i] = sums[2 + i] / (f32 ? n : n * l0(i));
   });
 }
 
