@@ -20,7 +20,7 @@
 // A growth of exactly 0 (mu_i dt + sigma_i sqrt(dt) Z rounding to -1, once in 1e8 draws of a coarse f32
 // grid) leaves M_i = 0 and 1 / g infinite, where the derivatives are finite. The block's partials are then NaN,
 // which the host sees in the sums, and sdesim_basket_again takes such blocks again in the form that keeps
-// the zero out of the product (CAREFUL): no test of a growth in the loop of every other run.
+// the zero out of the product (step_careful): no test of a growth in the loop of every other run.
 // No state is kept. The reverse sweep that this replaces wrote and read every state (49 GB for 8 assets x
 // 365 steps x 2^22 paths in f32): 26.1 ms for price and Greeks, 17.6 ms now, bound by VALU issue: a step's 8
 // draws are two thirds of it (350 instructions of ChaCha8, 80 of the normals), the 36 sums, 8
@@ -113,7 +113,6 @@ template <typename R, int D, bool ADJ>
 struct BasketPath {
   static constexpr int NL = BasketConst<D>::NL, NQ = BasketConst<D>::NQ;
   R X[D], H[NL], Q[D];
-  sde_u32 zeroed = 0u;  // CAREFUL: bit i set when an asset i's growth was 0; X[i] is then the product of the others
 
   __device__ __forceinline__ explicit BasketPath(const BasketArgs& a) {
 #pragma unroll
@@ -125,68 +124,58 @@ struct BasketPath {
     for (int q = 0; q < NL; ++q) H[q] = R(0);
   }
 
-  // CAREFUL: with one zero in the product only the zero's own step has a derivative, M_i there being the
-  // product of the other growths, so the sums start anew from that step and are closed by it; a second
-  // zero makes M_i 0.
-  template <bool CAREFUL>
   __device__ __forceinline__ void step(const BasketArgs& a, const R (&eps)[D]) {
 #pragma unroll
     for (int i = 0; i < D; ++i) {
       R c = basket_mdt<R>(a, i);
 #pragma unroll
       for (int k = 0; k <= i; ++k) c = c + basket_scl<R>(a, i, k) * eps[k];
-      if constexpr (CAREFUL) {
-        const bool zero = R(1) + c == R(0), past = ((zeroed >> i) & 1u) != 0u;
-        const R keep = zero && !past ? R(0) : R(1), r = past ? R(0) : zero ? R(1) : sde_recip(R(1) + c);
-        X[i] = X[i] + X[i] * (!zero ? c : past ? R(-1) : R(0));
-        Q[i] = Q[i] * keep + r;
+      X[i] = X[i] + X[i] * c;
+      if constexpr (ADJ) {
+        const R r = sde_recip(R(1) + c);
+        Q[i] = Q[i] + r;
 #pragma unroll
-        for (int k = 0; k <= i; ++k) H[i * (i + 1) / 2 + k] = H[i * (i + 1) / 2 + k] * keep + r * eps[k];
-        zeroed |= zero ? 1u << i : 0u;
-      } else {
-        X[i] = X[i] + X[i] * c;
-        if constexpr (ADJ) {
-          const R r = sde_recip(R(1) + c);
-          Q[i] = Q[i] + r;
-#pragma unroll
-          for (int k = 0; k <= i; ++k) H[i * (i + 1) / 2 + k] = H[i * (i + 1) / 2 + k] + r * eps[k];
-        }
+        for (int k = 0; k <= i; ++k) H[i * (i + 1) / 2 + k] = H[i * (i + 1) / 2 + k] + r * eps[k];
       }
     }
   }
 
-  // All steps of the path whose stream is `key`.
-  template <bool CAREFUL>
-  __device__ __forceinline__ void walk(const BasketArgs& a, const sde_u32 (&key)[8]) {
-    constexpr int U = SdeChunk<D>::U;  // steps in a whole number of ChaCha blocks
-    const int N = a.steps;
-    for (int n0 = 0; n0 < N; n0 += U) {
-      BasketNormals<R> noise;
-      basket_static_for<0, U>([&](auto u_) {
-        constexpr int u = u_;
-        if (U == 1 || n0 + u < N) {
-          R eps[D];
-          basket_static_for<0, D>([&](auto k_) {
-            constexpr int k = k_;
-            eps[k] = noise.template draw<u * D + k>(key, (sde_u64)n0 * D / 8);
-          });
-          step<CAREFUL>(a, eps);
-        }
-      });
+  // The same step where growths may be 0. With one zero in the product only the zero's own step has a derivative, M_i
+  // there being the product of the other growths, so the sums start anew from that step and are closed by it; a
+  // second zero makes M_i 0.
+  __device__ __forceinline__ void step_careful(const BasketArgs& a, const R (&eps)[D], sde_u32& zeroed) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      R c = basket_mdt<R>(a, i);
+#pragma unroll
+      for (int k = 0; k <= i; ++k) c = c + basket_scl<R>(a, i, k) * eps[k];
+      const bool zero = R(1) + c == R(0), past = ((zeroed >> i) & 1u) != 0u;
+      const R keep = zero && !past ? R(0) : R(1), r = past ? R(0) : zero ? R(1) : sde_recip(R(1) + c);
+      X[i] = X[i] + X[i] * (!zero ? c : past ? R(-1) : R(0));
+      Q[i] = Q[i] * keep + r;
+#pragma unroll
+      for (int k = 0; k <= i; ++k) H[i * (i + 1) / 2 + k] = H[i * (i + 1) / 2 + k] * keep + r * eps[k];
+      zeroed |= zero ? 1u << i : 0u;
     }
   }
 
   // The block's partials: price (payoff and payoff^2) or, with ADJ, price and derivatives, of the paths whose
-  // lanes have `live` set. All threads take part.
-  __device__ __forceinline__ void finish(const BasketArgs& a, bool live) {
+  // lanes have `live` set. All threads take part. ZEROED: bit i of `zeroed` is set when a growth of asset i was 0, and
+  // X[i] is the product of the others.
+  template <bool ZEROED = false>
+  __device__ __forceinline__ void finish(const BasketArgs& a, bool live, sde_u32 zeroed = 0u) {
     R w[D];
 #pragma unroll
     for (int i = 0; i < D; ++i) w[i] = (R)a.weight[i];
-    R XN[D];
-#pragma unroll
-    for (int i = 0; i < D; ++i) XN[i] = ADJ && ((zeroed >> i) & 1u) ? R(0) : X[i];
     R pay, dpay;
-    basket_payoff<R, D>(XN, w, (R)a.strike, (R)a.width, pay, dpay);
+    if constexpr (ZEROED) {
+      R XN[D];
+#pragma unroll
+      for (int i = 0; i < D; ++i) XN[i] = (zeroed >> i) & 1u ? R(0) : X[i];
+      basket_payoff<R, D>(XN, w, (R)a.strike, (R)a.width, pay, dpay);
+    } else {
+      basket_payoff<R, D>(X, w, (R)a.strike, (R)a.width, pay, dpay);
+    }
     if constexpr (ADJ) {
       R m[D], lh[D];
 #pragma unroll
@@ -200,7 +189,8 @@ struct BasketPath {
       // Derivative q of this path, q < 3 D + NL: d/dX0, d/dmu, d/dsigma, d/dL (q a constant after
       // unrolling).
       auto grad = [&](int q) -> double {
-        if (q < D) return (double)((((zeroed >> q) & 1u) ? R(0) : m[q]) / (R)a.x0[q]);
+        if (ZEROED && q < D && ((zeroed >> q) & 1u)) return (double)(R(0) / (R)a.x0[q]);
+        if (q < D) return (double)(m[q] / (R)a.x0[q]);
         if (q < 2 * D) return (double)(m[q - D] * dt * Q[q - D]);
         if (q < 3 * D) return (double)(m[q - 2 * D] * sdt * lh[q - 2 * D]);
         int i = 0;
@@ -223,14 +213,29 @@ struct BasketPath {
 template <typename R, int D, bool ADJ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
 sdesim_basket(const BasketArgs a) {
+  constexpr int U = SdeChunk<D>::U;  // steps in a whole number of ChaCha blocks
   sde_normal_tab_load<R>(a.normal_tab);
+  const int N = a.steps;
   const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const bool live = s < a.paths;
 
   sde_u32 key[8];
   sde_seed_from_u64(a.seed + (sde_u64)(live ? s : 0), key);
   BasketPath<R, D, ADJ> path(a);
-  path.template walk<false>(a, key);
+  for (int n0 = 0; n0 < N; n0 += U) {
+    BasketNormals<R> noise;
+    basket_static_for<0, U>([&](auto u_) {
+      constexpr int u = u_;
+      if (U == 1 || n0 + u < N) {
+        R eps[D];
+        basket_static_for<0, D>([&](auto k_) {
+          constexpr int k = k_;
+          eps[k] = noise.template draw<u * D + k>(key, (sde_u64)n0 * D / 8);
+        });
+        path.step(a, eps);
+      }
+    });
+  }
   path.finish(a, live);
 }
 
@@ -282,7 +287,7 @@ __global__ void __launch_bounds__(256) sdesim_basket_team(const BasketArgs a) {
             R eps[D];
 #pragma unroll
             for (int k = 0; k < D; ++k) eps[k] = noise[(r - 1) & 1][(q * U + u) * D + k][lane];
-            path.template step<false>(a, eps);
+            path.step(a, eps);
           }
         }
       }
@@ -292,11 +297,12 @@ __global__ void __launch_bounds__(256) sdesim_basket_team(const BasketArgs a) {
   path.finish(a, steps && live);
 }
 
-// The blocks whose partials of the derivatives are not all finite, once more: same paths, CAREFUL. blockDim is the
+// The blocks whose partials of the derivatives are not all finite, once more: same paths, step_careful. blockDim is the
 // first kernel's paths a block.
 template <typename R, int D>
 __global__ void __launch_bounds__(256) sdesim_basket_again(const BasketArgs a) {
-  constexpr int NQ = BasketConst<D>::NQ;
+  constexpr int NQ = BasketConst<D>::NQ, U = SdeChunk<D>::U;
+  const int N = a.steps;
   bool finite = true;
   for (int q = 2; q < NQ; ++q) {
     const double v = a.partials[(long long)blockIdx.x * NQ + q];
@@ -310,8 +316,22 @@ __global__ void __launch_bounds__(256) sdesim_basket_again(const BasketArgs a) {
   sde_u32 key[8];
   sde_seed_from_u64(a.seed + (sde_u64)(live ? s : 0), key);
   BasketPath<R, D, true> path(a);
-  path.template walk<true>(a, key);
-  path.finish(a, live);
+  sde_u32 zeroed = 0u;
+  for (int n0 = 0; n0 < N; n0 += U) {
+    BasketNormals<R> noise;
+    basket_static_for<0, U>([&](auto u_) {
+      constexpr int u = u_;
+      if (U == 1 || n0 + u < N) {
+        R eps[D];
+        basket_static_for<0, D>([&](auto k_) {
+          constexpr int k = k_;
+          eps[k] = noise.template draw<u * D + k>(key, (sde_u64)n0 * D / 8);
+        });
+        path.step_careful(a, eps, zeroed);
+      }
+    });
+  }
+  path.template finish<true>(a, live, zeroed);
 }
 
 // Sum of per-block partials per quantity: one block of 1024 threads each, whose loads of 8 bytes
