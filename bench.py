@@ -165,7 +165,7 @@ def main():
     ap.add_argument("--calib", action="store_true", help="run a 1 GiB device copy first (HBM counter calibration)")
     ap.add_argument("--only", default="", help="comma list of legs to run: f32,long,f64,term,batch,adjoint,lmm")
     ap.add_argument("--adjoint-storage", default="auto", choices=("auto", "tape", "checkpoints"),
-                    help="state storage of the basket and forward-rate adjoints")
+                    help="state storage of the forward-rate adjoint")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) > 1:
         print("bench.py measures one GPU only: paths are independent and the multi-GPU form "
@@ -276,7 +276,7 @@ def main():
                "greeks": 52, "adjoint_ms": times[True], "price_ms": times[False],
                "adjoint_over_price": times[True] / times[False],
                "path_steps_per_s_adjoint": AS * AN / (times[True] * 1e-3), "price": r["price"],
-               "storage": bk.storage, "state_bytes": 0}  # the derivatives are summed on the way forward
+               "state_bytes": 0}  # the derivatives are summed on the way forward
         del bk
 
     lmm = None

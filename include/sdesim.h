@@ -100,7 +100,8 @@ int64_t sdesim_plan_filtration_bytes(const sdesim_plan* plan);
 
 /* Run the plan on `stream`: the kernel writes the step-major filtration [T][P][S] into
  * d_filtration (device, may be NULL when SDESIM_OUT_FILTRATION is off) and, with
- * SDESIM_OUT_TERMINAL, reduces terminal moments into the plan. `d_injected` ([N*m][S] f64,
+ * SDESIM_OUT_TERMINAL, reduces terminal moments into the plan. An FP64 path does not depend on how
+ * many paths run with it; the moments' last bits do, with the order of their sums. `d_injected` ([N*m][S] f64,
  * device) is read only with SDESIM_INJECTED. Asynchronous. */
 int sdesim_plan_run(sdesim_plan* plan, void* d_filtration, const double* d_injected, void* stream);
 
@@ -219,8 +220,9 @@ int sdesim_batch_info(const sdesim_batch* b, int32_t* paths_per_lane, int32_t* b
  *   dX_i = (mu_i * X_i) * dt + sum_k (sigma_i * L_ik * X_i) * dW_k
  * on the grid dt = horizon / steps with pseudo-random draws of ChaCha8(seed + s); payoff on
  * B = sum_i w_i X_{N,i}: width * softplus((B - strike) / width), or max(B - strike, 0) if
- * width == 0. The adjoint checkpoints the state every 19 steps in HBM and recomputes each
- * segment during the reverse sweep.
+ * width == 0. The adjoint's derivatives are summed on the way forward: no state is kept. The order
+ * in which paths are summed depends on the path count and the device (blocks of 64 paths up to
+ * 128 paths per compute unit, of 256 beyond), and with it the results' last bits.
  * --------------------------------------------------------------------------------------- */
 typedef struct sdesim_basket sdesim_basket;
 

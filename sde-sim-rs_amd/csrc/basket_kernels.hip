@@ -1,4 +1,4 @@
-// basket_kernels.hip -- correlated GBM basket: price and pathwise adjoint (reverse sweep).
+// basket_kernels.hip -- correlated GBM basket: price and pathwise derivatives, summed on the way forward.
 //
 // Model: A assets, X_{n+1,i} = X_{n,i} + X_{n,i} (mu_i dt + sigma_i sqrt(dt) Z_{n,i}),
 // Z_n = L eps_n with L the lower Cholesky factor of the correlation and eps_{n,k} = Psi(u_{n,k})

@@ -459,7 +459,7 @@ __device__ __forceinline__ float sde_signed(SdeUnifX u, float sdt) { return sde_
 // Sequential inverse Poisson CDF capped at k = 200 (f64, as the reference). exp(-lambda) >= 1 - lambda, so
 // a u with u + lambda below 1 by more than the sum's and exp's rounding is 0 jumps without it. With few jumps a
 // step (lambda dt = 5e-4) 97 of 100 waves have no other lane, and the exponential was half of a step's chain:
-// 10,000 x 1000 steps of the jump diffusion take 193 instead of 295 us. The test also stands for lambda > 0 there,
+// 10,000 x 1000 steps of the jump diffusion took 193 instead of 295 us (150 now). The test also stands for lambda > 0 there,
 // so that steps in which a wave has jumps pay one addition for it (a difference of 5 % when it was three
 // operations more: jumps alone, 2^20 x 40, XOR, lambda dt = 0.0125).
 __device__ __forceinline__ double sde_inv_poisson(double u, double lambda) {
@@ -941,9 +941,9 @@ __device__ __forceinline__ void sde_path_kernel(const SimArgs& a) {
 // steps' times go through LDS as well: a scalar load per step, waited for together with the LDS reads, took
 // a fifth of the stepping wave's time. Each value is computed by the operations of sde_path_kernel, the
 // generated step settling which products are fused, so a path is the same bit for bit from either.
-// What bounds it now is the stepping wave's chain. GBM, 10,000 x 252 pseudo-random: 31 us instead of 80; the
-// jump diffusion, 10,000 x 1000: 295 instead of 588 (193 with its jumps' short cut); Heston RK, 65,537 x
-// 365, random shift: 302 instead of 388.
+// What bounds it now is the stepping wave's chain. Runs one after the other, against sde_path_kernel: GBM, 10,000 x
+// 252 pseudo-random, 24 instead of 72 us; the jump diffusion, 10,000 x 1000, 150 instead of 419; Heston RK, 65,537 x
+// 365, random shift, 235 instead of 353.
 // FP64 only: the FP32 step may be reassociated, and how depends on the code around it.
 //
 // A step's noise as the stepping wave reads it: Psi(u) of a Wiener increment, u of a jump, and (RK) whether

@@ -551,7 +551,7 @@ int32_t sdesim_process_index(const sdesim_universe* u, const char* name) {
 // Waves of a block in sde_team_kernel for this plan, or 1: one lane per path, sde_path_kernel. Teams are for
 // runs that leave SIMDs empty or nearly so: four waves, one per SIMD of a CU (five to twelve are no faster
 // even with a CU per block), up to 3/2 waves of paths per SIMD. There (98,304 paths) they still take
-// 62 against 81 us (GBM, XOR) and 152 against 162 (Heston moments); at 2 per SIMD 216 against 185. Three, up
+// 62 against 74 us (GBM, XOR) and 139 against 152 (Heston moments); at 2 per SIMD 216 against 185. Three, up
 // to a wave per SIMD, where the buffer of four exceeds a block's 64 KB of LDS. Not for FP32, nor where paths
 // part from any difference in a last bit; nor for fewer steps than one round produces, nor
 // where the partials of 64 paths each would outgrow the scratch array.

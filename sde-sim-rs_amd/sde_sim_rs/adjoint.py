@@ -3,8 +3,8 @@
 The price kernel runs the Euler step of the DSL form
     dX_i = (mu_i * X_i) * dt + sum_k (sigma_i * L_ik * X_i) * dW_k
 (src/sim/euler.rs:5-37 on the reference's equation language, with the Cholesky factor L of the
-correlation written into the coefficients) and a reverse-sweep adjoint kernel returns the
-path-averaged derivatives with respect to X0, mu, sigma and L. This module maps dL to the
+correlation written into the coefficients) and, with the adjoint, returns the path-averaged
+derivatives with respect to X0, mu, sigma and L, summed on the way forward. This module maps dL to the
 correlation matrix (reverse mode of the Cholesky factorisation) and wraps the pair in a
 torch.autograd.Function.
 """
