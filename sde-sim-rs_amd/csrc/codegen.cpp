@@ -620,7 +620,7 @@ class NoiseRoots {
   }
 
   // Whether the root's argument is a process x or max(x, 0) whose own drift a and noise b near 0, functions of x
-  // alone, have b^2 / x -> s^2 and 4 a >= s^2.
+  // alone, have b^2 / x -> s^2 and 4 a >= s^2, or b / x bounded and a >= 0.
   bool steadied(const Expr& arg) {
     const Expr* v = &arg;
     if (arg.op == Op::Call && arg.fn == Fn::Max && arg.args.size() == 2)
@@ -647,9 +647,12 @@ class NoiseRoots {
       return r;
     };
     try {
+      // b^2 / x at two points: constant for a root, falling in proportion where b is linear in x, or faster.
       const double s2 = sum(IncKind::Wiener, 0x1.0p-40) * 0x1.0p40, closer = sum(IncKind::Wiener, 0x1.0p-42) * 0x1.0p42;
-      return sum(IncKind::Wiener, 0.0) == 0.0 && s2 > 0.0 && closer >= 0.99 * s2 && closer <= 1.01 * s2 &&
-             4.0 * sum(IncKind::Time, 0.0) >= s2;
+      const double a = sum(IncKind::Time, 0.0);
+      if (sum(IncKind::Wiener, 0.0) != 0.0) return false;
+      if (4.0 * closer <= 1.01 * s2) return a >= 0.0;
+      return closer >= 0.99 * s2 && closer <= 1.01 * s2 && 4.0 * a >= s2;
     } catch (const std::exception&) {
       return false;  // a coefficient that does not evaluate fails where the kernel is generated
     }

@@ -53,7 +53,8 @@ std::string kernel_name(const CodegenOptions& o);
 // below 1 they come together (Heston's variance at 1.28: 1e-15 after 1024). Any other root has such a place too,
 // wherever its argument vanishes (0.8 sqrt(x (1 - x)) at 1 with a drift of 0.015 to it: 0.67 after 1550). So the
 // only roots of a Levy process in a noise coefficient that are taken to be harmless are those of a process x, or
-// max(x, 0), whose own drift and noise depend on x alone and have 4 a >= s^2 at 0; every other power below 1,
+// max(x, 0), whose own drift and noise depend on x alone and at 0 have 4 a >= s^2, or noise that vanishes like x
+// itself and a >= 0 (a geometric variance: differences stay in proportion to it); every other power below 1,
 // logarithm or inverse function counts. The f64 kernels of such universes, and the batch kernel's CIR
 // instances with 4 a < s^2, keep the library's logarithm, root and division, so that their paths stay bit for bit
 // those of the general inverse normal.

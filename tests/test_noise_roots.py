@@ -27,6 +27,13 @@ HESTON_VARIANCE = HESTON[1]
     (["dv = (2.0 * (0.04 - max(v, 0))) * dt + (0.2 * max(v, 0)^0.5) * dW1 + (-0.01) * dN1(3.0)"], True),
     # Another process's root, of a process that crosses 0.
     (["dS = (0.1 * S) * dt + (S * max(v, 0)^0.5) * dW1", "dv = (0.04 - v) * dt + (0.1) * dW2"], True),
+    # A process whose noise vanishes like itself, with a drift that keeps it there or not.
+    (["dS = (0.1 * S) * dt + (S * max(v, 0)^0.5) * dW1", "dv = (0.05 * v) * dt + (0.4 * v) * dW2"], False),
+    (["dS = (0.1 * S) * dt + (S * v^0.5) * dW1", "dv = (2.0 * (0.04 - v)) * dt + (0.4 * v) * dW2"], False),
+    (["dS = (0.1 * S) * dt + (S * v^0.5) * dW1", "dv = (2.0 * (-0.04 - v)) * dt + (0.4 * v) * dW2"], True),
+    (["dX = (2.0 * (0.04 - X)) * dt + (0.4 * X * max(X, 0)^0.5) * dW1"], False),
+    (["dS = (0.1 * S) * dt + (S * max(v, 0)^0.5) * dW1", "dv = (0.1) * dt + (0.4 * max(v, 0)^0.75) * dW2"], True),
+    (["dS = (0.1 * S) * dt + (S * max(v, 0)^0.5) * dW1", "dv = (0.04 - v) * dt"], False),
     # Through an algebraic process, as another power, as a logarithm or an inverse function.
     (["dX = (0.5 * (0.97 - X)) * dt + (0.8 * R) * dW1", "R = max(X * (1 - X), 0)^0.5"], True),
     (["dX = (0.5 * (0.97 - X)) * dt + (0.8 * A^0.5) * dW1", "A = X * (1 - X)"], True),
