@@ -247,6 +247,10 @@ class Plan:
             self._h = None
 
 
+# The most bytes of a string chunk: Arrow's string type has signed 32-bit offsets.
+_STRING_CHUNK_BYTES = (1 << 31) - 1
+
+
 def long_table(names, times, scenarios, values, chunk_rows=1 << 24):
     """The reference's long layout (src/filtration.rs:81-116, concatenated in scenario order by
     src/sim/mod.rs:88-91): columns scenario:i32, time:f64, process_name:str, value:f64, rows
@@ -266,7 +270,7 @@ def long_table(names, times, scenarios, values, chunk_rows=1 << 24):
     if vals.size != S * per:
         raise ValueError("values must hold scenarios x len(times) x len(names) entries")
     longest = max([len(n.encode("utf-8")) for n in names] + [1])
-    rows = max(1, min(int(chunk_rows), ((1 << 31) - 1) // longest))
+    rows = max(1, min(int(chunk_rows), _STRING_CHUNK_BYTES // longest))
     spc = max(1, rows // max(1, per))  # scenarios per chunk
     spc = min(spc, max(1, S))
     tpat = np.repeat(np.asarray(times, dtype=np.float64), P)
@@ -274,21 +278,27 @@ def long_table(names, times, scenarios, values, chunk_rows=1 << 24):
     # The name column's buffers, formed directly: a repetition of the names' bytes, and offsets in arithmetic
     # progression per name: 0.7 ms for 2.53e6 rows, whose decoding from dictionary indices took 8 of the whole
     # call's 12 ms (5 now).
+    # A chunk holds as many time points as fit Arrow's limit: those of the other columns' chunk, or, where one
+    # scenario's names alone exceed it, fewer.
     encoded = [n.encode("utf-8") for n in names]
-    ends = np.cumsum([0] + [len(e) for e in encoded], dtype=np.int32)
-    offsets = np.empty(spc * per + 1, dtype=np.int32)
+    sizes = [len(e) for e in encoded]
+    steps = max(1, min(spc * T, _STRING_CHUNK_BYTES // max(1, sum(sizes))))
+    ends = np.cumsum([0] + sizes, dtype=np.int32)
+    offsets = np.empty(steps * P + 1, dtype=np.int32)
     offsets[0] = 0
-    starts = np.arange(spc * T, dtype=np.int32) * ends[-1]
+    starts = np.arange(steps, dtype=np.int32) * ends[-1]
     for p in range(P):
         np.add(starts, ends[p + 1], out=offsets[1 + p::P])
-    name_chunk = pa.StringArray.from_buffers(spc * per, pa.py_buffer(offsets),
-                                             pa.py_buffer(b"".join(encoded) * (spc * T)))
+    name_chunk = pa.StringArray.from_buffers(steps * P, pa.py_buffer(offsets),
+                                             pa.py_buffer(b"".join(encoded) * steps))
     cols = {"scenario": [], "time": [], "process_name": [], "value": []}
     for s0 in range(0, S, spc):
         n = min(spc, S - s0)
         cols["scenario"].append(pa.array(np.repeat(np.arange(s0, s0 + n, dtype=np.int32), per)))
         cols["time"].append(time_chunk if n == spc else time_chunk.slice(0, n * per))
-        cols["process_name"].append(name_chunk if n == spc else name_chunk.slice(0, n * per))
+        for t0 in range(0, n * T, steps):
+            k = min(steps, n * T - t0)
+            cols["process_name"].append(name_chunk if k == steps else name_chunk.slice(0, k * P))
         cols["value"].append(pa.array(vals[s0 * per:(s0 + n) * per]))
     types = {"scenario": pa.int32(), "time": pa.float64(), "process_name": pa.string(), "value": pa.float64()}
     table = pa.table({k: pa.chunked_array(v, type=types[k]) for k, v in cols.items()})
